@@ -310,3 +310,27 @@ def test_backward_cfg4_full_size(hip_backend):
     scb = (ts.screened_spmm(A.abs().cuda(), diag.cuda(), torch.ones(A.shape[0], 1, device="cuda"),
                             threshold=thr).double().T @ G.abs().cuda().double()).squeeze(0).cpu() + 1e-30
     assert ((lhs - rhs).abs() / scb).max().item() <= 1e-4
+
+
+@pytest.mark.parametrize("n,N", [(1, 1), (3, 65), (63, 64), (64, 1), (65, 63), (127, 130), (129, 5), (192, 257), (321, 129)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_small_tiles_forward_and_backward(hip_backend, n, N, offset):
+    """The 64x64-tile kernels at the edges of their tiles, k-slabs and
+    alignment (`offset` floats into a buffer: rows on 4-byte boundaries), with
+    128-row tiles that the threshold skips whole. Each is a sum of at most
+    max(n, N) fp32 products in an order of its own: well inside 1e-4 of the
+    absolute products (TOL)."""
+    g = torch.Generator().manual_seed(1000 * n + N)
+
+    def operand(*shape):
+        flat = torch.randn(math.prod(shape) + offset, generator=g).cuda()
+        return flat[offset:].view(shape).requires_grad_(True)
+
+    A, B = operand(n, n), operand(n, N)
+    G = operand(n, N).detach()
+    diag = torch.pow(10.0, -4.0 * torch.arange(n) / max(n - 1, 1)).float().cuda()  # 1 .. 1e-4, descending
+    thr = 1.0437e-5  # masks pairs of small rows (whole tiles for n > 128); no pair lies on it
+    C = ts.screened_spmm(A, diag, B, thr)
+    _check(A.detach(), diag, B.detach(), thr, C.detach())
+    dA, dB = torch.autograd.grad(C, (A, B), G)
+    _check_backward(A.detach(), diag, B.detach(), thr, G, dA, dB, TOL)

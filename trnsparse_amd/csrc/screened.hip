@@ -22,15 +22,17 @@
 //                       structure (direct-to-LDS slab ring, 64x64 wave
 //                       tiles); the mask multiplies the A fragments after
 //                       their LDS read; the K loop visits active k-tiles.
-//   screened_f32_mfma   the register-staged variant on the shared MFMA core
-//                       (mfma_f32.h), for operands past 4 GiB.
+//   screened_f32_flex   fp32 on 64x64 tiles (f32_flex.h): any alignment, any
+//                       size, and grids whose 128x128 tiles leave CUs idle.
 //   screened_f64_dma    fp64 (even m and strides): the same structure on
 //                       v_mfma_f64_16x16x4_f64 (mfma_f64.h operand tiles).
-//   screened_generic    other or unaligned operands: one thread per output.
-//   screened_bwd_a_f32 / screened_bwd_b_f32 / screened_bwd_*_generic
-//                       the backward (below).
+//   screened_generic    fp64 operands of odd sizes or alignment: one thread
+//                       per output.
+//   screened_bwd_a_f32 / screened_bwd_b_f32 / screened_bwd_*_flex /
+//   screened_bwd_*_generic   the backward (below).
 #include <atomic>
 
+#include "f32_flex.h"
 #include "lds_dma.h"
 #include "mfma_f32.h"
 #include "mfma_f64.h"
@@ -40,7 +42,6 @@ namespace {
 
 namespace T32 = tsp::f32tile;
 constexpr int TILE = 128;
-constexpr int KC = 64;
 
 template <typename QT>
 __device__ inline QT qsqrt(QT v);
@@ -66,83 +67,6 @@ __global__ __launch_bounds__(TILE) void screened_q(const QT* __restrict__ diag, 
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
   __syncthreads();
   if (threadIdx.x == 0) qmax[blockIdx.x] = red[0] > red[1] ? red[0] : red[1];
-}
-
-template <typename QT>
-struct ScreenedSlabs {
-  const float* __restrict__ A;
-  const float* __restrict__ B;
-  const QT* __restrict__ Q;
-  const QT* __restrict__ qmax;
-  int64_t lda, ldb, m, ncols, row0, n0;
-  QT thr, qI;
-  int nkt;
-  int kt;  // k tile of the current slab group (advanced as slabs are requested in order)
-  T32::Coords<KC> q;
-
-  __device__ bool active(int t) const { return qI * qmax[t] > thr; }
-  __device__ int count() const {
-    int c = 0;
-    for (int t = 0; t < nkt; ++t) c += active(t) ? 1 : 0;
-    return c;
-  }
-  __device__ void load(int s, f32x4 (&a)[T32::Slab<KC>::NA], f32x4 (&b)[T32::Slab<KC>::NB]) {
-    constexpr int PER = TILE / KC;  // slabs per k tile
-    if ((s % PER) == 0) {
-      ++kt;
-      while (!active(kt)) ++kt;
-    }
-    const int kk = (s % PER) * KC;
-    const int64_t kc = (int64_t)kt * TILE + kk + q.ac;
-    QT qk[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) qk[i] = kc + i < m ? Q[kc + i] : (QT)0;
-#pragma unroll
-    for (int j = 0; j < T32::Slab<KC>::NA; ++j) {
-      const int64_t r = row0 + q.ar + j * q.astep;
-      a[j] = T32::load4_guard(A, r, kc, m, m, lda);
-      const QT qa = r < m ? Q[r] : (QT)0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[j][i] *= (qa * qk[i] > thr) ? 1.0f : 0.0f;
-    }
-    const int64_t brow = (int64_t)kt * TILE + kk + q.br;
-#pragma unroll
-    for (int j = 0; j < T32::Slab<KC>::NB; ++j) b[j] = T32::load4_guard(B, brow + 16 * j, n0 + q.bc, m, ncols, ldb);
-  }
-};
-
-template <typename QT>
-__global__ __launch_bounds__(T32::NTHR) void screened_f32_mfma(
-    const float* __restrict__ A, int64_t lda, const QT* __restrict__ Q, const QT* __restrict__ qmax, QT thr,
-    int64_t m, const float* __restrict__ B, int64_t ldb, int64_t ncols, float* __restrict__ C, int64_t ldc, int nmt,
-    int nnt) {
-  __shared__ __attribute__((aligned(16))) float lds[T32::Slab<KC>::LDS_FLOATS];
-  // XCD-aware: the column tiles of one row panel of A share an XCD (and its L2).
-  int64_t mt64;
-  int nt;
-  if (!T32::tile_item(blockIdx.x, nmt, nnt, nullptr, mt64, nt)) return;
-  const int mt = (int)mt64;
-
-  ScreenedSlabs<QT> src;
-  src.A = A;
-  src.B = B;
-  src.Q = Q;
-  src.qmax = qmax;
-  src.lda = lda;
-  src.ldb = ldb;
-  src.m = m;
-  src.ncols = ncols;
-  src.row0 = (int64_t)mt * TILE;
-  src.n0 = (int64_t)nt * T32::BN;
-  src.thr = thr;
-  src.qI = qmax[mt];
-  src.nkt = (int)tsp::ceil_div(m, TILE);
-  src.kt = -1;
-  const int nsteps = src.count() * (TILE / KC);
-
-  f32x16 acc0 = {}, acc1 = {};
-  T32::run<KC>(src, nsteps, lds, src.q, acc0, acc1);
-  T32::store_tile(C, ldc, src.row0, src.n0, m, ncols, src.q, acc0, acc1, [](float v) { return v; });
 }
 
 // screened_f32_dma<QT>: fp32 A and B, the streamed MFMA structure of
@@ -420,6 +344,115 @@ __global__ __launch_bounds__(256) void screened_f64_dma(
 #define SCREENED_KC 32
 #endif
 
+// ------------------------------------------------------- small tiles (fp32)
+//
+// The products on 64x64 tiles of any alignment (f32_flex.h): the mask
+// multiplies each A element once, while it is staged. The tile skip keeps
+// its 128-row granularity. Rows that are not 16-byte aligned always take
+// them: n = N = 1111 forward 767 -> 62 us, dA 4080 -> 54, dB 834 -> 64 against
+// one thread per output (host-timed calls, launch of screened_q included).
+namespace X = tsp::flex;
+constexpr int SPT = TILE / X::KC;  // slabs per 128-row tile
+
+// Whether aligned operands with a row_items x col_items output are faster on
+// 64x64 tiles. The streamed kernels own a CU (or share it in pairs) with
+// 128x128 tiles, so what counts is how many tiles the fullest of the 256 CUs
+// gets. Costs are ns per k, measured: a lone 128-tile on a CU `one`, two at
+// once `two`, each 64-tile `small`. Forward at 88 / 139 / 21: n = 1024 (64
+// tiles) 90 -> 34 us, 1536 137 -> 106, 3072 (576 tiles, 2.25 per CU) 674 ->
+// 573, while 2048 x 2048 (182 against 179) is even and 4096 (1024 tiles, 4 per
+// CU) keeps the streamed kernel's 1137 against 1314. dA at 68 / 136 / 18: 3072
+// 623 -> 505, 4096 keeps 1093 (1167). dB at 77 / 154 / 21: 3072 705 -> 582,
+// 4096 keeps 1249 (1358).
+bool small_tiles_faster(int64_t row_items, int64_t col_items, int one, int two, int small) {
+  const int64_t big = tsp::ceil_div(tsp::ceil_div(row_items, TILE) * tsp::ceil_div(col_items, TILE), 256);
+  const int64_t tiny = tsp::ceil_div(tsp::ceil_div(row_items, X::TM) * tsp::ceil_div(col_items, X::TM), 256);
+  return big / 2 * two + big % 2 * one > tiny * small;
+}
+
+// Walks the 128-row tiles t with qo * qmax[t] > thr in order.
+template <typename QT>
+struct ActiveTiles {
+  const QT* __restrict__ qmax;
+  QT qo, thr;
+  int t;
+  __device__ ActiveTiles(const QT* qmax_, int own, QT thr_) : qmax(qmax_), qo(qmax_[own]), thr(thr_), t(-1) {}
+  // slabs of all active tiles (rows at or past m, in the last tile, have none)
+  __device__ int slabs(int nkt, int64_t m) const {
+    int c = 0;
+    for (int t0 = 0; t0 < nkt; t0 += 64) {
+      const int i = t0 + (int)(threadIdx.x & 63);
+      c += __popcll(__ballot(i < nkt && qo * qmax[i < nkt ? i : 0] > thr));
+    }
+    c *= SPT;
+    if (qo * qmax[nkt - 1] > thr) c -= SPT - (int)tsp::ceil_div(m - (int64_t)(nkt - 1) * TILE, X::KC);
+    return c;
+  }
+  // first row of slab s (called for s = 0, 1, ...)
+  __device__ int64_t row(int s) {
+    if (s % SPT == 0) {
+      ++t;
+      while (!(qo * qmax[t] > thr)) ++t;
+    }
+    return (int64_t)t * TILE + (s % SPT) * X::KC;
+  }
+};
+
+// C = (A * mask) B: A rows of the tile (ROW), B rows k (COL).
+template <typename QT>
+struct FlexFwd {
+  const float *A, *B;
+  const QT* Q;
+  int64_t lda, ldb, m, ncols, row0, n0;
+  ActiveTiles<QT> act;
+  QT qr[2];
+  struct Regs {
+    X::Row x;
+    X::Col y;
+    QT qk[4];
+  };
+  __device__ void load(int s, Regs& r) {
+    const int64_t k0 = act.row(s);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r.qk[e] = Q[k0 + X::Row::k() + e];  // zeros up to whole 128-row tiles
+    r.x.load(A, lda, row0, m, k0, m);
+    r.y.load(B, ldb, k0, m, n0, ncols);
+  }
+  __device__ void finish(Regs& r) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r.x.v[j][e] *= (qr[j] * r.qk[e] > act.thr) ? 1.0f : 0.0f;
+  }
+};
+
+template <typename QT>
+__global__ __launch_bounds__(X::NTHR, 4) void screened_f32_flex(
+    const float* __restrict__ A, int64_t lda, const QT* __restrict__ Q, const QT* __restrict__ qmax, QT thr,
+    int64_t m, const float* __restrict__ B, int64_t ldb, int64_t ncols, float* __restrict__ C, int64_t ldc, int nmt,
+    int nnt) {
+  __shared__ __attribute__((aligned(16))) float lds[X::LDS_FLOATS];
+  int64_t mt;
+  int nt;
+  // XCD-aware: the column tiles of one row panel of A share an XCD (and its L2)
+  if (!T32::tile_item(blockIdx.x, nmt, nnt, nullptr, mt, nt)) return;
+  const int64_t row0 = mt * X::TM, n0 = (int64_t)nt * X::TM;
+  FlexFwd<QT> src{A, B, Q, lda, ldb, m, ncols, row0, n0, {qmax, (int)(row0 / TILE), thr}, {}};
+#pragma unroll
+  for (int j = 0; j < 2; ++j) src.qr[j] = Q[row0 + X::Row::i() + 32 * j];
+  float acc[8];
+  X::run(src, src.act.slabs((int)tsp::ceil_div(m, TILE), m), lds, acc);
+  const X::Out o;
+  const int64_t c = n0 + o.col;
+  if (c < ncols) {
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      const int64_t r = row0 + o.row(v);
+      if (r < m) C[r * ldc + c] = acc[v];
+    }
+  }
+}
+
 template <typename T, typename QT>
 __global__ __launch_bounds__(256) void screened_generic(const T* __restrict__ A, int64_t lda, const QT* __restrict__ Q,
                                                        QT thr, int64_t m, const T* __restrict__ B, int64_t ldb,
@@ -456,8 +489,10 @@ __global__ __launch_bounds__(256) void screened_generic(const T* __restrict__ A,
 //       A tile [k = rows i][columns] is the A^T operand (k tile reads),
 //       masked after its LDS read with Q_i of the slab staged beside the
 //       ring; dC rows of I are the [k][n] operand.
-//   screened_bwd_a_generic / screened_bwd_b_generic   fp64 and operands the
-//       streamed kernels do not take: one thread per output.
+//   screened_bwd_a_flex / screened_bwd_b_flex   the same products on 64x64
+//       tiles (f32_flex.h).
+//   screened_bwd_a_generic / screened_bwd_b_generic   fp64: one thread per
+//       output.
 namespace P = tsp::f32pair;
 
 template <typename QT>
@@ -661,6 +696,104 @@ __global__ __launch_bounds__(256) void screened_bwd_b_f32(const float* __restric
   }
 }
 
+// dA = (G B^T) * mask: rows of G and of B (both ROW), k = the N columns.
+struct FlexBwdA {
+  const float *G, *B;
+  int64_t ldg, ldb, m, ncols, r0, c0;
+  struct Regs {
+    X::Row x, y;
+  };
+  __device__ void load(int s, Regs& r) {
+    r.x.load(G, ldg, r0, m, (int64_t)s * X::KC, ncols);
+    r.y.load(B, ldb, c0, m, (int64_t)s * X::KC, ncols);
+  }
+  __device__ void finish(Regs&) {}
+};
+
+template <typename QT>
+__global__ __launch_bounds__(X::NTHR, 4) void screened_bwd_a_flex(const float* __restrict__ G, int64_t ldg,
+                                                               const float* __restrict__ B, int64_t ldb,
+                                                               int64_t ncols, const QT* __restrict__ Q,
+                                                               const QT* __restrict__ qmax, QT thr, int64_t m,
+                                                               int nmt, float* __restrict__ dA, int64_t ldda) {
+  __shared__ __attribute__((aligned(16))) float lds[X::LDS_FLOATS];
+  // XCD-aware: XCD x takes a contiguous range of tiles, as in screened_bwd_a_f32
+  const int64_t ntiles = (int64_t)nmt * nmt, per = tsp::ceil_div(ntiles, 8);
+  const int64_t slot = blockIdx.x >> 3, tix = (blockIdx.x & 7) * per + slot;
+  if (slot >= per || tix >= ntiles) return;
+  const int64_t r0 = tix / nmt * X::TM, c0 = tix % nmt * X::TM;
+  float acc[8] = {};
+  if (qmax[r0 / TILE] * qmax[c0 / TILE] > thr) {  // else every pair is masked: zeros
+    FlexBwdA src{G, B, ldg, ldb, m, ncols, r0, c0};
+    X::run(src, (int)tsp::ceil_div(ncols, X::KC), lds, acc);
+  }
+  const X::Out o;
+  const int64_t c = c0 + o.col;
+  if (c < m) {
+    const QT qc = Q[c];
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      const int64_t r = r0 + o.row(v);
+      if (r < m) dA[r * ldda + c] = acc[v] * ((Q[r] * qc > thr) ? 1.0f : 0.0f);
+    }
+  }
+}
+
+// dB = (A * mask)^T G: columns of A (COL, k = the rows i), G rows i (COL).
+template <typename QT>
+struct FlexBwdB {
+  const float *A, *G;
+  const QT* Q;
+  int64_t lda, ldg, m, ncols, k0, n0;
+  ActiveTiles<QT> act;
+  QT qc[4];
+  struct Regs {
+    X::Col x, y;
+    QT qi[2];
+  };
+  __device__ void load(int s, Regs& r) {
+    const int64_t i0 = act.row(s);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) r.qi[j] = Q[i0 + X::Col::k() + 32 * j];  // zeros up to whole 128-row tiles
+    r.x.load(A, lda, i0, m, k0, m);
+    r.y.load(G, ldg, i0, m, n0, ncols);
+  }
+  __device__ void finish(Regs& r) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r.x.v[j][e] *= (r.qi[j] * qc[e] > act.thr) ? 1.0f : 0.0f;
+  }
+};
+
+template <typename QT>
+__global__ __launch_bounds__(X::NTHR, 4) void screened_bwd_b_flex(const float* __restrict__ A, int64_t lda,
+                                                               const float* __restrict__ G, int64_t ldg,
+                                                               int64_t ncols, const QT* __restrict__ Q,
+                                                               const QT* __restrict__ qmax, QT thr, int64_t m,
+                                                               int nmt, int nnt, float* __restrict__ dB,
+                                                               int64_t lddb) {
+  __shared__ __attribute__((aligned(16))) float lds[X::LDS_FLOATS];
+  int64_t jt;
+  int nt;
+  if (!T32::tile_item(blockIdx.x, nmt, nnt, nullptr, jt, nt)) return;
+  const int64_t k0 = jt * X::TM, n0 = (int64_t)nt * X::TM;
+  FlexBwdB<QT> src{A, G, Q, lda, ldg, m, ncols, k0, n0, {qmax, (int)(k0 / TILE), thr}, {}};
+#pragma unroll
+  for (int c = 0; c < 4; ++c) src.qc[c] = Q[k0 + X::Col::i() + c];
+  float acc[8];
+  X::run(src, src.act.slabs((int)tsp::ceil_div(m, TILE), m), lds, acc);
+  const X::Out o;
+  const int64_t c = n0 + o.col;
+  if (c < ncols) {
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      const int64_t r = k0 + o.row(v);
+      if (r < m) dB[r * lddb + c] = acc[v];
+    }
+  }
+}
+
 // dA[r][c] = (sum_n G[r][n] B[c][n]) * mask(r, c)
 template <typename T, typename QT>
 __global__ __launch_bounds__(256) void screened_bwd_a_generic(const T* __restrict__ G, int64_t ldg,
@@ -712,8 +845,16 @@ int launch_backward(const void* A, int dtype, int64_t lda, const void* diag, dou
     return (ld % 4) == 0 && ((uintptr_t)p % 16) == 0 && (m + TILE) * ld * 4 + 4 * TILE <= (int64_t)UINT32_MAX;
   };
   const bool f32 = dtype == TSP_F32 && fits(G, ldg);
+  const int64_t nmt64 = tsp::ceil_div(m, X::TM);
   if (dA) {
-    if (f32 && fits(B, ldb)) {
+    if (dtype == TSP_F32 && (!(f32 && fits(B, ldb)) || small_tiles_faster(m, m, 68, 136, 18))) {
+      const int64_t grid = tsp::ceil_div(nmt64 * nmt64, 8) * 8;
+      if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm_backward: problem too large");
+      hipLaunchKernelGGL((screened_bwd_a_flex<QT>), dim3((unsigned)grid), dim3(X::NTHR), 0, st, (const float*)G, ldg,
+                         (const float*)B, ldb, ncols, (const QT*)Q, (const QT*)qmax, thr, m, (int)nmt64, (float*)dA,
+                         ldda);
+      rc = tsp::check_launch("screened_bwd_a_flex launch");
+    } else if (dtype == TSP_F32) {
       const int64_t grid = tsp::ceil_div(nmt * nmt, 8) * 8;
       if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm_backward: problem too large");
       hipLaunchKernelGGL((screened_bwd_a_f32<QT>), dim3((unsigned)grid), dim3(256), 0, st, (const float*)G, ldg,
@@ -723,19 +864,21 @@ int launch_backward(const void* A, int dtype, int64_t lda, const void* diag, dou
     } else {
       const int64_t grid = tsp::ceil_div(m * m, 256);
       if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm_backward: problem too large");
-      if (dtype == TSP_F32)
-        hipLaunchKernelGGL((screened_bwd_a_generic<float, QT>), dim3((unsigned)grid), dim3(256), 0, st,
-                           (const float*)G, ldg, (const float*)B, ldb, ncols, (const QT*)Q, thr, m, (float*)dA, ldda);
-      else
-        hipLaunchKernelGGL((screened_bwd_a_generic<double, QT>), dim3((unsigned)grid), dim3(256), 0, st,
-                           (const double*)G, ldg, (const double*)B, ldb, ncols, (const QT*)Q, thr, m, (double*)dA,
-                           ldda);
+      hipLaunchKernelGGL((screened_bwd_a_generic<double, QT>), dim3((unsigned)grid), dim3(256), 0, st,
+                         (const double*)G, ldg, (const double*)B, ldb, ncols, (const QT*)Q, thr, m, (double*)dA, ldda);
       rc = tsp::check_launch("screened_bwd_a_generic launch");
     }
     if (rc) return rc;
   }
   if (dB) {
-    if (f32 && fits(A, lda)) {
+    if (dtype == TSP_F32 && (!(f32 && fits(A, lda)) || small_tiles_faster(m, ncols, 77, 154, 21))) {
+      const int64_t nnt = tsp::ceil_div(ncols, X::TM), grid = tsp::ceil_div(nmt64, 8) * 8 * nnt;
+      if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm_backward: problem too large");
+      hipLaunchKernelGGL((screened_bwd_b_flex<QT>), dim3((unsigned)grid), dim3(X::NTHR), 0, st, (const float*)A, lda,
+                         (const float*)G, ldg, ncols, (const QT*)Q, (const QT*)qmax, thr, m, (int)nmt64, (int)nnt,
+                         (float*)dB, lddb);
+      rc = tsp::check_launch("screened_bwd_b_flex launch");
+    } else if (dtype == TSP_F32) {
       const int64_t nnt = tsp::ceil_div(ncols, TILE);
       const int64_t grid = tsp::ceil_div(nmt, 8) * 8 * nnt;
       if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm_backward: problem too large");
@@ -746,13 +889,8 @@ int launch_backward(const void* A, int dtype, int64_t lda, const void* diag, dou
     } else {
       const int64_t grid = tsp::ceil_div(m * ncols, 256);
       if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm_backward: problem too large");
-      if (dtype == TSP_F32)
-        hipLaunchKernelGGL((screened_bwd_b_generic<float, QT>), dim3((unsigned)grid), dim3(256), 0, st,
-                           (const float*)A, lda, (const float*)G, ldg, ncols, (const QT*)Q, thr, m, (float*)dB, lddb);
-      else
-        hipLaunchKernelGGL((screened_bwd_b_generic<double, QT>), dim3((unsigned)grid), dim3(256), 0, st,
-                           (const double*)A, lda, (const double*)G, ldg, ncols, (const QT*)Q, thr, m, (double*)dB,
-                           lddb);
+      hipLaunchKernelGGL((screened_bwd_b_generic<double, QT>), dim3((unsigned)grid), dim3(256), 0, st,
+                         (const double*)A, lda, (const double*)G, ldg, ncols, (const QT*)Q, thr, m, (double*)dB, lddb);
       rc = tsp::check_launch("screened_bwd_b_generic launch");
     }
     if (rc) return rc;
@@ -771,9 +909,20 @@ int launch(const void* A, int dtype, int64_t lda, const void* diag, double thr_s
   hipLaunchKernelGGL((screened_q<QT>), dim3((unsigned)nmt), dim3(TILE), 0, st, (const QT*)diag, m, Q, qmax);
   int rc = tsp::check_launch("screened_q launch");
   if (rc) return rc;
-  if (dtype == TSP_F32 && (lda % 4) == 0 && (ldb % 4) == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)B % 16) == 0 &&
-      (m + TILE) * lda * 4 + 4 * TILE <= (int64_t)UINT32_MAX && (m + TILE) * ldb * 4 + 4 * TILE <= (int64_t)UINT32_MAX) {
-    // (the streamed kernel's buffer offsets fit 32 bits)
+  // streamed fp32 kernel: 16-byte aligned rows, buffer offsets within 32 bits
+  const bool fits = (lda % 4) == 0 && (ldb % 4) == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)B % 16) == 0 &&
+                    (m + TILE) * lda * 4 + 4 * TILE <= (int64_t)UINT32_MAX &&
+                    (m + TILE) * ldb * 4 + 4 * TILE <= (int64_t)UINT32_MAX;
+  if (dtype == TSP_F32 && (!fits || small_tiles_faster(m, ncols, 88, 139, 21))) {
+    const int64_t nmt64 = tsp::ceil_div(m, X::TM), nnt = tsp::ceil_div(ncols, X::TM);
+    const int64_t grid = tsp::ceil_div(nmt64, 8) * 8 * nnt;
+    if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm: problem too large");
+    hipLaunchKernelGGL((screened_f32_flex<QT>), dim3((unsigned)grid), dim3(X::NTHR), 0, st, (const float*)A, lda,
+                       (const QT*)Q, (const QT*)qmax, thr, m, (const float*)B, ldb, ncols, (float*)C, ldc, (int)nmt64,
+                       (int)nnt);
+    return tsp::check_launch("screened_f32_flex launch");
+  }
+  if (dtype == TSP_F32) {
     const int64_t nnt = tsp::ceil_div(ncols, TILE);
     const int64_t grid = tsp::ceil_div(nmt, 8) * 8 * nnt;
     if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm: problem too large");
@@ -781,15 +930,6 @@ int launch(const void* A, int dtype, int64_t lda, const void* diag, double thr_s
                        (const QT*)Q, (const QT*)qmax, thr, m, (const float*)B, ldb, ncols, (float*)C, ldc, (int)nmt,
                        (int)nnt);
     return tsp::check_launch("screened_f32_dma launch");
-  }
-  if (dtype == TSP_F32 && (lda % 4) == 0 && (ldb % 4) == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)B % 16) == 0) {
-    const int64_t nnt = tsp::ceil_div(ncols, T32::BN);
-    const int64_t grid = tsp::ceil_div(nmt, 8) * 8 * nnt;
-    if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm: problem too large");
-    hipLaunchKernelGGL((screened_f32_mfma<QT>), dim3((unsigned)grid), dim3(T32::NTHR), 0, st, (const float*)A, lda,
-                       (const QT*)Q, (const QT*)qmax, thr, m, (const float*)B, ldb, ncols, (float*)C, ldc, (int)nmt,
-                       (int)nnt);
-    return tsp::check_launch("screened_f32_mfma launch");
   }
   if (dtype == TSP_F64 && (m % 2) == 0 && (lda % 2) == 0 && (ldb % 2) == 0 && ((uintptr_t)A % 16) == 0 &&
       ((uintptr_t)B % 16) == 0 && (m + TILE) * lda * 8 + 8 * TILE <= (int64_t)UINT32_MAX &&
@@ -804,12 +944,8 @@ int launch(const void* A, int dtype, int64_t lda, const void* diag, double thr_s
   }
   const int64_t grid = tsp::ceil_div(m * ncols, 256);
   if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm: problem too large for the generic kernel");
-  if (dtype == TSP_F32)
-    hipLaunchKernelGGL((screened_generic<float, QT>), dim3((unsigned)grid), dim3(256), 0, st, (const float*)A, lda,
-                       (const QT*)Q, thr, m, (const float*)B, ldb, ncols, (float*)C, ldc);
-  else
-    hipLaunchKernelGGL((screened_generic<double, QT>), dim3((unsigned)grid), dim3(256), 0, st, (const double*)A, lda,
-                       (const QT*)Q, thr, m, (const double*)B, ldb, ncols, (double*)C, ldc);
+  hipLaunchKernelGGL((screened_generic<double, QT>), dim3((unsigned)grid), dim3(256), 0, st, (const double*)A, lda,
+                     (const QT*)Q, thr, m, (const double*)B, ldb, ncols, (double*)C, ldc);
   return tsp::check_launch("screened_generic launch");
 }
 
