@@ -278,3 +278,39 @@ def test_small_blocks_at_scale(hip_backend, b, dtype):
         exact = Gi @ Bj.transpose(0, 2, 1)
         scale = np.abs(Gi) @ np.abs(Bj).transpose(0, 2, 1)
         assert ref.scaled_error(dA[s0:s0 + 4096], exact, scale) <= tol
+
+
+@pytest.mark.parametrize("b", [16, 32, 64, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("mb,nbc,cut,N", [(1, 1, 0, 1), (3, 2, 5, 63), (2, 5, 1, 65), (70, 3, 0, 130), (3, 140, 7, 129)])
+def test_small_tiles_edges(hip_backend, b, dtype, mb, nbc, cut, N):
+    """The small-tile kernels (bsr_flex.hip), forward and both gradients, at
+    odd column counts around their tiles and slabs, ragged m and n (`cut`
+    rows and columns short of whole blocks), empty block rows and lists past
+    64 entries; operands one element into their buffers. Tolerances as for
+    the other cases: the scale of each element's products."""
+    if b == 128 and mb * nbc > 100:
+        mb, nbc = min(mb, 67), min(nbc, 66)
+    g = torch.Generator().manual_seed(b + N)
+    keep = torch.rand(mb, nbc, generator=g) < 0.8
+    keep[0, 0] = True
+    if mb > 2:
+        keep[1] = False
+    bsr = W.bsr_from_block_mask(keep, b)
+    m, n = mb * b - cut, nbc * b - cut
+    blocks = torch.randn(bsr.n_blocks, b, b, generator=g).to(dtype)
+    bsr = ts.BSRMatrix(blocks, bsr.block_col_indices, bsr.block_row_ptrs, (m, n), b)
+
+    def odd(rows):
+        return torch.randn(rows * N + 1, generator=g).to(dtype).cuda()[1:].view(rows, N)
+
+    B, G = odd(n).requires_grad_(True), odd(m)
+    Ad = ts.BSRMatrix(blocks.cuda().requires_grad_(True), bsr.block_col_indices, bsr.block_row_ptrs, (m, n), b)
+    C = ts.bsr_spmm(Ad, B)
+    db, dB = torch.autograd.grad(C, (Ad.blocks, B), G)
+    args = (_np(blocks), bsr.block_col_indices.numpy(), bsr.block_row_ptrs.numpy(), (m, n), b, _np(B))
+    assert ref.scaled_error(_np(C), ref.bsr_spmm(*args), ref.bsr_spmm(*args, absolute=True)) <= TOL[dtype]
+    exact_b, exact_B = ref.bsr_spmm_backward(*args, _np(G))
+    scale_b, scale_B = ref.bsr_spmm_backward(*args, _np(G), absolute=True)
+    assert ref.scaled_error(_np(db), exact_b, scale_b) <= TOL[dtype]
+    assert ref.scaled_error(_np(dB), exact_B, scale_B) <= TOL[dtype]

@@ -31,24 +31,27 @@
 //                        v_mfma_f32_32x32x16_bf16 (operand forms at the kernels).
 //   bsr_sddmm_f64_mfma / bsr_spmm_t_f64_mfma   b == 128, fp64: the same two
 //                        products on v_mfma_f64_16x16x4_f64.
-//   bsr_sddmm_small<b>   b in {8, 16, 32, 64}, fp32 / bf16: a wavefront per
-//                        stored block on fp32 MFMAs, operands straight from
-//                        memory (details at the kernel); dB at these block
-//                        sizes is bsr_spmm.hip's small-block kernel walking
-//                        the block-column view with A transposed.
+//   bsr_sddmm_small<b>   b in {8, 16, 32}, fp32 / bf16 with few columns: a
+//                        wavefront per stored block on fp32 MFMAs, operands
+//                        straight from memory (details at the kernel); dB at
+//                        b = 8 and 16 is bsr_spmm.hip's small-block kernel
+//                        walking the block-column view with A transposed.
+//   bsr_flex             (bsr_flex.hip) both products on tiles of at most
+//                        64x64, for fp32 and bf16 at b = 16, 32, 64, 128
+//                        where the kernels above do not apply or leave CUs
+//                        idle.
 //   bsr_sddmm_generic / bsr_spmm_t_generic   any block size, f32 / f64 / bf16
 //                        (accumulating in f32, f64 for f64): one thread per
 //                        output element.
 #include "common.h"
 
 #include "lds_dma.h"
-#include "mfma_f32.h"
+#include "tile_item.h"
 #include "mfma_f64.h"
 #include "f32_pair_tiles.h"
 
 namespace {
 
-namespace T32 = tsp::f32tile;
 using tsp::dma::i32x4;
 using namespace tsp::f32pair;
 
@@ -134,7 +137,7 @@ __global__ __launch_bounds__(256) void bsr_spmm_t_f32_dma(
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NST * STAGE];
   int64_t col;
   int ntile;
-  if (!T32::tile_item(blockIdx.x, nbc, nt, order, col, ntile)) return;
+  if (!tsp::tile_item(blockIdx.x, nbc, nt, order, col, ntile)) return;
   const int64_t n0 = (int64_t)ntile * BS;
   const int64_t start = cp[col];
   const int nblk = (int)(cp[col + 1] - start);
@@ -565,7 +568,7 @@ __global__ __launch_bounds__(256) void bsr_spmm_t_bf16_mfma(
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NST * S::STAGE];
   int64_t col;
   int ntile;
-  if (!T32::tile_item(blockIdx.x, nbc, nt, order, col, ntile)) return;
+  if (!tsp::tile_item(blockIdx.x, nbc, nt, order, col, ntile)) return;
   const int64_t n0 = (int64_t)ntile * BS;
   const int64_t start = cp[col];
   const int nblk = (int)(cp[col + 1] - start);
@@ -706,7 +709,7 @@ __global__ __launch_bounds__(256) void bsr_spmm_t_f64_mfma(
   __shared__ __attribute__((aligned(1024))) uint8_t lds[f64b::NST * f64b::STAGE];
   int64_t col;
   int ntile;
-  if (!T32::tile_item(blockIdx.x, nbc, nt, order, col, ntile)) return;
+  if (!tsp::tile_item(blockIdx.x, nbc, nt, order, col, ntile)) return;
   const int64_t n0 = (int64_t)ntile * BS;
   const int64_t start = cp[col];
   const int nblk = (int)(cp[col + 1] - start);
@@ -807,15 +810,15 @@ __global__ __launch_bounds__(256) void bsr_spmm_t_generic(const T* __restrict__ 
 
 // ---------------------------------------------------------- small blocks
 //
-// bsr_sddmm_small<b>: dA for b = 8, 16, 32, 64 (fp32 or bf16, fp32
+// bsr_sddmm_small<b>: dA for b = 8, 16, 32 (fp32 or bf16, fp32
 // accumulation): a wavefront per stored block k = (i, j), four per
 // workgroup, XCD x taking the x-th eighth of the blocks (neighbouring blocks
 // share block rows). dA_k = dC[rows of i] . B[rows of j]^T over the N
 // columns; both operands are rows with k contiguous, so each lane reads 4
 // consecutive k of its dC row and of its B row per step (k permuted the same
 // way on both operands, so the products pair up):
-//   b = 32, 64: v_mfma_f32_32x32x2_f32, (b/32)^2 subtiles; lane half h takes
-//     k = 8g + 4h + c at step (g, c);
+//   b = 32: v_mfma_f32_32x32x2_f32; lane half h takes k = 8g + 4h + c at step
+//     (g, c);
 //   b = 16: v_mfma_f32_16x16x4_f32; lane group q takes k = 16g + 4q + c;
 //   b = 8: v_mfma_f32_4x4x1_16b_f32, its 16 products = 2 x 2 subtiles of
 //     4x4 x 4 k-slices: lane l feeds product l/4 = (k-slice s = (l/4) % 4,
@@ -835,7 +838,7 @@ __device__ inline f32x4 ld4v<uint16_t>(const uint16_t* p) {
 }
 
 // k steps of operands in flight per lane (small-block dA kernels): 3 measured
-// no faster at b = 8, 16, 32 and slower at b = 64 (more registers)
+// no faster at b = 8, 16, 32
 constexpr int SDDMM_PF = 1;
 
 template <int BSZ, typename T>
@@ -843,7 +846,7 @@ __global__ __launch_bounds__(256) void bsr_sddmm_small(const T* __restrict__ G, 
                                                        const T* __restrict__ B, int64_t ldb, int64_t n, int64_t ncols,
                                                        const int64_t* __restrict__ brow, const int64_t* __restrict__ ci,
                                                        int64_t nnzb, T* __restrict__ out, int vec) {
-  static_assert(BSZ == 8 || BSZ == 16 || BSZ == 32 || BSZ == 64, "block size");
+  static_assert(BSZ == 8 || BSZ == 16 || BSZ == 32, "block size");
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t per = gridDim.x >> 3;
   const int64_t kb = ((int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3)) * 4 + w;
@@ -1084,10 +1087,8 @@ int launch_sddmm_small(int64_t bs, const void* G, int64_t ldg, int64_t m, const 
     TSP_SD_SMALL(8);
   else if (bs == 16)
     TSP_SD_SMALL(16);
-  else if (bs == 32)
-    TSP_SD_SMALL(32);
   else
-    TSP_SD_SMALL(64);
+    TSP_SD_SMALL(32);
 #undef TSP_SD_SMALL
   return tsp::check_launch("bsr_sddmm_small launch");
 }
@@ -1106,6 +1107,23 @@ extern "C" int tsp_bsr_sddmm(const void* G, int64_t ldg, int64_t m, const void* 
   if (n_blocks == 0) return TSP_OK;
   if (!G || !B || !block_rows || !block_col_indices || !grad_blocks) return tsp::fail(TSP_EINVAL, "tsp_bsr_sddmm: null pointer");
   hipStream_t st = (hipStream_t)stream;
+  // Small tiles (bsr_flex.hip). At b = 128 the streamed fp32 kernel forms one
+  // 128x128 block per CU at a time, so the fullest CU counts: ns per column of
+  // dC, measured, 68 per block on a CU against 18 per 64x64 part. 8192^2, 10 %
+  // blocks (410), N = 512: 73 against 73 us; 320 blocks 73 against 52; 512
+  // blocks 76 against 83; 19 blocks (N = 256) 19 against 8. Below b = 64 a
+  // wavefront per block wins for few columns: 8192^2, 10 % blocks of 32, N = 64
+  // 20 against 26 us, N = 512 124 against 93; of 16, N = 128 53 against 53, N =
+  // 512 194 against 132.
+  const bool flex = (dtype == TSP_F32 || dtype == TSP_BF16) &&
+                    (block_size == BS || block_size == 64 || ((block_size == 16 || block_size == 32) && ncols >= 128));
+  auto run_flex = [&] {
+    return tsp::launch_bsr_flex_sddmm(dtype, block_size, G, ldg, m, B, ldb, n, ncols, block_rows, block_col_indices,
+                                      n_blocks, grad_blocks, st);
+  };
+  if (flex && dtype == TSP_F32 && block_size == BS &&
+      68 * tsp::ceil_div(n_blocks, 256) > 18 * tsp::ceil_div(4 * n_blocks, 256))
+    return run_flex();
   if (dtype == TSP_F32 && block_size == BS && ncols % 4 == 0 && ldg % 4 == 0 && ldb % 4 == 0 && aligned16(G) &&
       aligned16(B) && (m + BS) * ldg * 4 <= (int64_t)UINT32_MAX - 64 && (n + BS) * ldb * 4 <= (int64_t)UINT32_MAX - 64) {
     const int64_t grid = tsp::ceil_div(n_blocks, 8) * 8;
@@ -1131,7 +1149,8 @@ extern "C" int tsp_bsr_sddmm(const void* G, int64_t ldg, int64_t m, const void* 
                        (const double*)B, ldb, n, ncols, block_rows, block_col_indices, n_blocks, (double*)grad_blocks);
     return tsp::check_launch("bsr_sddmm_f64_mfma launch");
   }
-  if (block_size == 8 || block_size == 16 || block_size == 32 || block_size == 64) {
+  if (flex) return run_flex();
+  if (block_size == 8 || block_size == 16 || block_size == 32) {
     if (dtype == TSP_F32)
       return launch_sddmm_small<float>(block_size, G, ldg, m, B, ldb, n, ncols, block_rows, block_col_indices, n_blocks,
                                        grad_blocks, st);
@@ -1219,6 +1238,15 @@ extern "C" int tsp_bsr_spmm_t(const void* blocks, int dtype, const int64_t* col_
   // blocks is only read for stored blocks (it may be null for an empty pattern)
   if (!col_ptrs || !col_block_ids || !col_block_rows || !out || !X) return tsp::fail(TSP_EINVAL, "tsp_bsr_spmm_t: null pointer");
   hipStream_t st = (hipStream_t)stream;
+  // Small tiles (bsr_flex.hip), as in the forward: 8192^2, 10 % blocks, N = 512
+  // (256 tiles) 102 against 82 us; 16384^2, N = 512 (512 tiles) 246 against 281.
+  const bool flex = (dtype == TSP_F32 || dtype == TSP_BF16) && tsp::ceil_div(m, block_size) <= INT32_MAX &&
+                    (block_size == 16 || block_size == 32 || block_size == 64 || block_size == BS);
+  auto run_flex = [&] {
+    return tsp::launch_bsr_flex_t(dtype, block_size, blocks, col_ptrs, col_block_rows, col_block_ids, n_block_cols, m,
+                                  n, X, ldx, ncols, out, ldo, col_order, st);
+  };
+  if (flex && dtype == TSP_F32 && block_size == BS && n_block_cols * tsp::ceil_div(ncols, BS) < 400) return run_flex();
   if (dtype == TSP_F32 && block_size == BS && ldx % 4 == 0 && aligned16(X) && aligned16(blocks) &&
       (m + BS) * ldx * 4 + 4 * BS <= (int64_t)UINT32_MAX) {
     const int64_t nt = tsp::ceil_div(ncols, BS);
@@ -1249,10 +1277,10 @@ extern "C" int tsp_bsr_spmm_t(const void* blocks, int dtype, const int64_t* col_
                        (double*)out, ldo, n, col_order);
     return tsp::check_launch("bsr_spmm_t_f64_mfma launch");
   }
-  if ((block_size == 8 || block_size == 16 || block_size == 32 || block_size == 64) &&
-      (dtype == TSP_F32 || dtype == TSP_BF16))
+  if (dtype != TSP_F64 && tsp::small_blocks_whole(block_size, dtype == TSP_F32 ? 4 : 2, blocks, X, ldx, ncols))
     return tsp::launch_bsr_small_t(dtype, block_size, blocks, col_ptrs, col_block_rows, col_block_ids, n_block_cols, m,
                                    n, X, ldx, ncols, out, ldo, st);
+  if (flex) return run_flex();
   const int64_t grid = tsp::ceil_div(n * ncols, 256);
   if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsr_spmm_t: too large for the generic kernel");
 #define SPMMT_GEN(T)                                                                                                     \

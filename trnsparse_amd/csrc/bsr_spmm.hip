@@ -10,21 +10,20 @@
 // each workgroup reads the B row-panels of its block row in place.
 //
 // Kernels
-//   bsr_spmm_f32_mfma  b == 128, fp32.  One workgroup = one 128x128 tile of C
-//                      (block row i, column tile t). 8 waves in a 4(M)x2(N)
-//                      grid, each wave a 32x64 sub-tile as two 32x32 MFMA
-//                      accumulators (v_mfma_f32_32x32x2_f32). The K loop runs
-//                      over the row's blocks in 64-wide k-slabs staged through
-//                      a double-buffered LDS ring (137 KiB: one workgroup per
-//                      CU); the next slab's loads are in flight while the
-//                      current one is consumed.
+//   bsr_spmm_f32_dma   b == 128, fp32 with 16-byte aligned rows and enough
+//                      128x128 tiles of C to fill the chip: one tile per
+//                      workgroup, streamed through LDS (below).
+//   bsr_flex           (bsr_flex.hip) fp32 MFMA on tiles of at most 64x64:
+//                      b == 128 otherwise, b == 64 and 32, b == 16 for rows
+//                      and column counts that the small-block kernel does not
+//                      read whole.
 //   bsr_spmm_bf16_mfma b == 128, bf16 in, fp32 accumulation, fp32/bf16 out
 //                      (v_mfma_f32_32x32x16_bf16, 64x32 wave tiles,
 //                      direct-to-LDS 4-deep ring, B operand through LDS
 //                      transpose reads).
 //   bsr_spmm_f64_dma   b == 128, fp64 (v_mfma_f64_16x16x4_f64, the streamed
 //                      structure of bsr_spmm_f32_dma).
-//   bsr_spmm_small<b>  b in {8, 16, 32, 64}, fp32 or bf16 in (fp32 MFMA,
+//   bsr_spmm_small<b>  b in {8, 16}, fp32 or bf16 in (fp32 MFMA,
 //                      bf16 widened exactly at the load), fp32 / bf16 out: a
 //                      wavefront per (block row, 64 columns of C), operands
 //                      straight from memory into MFMA registers (b = 8 on
@@ -35,81 +34,24 @@
 // Scheduling: rows are ranked heaviest first (tsp_bsr_row_order) and dealt
 // to the 8 XCDs in boustrophedon order; the column tiles of one block row sit
 // in consecutive slots of one XCD, so the tiles sharing an A block run side
-// by side on one L2 (mfma_f32.h, tile_item). With one workgroup per CU the
+// by side on one L2 (tile_item.h). With one workgroup per CU the
 // in-order hardware dispatcher is then a longest-processing-time list
 // scheduler within each XCD.
 #include "common.h"
 
 #include "lds_dma.h"
-#include "mfma_f32.h"
+#include "tile_item.h"
 #include "mfma_f64.h"
 
 namespace {
 
-namespace T32 = tsp::f32tile;
 constexpr int BS = 128;  // block size served by the MFMA kernels
-constexpr int KC = 64;   // fp32 k-slab (two slabs per stored block)
-
-// Slab source of one (block row, column tile) item: slab s is k-slab s%2 of
-// the (s/2)-th stored block of the row; B rows come straight from the
-// row-panel of that block's column (no gathered copy of B).
-struct BsrSlabs {
-  const float* __restrict__ blocks;
-  const int64_t* __restrict__ ci;
-  const float* __restrict__ B;
-  int64_t start, n, ncols, ldb, n0;
-  T32::Coords<KC> q;
-  __device__ void load(int s, f32x4 (&a)[T32::Slab<KC>::NA], f32x4 (&b)[T32::Slab<KC>::NB]) const {
-    const int64_t idx = start + s / (BS / KC);
-    const int kk = (s % (BS / KC)) * KC;
-    const float* ab = blocks + idx * (BS * BS) + kk + q.ac;
-#pragma unroll
-    for (int i = 0; i < T32::Slab<KC>::NA; ++i) a[i] = *(const f32x4*)(ab + (q.ar + i * q.astep) * BS);
-    const int64_t brow = ci[idx] * BS + kk + q.br;
-#pragma unroll
-    for (int i = 0; i < T32::Slab<KC>::NB; ++i) b[i] = T32::load4_guard(B, brow + 16 * i, n0 + q.bc, n, ncols, ldb);
-  }
-};
-
-template <typename OutT>
-__device__ inline OutT cvt_out(float v);
-template <>
-__device__ inline float cvt_out<float>(float v) { return v; }
-template <>
-__device__ inline uint16_t cvt_out<uint16_t>(float v) { return tsp::f32_to_bf16_bits(v); }
-
-template <typename OutT>
-__global__ __launch_bounds__(T32::NTHR) void bsr_spmm_f32_mfma(
-    const float* __restrict__ blocks, const int64_t* __restrict__ rp, const int64_t* __restrict__ ci,
-    int64_t mb, int nt, int64_t m, int64_t n, const float* __restrict__ B, int64_t ldb,
-    int64_t ncols, OutT* __restrict__ C, int64_t ldc, const int32_t* __restrict__ order) {
-  __shared__ __attribute__((aligned(16))) float lds[T32::Slab<KC>::LDS_FLOATS];
-  int64_t row;
-  int ntile;
-  if (!T32::tile_item(blockIdx.x, mb, nt, order, row, ntile)) return;
-
-  BsrSlabs src;
-  src.blocks = blocks;
-  src.ci = ci;
-  src.B = B;
-  src.start = rp[row];
-  src.n = n;
-  src.ncols = ncols;
-  src.ldb = ldb;
-  src.n0 = (int64_t)ntile * T32::BN;
-  const int nsteps = (int)(rp[row + 1] - src.start) * (BS / KC);
-
-  f32x16 acc0 = {}, acc1 = {};
-  T32::run<KC>(src, nsteps, lds, src.q, acc0, acc1);
-  T32::store_tile(C, ldc, row * BS, src.n0, m, ncols, src.q, acc0, acc1, cvt_out<OutT>);
-}
 
 // ------------------------------------------------------- fp32 MFMA, streamed
 //
 // bsr_spmm_f32_dma<KC>: b == 128, fp32. Same tile (128x128 of C per
 // workgroup, one block row x one 128-column tile) and scheduling (tile_item:
-// heaviest rows first, boustrophedon over the XCDs) as bsr_spmm_f32_mfma,
-// restructured for issue efficiency:
+// heaviest rows first, boustrophedon over the XCDs) as the other kernels:
 //   * 4 waves, each a 64x64 sub-tile as four independent 32x32
 //     v_mfma_f32_32x32x2_f32 accumulators: per 8 k a wave reads two 16-byte
 //     A fragments and four 8-byte B pairs for 16 MFMAs. The two column
@@ -158,7 +100,7 @@ __global__ __launch_bounds__(256) void bsr_spmm_f32_dma(
   __shared__ __attribute__((aligned(1024))) uint8_t lds[G::NST * G::STAGE];
   int64_t row;
   int ntile;
-  if (!T32::tile_item(blockIdx.x, mb, nt, order, row, ntile)) return;
+  if (!tsp::tile_item(blockIdx.x, mb, nt, order, row, ntile)) return;
   const int64_t n0 = (int64_t)ntile * 128;
   const int64_t start = rp[row];
   const int nblk = (int)(rp[row + 1] - start);
@@ -324,7 +266,7 @@ __global__ __launch_bounds__(256) void bsr_spmm_f64_dma(
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NST * STAGE];
   int64_t row;
   int ntile;
-  if (!T32::tile_item(blockIdx.x, mb, nt, order, row, ntile)) return;
+  if (!tsp::tile_item(blockIdx.x, mb, nt, order, row, ntile)) return;
   const int64_t n0 = (int64_t)ntile * 128;
   const int64_t start = rp[row];
   const int nblk = (int)(rp[row + 1] - start);
@@ -452,7 +394,7 @@ __global__ __launch_bounds__(512) void bsr_spmm_bf16_mfma(
   __shared__ __attribute__((aligned(1024))) uint8_t lds[bf::NST * bf::STAGE];
   int64_t row;
   int ntile;
-  if (!T32::tile_item(blockIdx.x, mb, nt, order, row, ntile)) return;
+  if (!tsp::tile_item(blockIdx.x, mb, nt, order, row, ntile)) return;
   const int64_t n0 = (int64_t)ntile * 128;
   const int64_t start = rp[row];
   const int nblk = (int)(rp[row + 1] - start);
@@ -468,9 +410,9 @@ __global__ __launch_bounds__(512) void bsr_spmm_bf16_mfma(
   // on the slab path.
   if (nblk <= 0) {
     // empty block row: zero tile
-    f32x16 z = {};
-    T32::Coords<64> q;
-    T32::store_tile(C, ldc, row * BS, n0, m, ncols, q, z, z, cvt_out<OutT>);
+    const int64_t c = n0 + (tid & 127);
+    for (int64_t r = row * BS + (tid >> 7); r < row * BS + BS && r < m; r += 4)
+      if (c < ncols) C[r * ldc + c] = tsp::from_acc<OutT>(0.f);
     return;
   }
   int cbase = 0;
@@ -572,25 +514,19 @@ __global__ __launch_bounds__(512) void bsr_spmm_bf16_mfma(
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const int64_t r = r0 + 8 * (v >> 2) + (v & 3);
-      if (r < m) C[r * ldc + c0] = cvt_out<OutT>(acc0[v]);
-      if (r + 32 < m) C[(r + 32) * ldc + c0] = cvt_out<OutT>(acc1[v]);
+      if (r < m) C[r * ldc + c0] = tsp::from_acc<OutT>(acc0[v]);
+      if (r + 32 < m) C[(r + 32) * ldc + c0] = tsp::from_acc<OutT>(acc1[v]);
     }
   }
 }
 
 // ------------------------------------------------------ small block sizes
 //
-// bsr_spmm_small<BSZ>: b = 8, 16, 32 or 64. A block row of C is only b rows, so
+// bsr_spmm_small<BSZ>: b = 8 or 16. A block row of C is only b rows, so
 // a wavefront owns one (block row, 64-column) tile of C and walks the row's
 // stored blocks with its operands loaded directly into registers (4 waves
 // per workgroup take consecutive column tiles of one block row and share
 // its A blocks through L1):
-//   b = 32, 64: v_mfma_f32_32x32x2_f32, b/32 row subtiles x 2 column
-//     subtiles; at step 4g + c lane half h supplies k = 8g + 4h + c, so the
-//     lane's A values for four MFMAs are one 16-byte read of its block row
-//     (8 bytes for bf16); its column in subtile u is n0 + 2 (lane % 32) + u,
-//     so its B values of both subtiles are one 8-byte read of row
-//     8g + 4h + c;
 //   b = 8: v_mfma_f32_4x4x1_16b_f32 (16 products of 4x4 per instruction
 //     as 2 row groups x 8 column groups, 4 instructions per k for the 128
 //     columns), 8 k-steps per block; B rows as 16-byte reads split between
@@ -616,20 +552,6 @@ __device__ inline f32x4 load4_acc<uint16_t>(const uint16_t* p) {
                tsp::bf16_bits_to_f32(v[3])};
 }
 
-template <typename T>
-__device__ inline f32x2 load2_acc(const T* p);
-template <>
-__device__ inline f32x2 load2_acc<float>(const float* p) { return *(const f32x2*)p; }
-template <>
-__device__ inline f32x2 load2_acc<uint16_t>(const uint16_t* p) {
-  const uint32_t v = *(const uint32_t*)p;
-  return f32x2{tsp::bf16_bits_to_f32((uint16_t)(v & 0xffffu)), tsp::bf16_bits_to_f32((uint16_t)(v >> 16))};
-}
-// 2 consecutive outputs of one row as one store (8 bytes fp32, 4 bytes bf16)
-__device__ inline void store2_out(float* p, float a, float b) { *(f32x2*)p = f32x2{a, b}; }
-__device__ inline void store2_out(uint16_t* p, float a, float b) {
-  *(uint32_t*)p = (uint32_t)tsp::f32_to_bf16_bits(a) | ((uint32_t)tsp::f32_to_bf16_bits(b) << 16);
-}
 // 4 consecutive outputs of one row as one store (16 bytes fp32, 8 bytes bf16)
 __device__ inline void store4_out(float* p, f32x4 v) { *(f32x4*)p = v; }
 __device__ inline void store4_out(uint16_t* p, f32x4 v) {
@@ -649,7 +571,7 @@ __global__ __launch_bounds__(256) void bsr_spmm_small(const T* __restrict__ bloc
                                                       const T* __restrict__ B, int64_t ldb, int64_t ncols,
                                                       OutT* __restrict__ C, int64_t ldc, int64_t nct, int vec,
                                                       const int64_t* __restrict__ bid = nullptr) {
-  static_assert(BSZ == 8 || BSZ == 16 || BSZ == 32 || BSZ == 64, "block size");
+  static_assert(BSZ == 8 || BSZ == 16, "block size");
   constexpr int TW = BSZ == 8 ? 128 : 64;  // columns of C per wavefront
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   // XCD x (= blockIdx % 8) takes the x-th eighth of the workgroups in row
@@ -750,7 +672,7 @@ __global__ __launch_bounds__(256) void bsr_spmm_small(const T* __restrict__ bloc
           if (nc + u < ncols) cr[u] = tsp::from_acc<OutT>(acc[u][i]);
       }
     }
-  } else if constexpr (BSZ == 16) {
+  } else {
     // lane group q = lane / 16 supplies k = 4q + c at step c; lane l16's
     // column in subtile u is n0 + 4 l16 + u, so one 16-byte load per step
     // reads its B row's columns of all 4 subtiles
@@ -818,69 +740,6 @@ __global__ __launch_bounds__(256) void bsr_spmm_small(const T* __restrict__ bloc
           if (nc + u < ncols) cr[u] = tsp::from_acc<OutT>(acc[u][r]);
       }
     }
-  } else {
-    // lane half h supplies k = 8g + 4h + c at step (g, c); lane l32's column
-    // in subtile u is n0 + 2 l32 + u, so one 8-byte load per step reads its
-    // B row's columns of both subtiles
-    constexpr int RT = BSZ / 32;
-    const int h = lane >> 5, l32 = lane & 31;
-    const int64_t nc = n0 + 2 * l32;
-    const bool cfull = (vec & 4) && n0 + 64 <= ncols;
-    f32x16 acc[RT][2];
-#pragma unroll
-    for (int t = 0; t < RT; ++t) acc[t][0] = acc[t][1] = f32x16{};
-    for (int64_t idx = start; idx < end; ++idx) {
-      const int64_t kb = ci[idx] * BSZ;
-      const bool bfull = cfull && kb + BSZ <= n;
-      const T* Ab = block_of(idx);
-#pragma unroll
-      for (int g = 0; g < BSZ / 8; ++g) {
-        f32x4 a[RT];
-#pragma unroll
-        for (int t = 0; t < RT; ++t) {
-          if constexpr (TA) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) a[t][c] = aop(Ab, 32 * t + l32, 8 * g + 4 * h + c);
-          } else {
-            a[t] = load4_acc<T>(Ab + (32 * t + l32) * BSZ + 8 * g + 4 * h);
-          }
-        }
-        f32x2 bv[4];
-        if (bfull) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) bv[c] = load2_acc<T>(B + (kb + 8 * g + 4 * h + c) * ldb + nc);
-        } else {
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int u = 0; u < 2; ++u) bv[c][u] = bval(kb + 8 * g + 4 * h + c, nc + u);
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-          for (int t = 0; t < RT; ++t)
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-              acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t][c], bv[c][u], acc[t][u], 0, 0, 0);
-      }
-    }
-    // element v of subtile (t, u): row 32t + 8(v/4) + 4h + v%4, column n0 + 2 l32 + u
-    const bool vstore = cfull && (vec & 8);
-#pragma unroll
-    for (int t = 0; t < RT; ++t)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t rr = row * BSZ + 32 * t + 8 * (v >> 2) + 4 * h + (v & 3);
-        if (rr >= m) continue;
-        OutT* cr = C + rr * ldc + nc;
-        if (vstore) {
-          store2_out(cr, acc[t][0][v], acc[t][1][v]);
-        } else {
-#pragma unroll
-          for (int u = 0; u < 2; ++u)
-            if (nc + u < ncols) cr[u] = tsp::from_acc<OutT>(acc[t][u][v]);
-        }
-      }
   }
 }
 
@@ -891,23 +750,16 @@ int launch_small(int64_t bs, const void* blocks, const int64_t* rp, const int64_
   const int64_t nct = tsp::ceil_div(ncols, bs == 8 ? 128 : 64);
   const int64_t grid = tsp::ceil_div(tsp::ceil_div(mb * nct, 4), 8) * 8;
   if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsr_spmm: problem too large");
-  // bits 0 / 1: B rows read / C rows written 4 columns at a time (b = 8, 16);
-  // bits 2 / 3: 2 columns at a time (b = 32, 64)
+  // bits 0 / 1: B rows read / C rows written 4 columns at a time
   const int vec = (((uintptr_t)B % (4 * sizeof(T))) == 0 && ldb % 4 == 0 ? 1 : 0) |
-                  (((uintptr_t)C % (4 * sizeof(OutT))) == 0 && ldc % 4 == 0 ? 2 : 0) |
-                  (((uintptr_t)B % (2 * sizeof(T))) == 0 && ldb % 2 == 0 ? 4 : 0) |
-                  (((uintptr_t)C % (2 * sizeof(OutT))) == 0 && ldc % 2 == 0 ? 8 : 0);
+                  (((uintptr_t)C % (4 * sizeof(OutT))) == 0 && ldc % 4 == 0 ? 2 : 0);
 #define TSP_SMALL(BSZ)                                                                                     \
   hipLaunchKernelGGL((bsr_spmm_small<BSZ, T, OutT, TA>), dim3((unsigned)grid), dim3(256), 0, st, (const T*)blocks, \
                      rp, ci, mb, m, n, (const T*)B, ldb, ncols, (OutT*)C, ldc, nct, vec, bid)
   if (bs == 8)
     TSP_SMALL(8);
-  else if (bs == 16)
-    TSP_SMALL(16);
-  else if (bs == 32)
-    TSP_SMALL(32);
   else
-    TSP_SMALL(64);
+    TSP_SMALL(16);
 #undef TSP_SMALL
   return tsp::check_launch("bsr_spmm_small launch");
 }
@@ -980,7 +832,17 @@ int launch_generic(const void* blocks, const int64_t* rp, const int64_t* ci, int
 
 }  // namespace
 
-// dB = A^T X for block sizes 8, 16, 32 and 64 (the backward of bsr_spmm):
+// At b = 16 the small-block kernel beats the tiles of bsr_flex where it reads
+// B rows in whole 16-byte pieces and its 64-column tiles are nearly full
+// (8192^2, 10 % blocks: N = 256 53 against 77 us, N = 64 37 against 45); reading
+// element by element it loses (N = 65 68 against 49, N = 509 247 against 168;
+// 3000^2, 20 %, N = 80 44 against 26).
+bool tsp::small_blocks_whole(int64_t b, int64_t elem, const void* blocks, const void* B, int64_t ldb, int64_t ncols) {
+  if ((uintptr_t)blocks % 16) return false;
+  return b == 8 || (b == 16 && (uintptr_t)B % (4 * elem) == 0 && ldb % 4 == 0 && (ncols % 64 == 0 || ncols >= 256));
+}
+
+// dB = A^T X for block sizes 8 and 16 (the backward of bsr_spmm):
 // bsr_spmm_small over the block-column view with A transposed at the load.
 // X has m rows; dB has n rows. f32 in and out, or bf16 in and out.
 int tsp::launch_bsr_small_t(int dtype, int64_t bs, const void* blocks, const int64_t* col_ptrs,
@@ -1020,7 +882,19 @@ extern "C" int tsp_bsr_spmm(const void* blocks, int dtype, const int64_t* block_
   if (!block_row_ptrs || !C || (n > 0 && !B) || (n_blocks > 0 && (!blocks || !block_col_indices)))
     return tsp::fail(TSP_EINVAL, "tsp_bsr_spmm: null pointer");
   const int64_t mb = tsp::ceil_div(m, block_size);
-
+  // Block sizes of the small-tile kernels (bsr_flex.hip). At b = 128 the
+  // streamed fp32 kernel, one 128x128 tile per CU at a time, needs about 1.5
+  // tiles per CU: 8192^2, 10 % blocks, N = 512 (256 tiles) 103 against 81 us,
+  // N = 256 (128 tiles) 100 against 49; 12800 x 8192, 5 %, N = 512 (400 tiles)
+  // 63 against 64; 16384^2, N = 512 (512 tiles) 260 against 304.
+  const bool flex = (dtype == TSP_F32 || dtype == TSP_BF16) && n_blocks <= INT32_MAX &&
+                    tsp::ceil_div(n, block_size) <= INT32_MAX &&
+                    (block_size == 16 || block_size == 32 || block_size == 64 || block_size == BS);
+  auto run_flex = [&] {
+    return tsp::launch_bsr_flex(dtype, out_dtype, block_size, blocks, block_row_ptrs, block_col_indices, mb, m, n, B,
+                                ldb, ncols, C, ldc, row_order, st);
+  };
+  if (flex && dtype == TSP_F32 && block_size == BS && mb * tsp::ceil_div(ncols, 128) < 400) return run_flex();
   if (dtype == TSP_F32 && block_size == BS && (ldb % 4) == 0 && ((uintptr_t)B % 16) == 0 &&
       ((uintptr_t)blocks % 16) == 0 && (n + BS) * ldb * 4 + 4 * BS <= (int64_t)UINT32_MAX) {
     // (the kernel's B offsets, rows < n + 128 and columns < ldb + 128, fit 32 bits)
@@ -1030,16 +904,6 @@ extern "C" int tsp_bsr_spmm(const void* blocks, int dtype, const int64_t* block_
     hipLaunchKernelGGL(bsr_spmm_f32_dma<F32_DMA_KC>, dim3((unsigned)grid), dim3(256), 0, st, (const float*)blocks, block_row_ptrs,
                        block_col_indices, mb, (int)nt, m, n, (const float*)B, ldb, ncols, (float*)C, ldc, row_order);
     return tsp::check_launch("bsr_spmm_f32_dma launch");
-  }
-  if (dtype == TSP_F32 && block_size == BS && (ldb % 4) == 0 && ((uintptr_t)B % 16) == 0 &&
-      ((uintptr_t)blocks % 16) == 0) {
-    const int64_t nt = tsp::ceil_div(ncols, T32::BN);
-    const int64_t grid = tsp::ceil_div(mb, 8) * 8 * nt;
-    if (grid > INT32_MAX || nt > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsr_spmm: problem too large");
-    hipLaunchKernelGGL((bsr_spmm_f32_mfma<float>), dim3((unsigned)grid), dim3(T32::NTHR), 0, st, (const float*)blocks,
-                       block_row_ptrs, block_col_indices, mb, (int)nt, m, n, (const float*)B, ldb, ncols,
-                       (float*)C, ldc, row_order);
-    return tsp::check_launch("bsr_spmm_f32_mfma launch");
   }
   if (dtype == TSP_BF16 && block_size == BS && (ldb % 8) == 0 && ((uintptr_t)B % 16) == 0 &&
       ((uintptr_t)blocks % 16) == 0 && (n + BS) * ldb * 2 + 2 * BS <= (int64_t)UINT32_MAX) {
@@ -1067,7 +931,7 @@ extern "C" int tsp_bsr_spmm(const void* blocks, int dtype, const int64_t* block_
                        block_col_indices, mb, (int)nt, m, n, (const double*)B, ldb, ncols, (double*)C, ldc, row_order);
     return tsp::check_launch("bsr_spmm_f64_dma launch");
   }
-  if ((block_size == 8 || block_size == 16 || block_size == 32 || block_size == 64) && ((uintptr_t)blocks % 16) == 0) {
+  if (dtype != TSP_F64 && tsp::small_blocks_whole(block_size, dtype == TSP_F32 ? 4 : 2, blocks, B, ldb, ncols)) {
     if (dtype == TSP_F32)
       return launch_small<float, float>(block_size, blocks, block_row_ptrs, block_col_indices, mb, m, n, B, ldb, ncols,
                                         C, ldc, st);
@@ -1078,6 +942,7 @@ extern "C" int tsp_bsr_spmm(const void* blocks, int dtype, const int64_t* block_
       return launch_small<uint16_t, uint16_t>(block_size, blocks, block_row_ptrs, block_col_indices, mb, m, n, B, ldb,
                                               ncols, C, ldc, st);
   }
+  if (flex) return run_flex();
   if (dtype == TSP_F32) return launch_generic<float, float>(blocks, block_row_ptrs, block_col_indices, block_size, m, n, B, ldb, ncols, C, ldc, st);
   if (dtype == TSP_F64) return launch_generic<double, double>(blocks, block_row_ptrs, block_col_indices, block_size, m, n, B, ldb, ncols, C, ldc, st);
   if (out_dtype == TSP_F32) return launch_generic<uint16_t, float>(blocks, block_row_ptrs, block_col_indices, block_size, m, n, B, ldb, ncols, C, ldc, st);

@@ -31,11 +31,27 @@ int check_launch(const char* what);
 // instead of hipMemsetAsync so callers may capture the work in a HIP graph).
 int zero_fill(void* p, int64_t bytes, hipStream_t st);
 
-// dB = A^T X of bsr_spmm's backward at block sizes 8, 16, 32, 64 (fp32 or
+// Whether bsr_spmm_small serves these operands (block sizes 8 and 16; B or, in
+// the backward, dC).
+bool small_blocks_whole(int64_t b, int64_t elem, const void* blocks, const void* B, int64_t ldb, int64_t ncols);
+// dB = A^T X of bsr_spmm's backward at block sizes 8 and 16 (fp32 or
 // bf16 in and out), defined with the small-block forward kernel.
 int launch_bsr_small_t(int dtype, int64_t bs, const void* blocks, const int64_t* col_ptrs,
                        const int64_t* col_block_rows, const int64_t* col_block_ids, int64_t n_block_cols, int64_t m,
                        int64_t n, const void* X, int64_t ldx, int64_t ncols, void* out, int64_t ldo, hipStream_t st);
+
+// The BSR products on small tiles (bsr_flex.hip): block sizes 16, 32, 64, 128,
+// fp32 or bf16, any alignment; lists of fewer than 2^31 blocks.
+int launch_bsr_flex(int dtype, int out_dtype, int64_t b, const void* blocks, const int64_t* rp, const int64_t* ci,
+                    int64_t mb, int64_t m, int64_t n, const void* B, int64_t ldb, int64_t ncols, void* C, int64_t ldc,
+                    const int32_t* order, hipStream_t st);
+int launch_bsr_flex_t(int dtype, int64_t b, const void* blocks, const int64_t* col_ptrs,
+                      const int64_t* col_block_rows, const int64_t* col_block_ids, int64_t n_block_cols, int64_t m,
+                      int64_t n, const void* G, int64_t ldg, int64_t ncols, void* out, int64_t ldo,
+                      const int32_t* order, hipStream_t st);
+int launch_bsr_flex_sddmm(int dtype, int64_t b, const void* G, int64_t ldg, int64_t m, const void* B, int64_t ldb,
+                          int64_t n, int64_t ncols, const int64_t* brow, const int64_t* bcol, int64_t nnzb, void* out,
+                          hipStream_t st);
 
 // ---------------------------------------------------------------- bf16
 // Round-to-nearest-even fp32 -> bf16 bit pattern (NaN kept quiet), the same

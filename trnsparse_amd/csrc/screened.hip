@@ -34,13 +34,12 @@
 
 #include "f32_flex.h"
 #include "lds_dma.h"
-#include "mfma_f32.h"
+#include "tile_item.h"
 #include "mfma_f64.h"
 #include "f32_pair_tiles.h"
 
 namespace {
 
-namespace T32 = tsp::f32tile;
 constexpr int TILE = 128;
 
 template <typename QT>
@@ -103,7 +102,7 @@ __global__ __launch_bounds__(256) void screened_f32_dma(
   __shared__ __attribute__((aligned(16))) QT qs[2][SKC];
   int64_t mt64;
   int ntile;
-  if (!T32::tile_item(blockIdx.x, nmt, nnt, nullptr, mt64, ntile)) return;
+  if (!tsp::tile_item(blockIdx.x, nmt, nnt, nullptr, mt64, ntile)) return;
   const int mt = (int)mt64;
   const int64_t row0 = (int64_t)mt * TILE, n0 = (int64_t)ntile * TILE;
   const QT qI = qmax[mt];
@@ -252,7 +251,7 @@ __global__ __launch_bounds__(256) void screened_f64_dma(
   __shared__ __attribute__((aligned(16))) QT qs[2][F::KC];
   int64_t mt64;
   int ntile;
-  if (!T32::tile_item(blockIdx.x, nmt, nnt, nullptr, mt64, ntile)) return;
+  if (!tsp::tile_item(blockIdx.x, nmt, nnt, nullptr, mt64, ntile)) return;
   const int mt = (int)mt64;
   const int64_t row0 = (int64_t)mt * TILE, n0 = (int64_t)ntile * TILE;
   const QT qI = qmax[mt];
@@ -352,6 +351,10 @@ __global__ __launch_bounds__(256) void screened_f64_dma(
 // them: n = N = 1111 forward 767 -> 62 us, dA 4080 -> 54, dB 834 -> 64 against
 // one thread per output (host-timed calls, launch of screened_q included).
 namespace X = tsp::flex;
+constexpr int FT = 64;  // output tile: FT x FT
+typedef X::Split<32, FT, FT> FSplit;
+typedef X::Row<float, FT> FRow;
+typedef X::Col<float, FT, 32> FCol;
 constexpr int SPT = TILE / X::KC;  // slabs per 128-row tile
 
 // Whether aligned operands with a row_items x col_items output are faster on
@@ -366,7 +369,7 @@ constexpr int SPT = TILE / X::KC;  // slabs per 128-row tile
 // 4096 keeps 1249 (1358).
 bool small_tiles_faster(int64_t row_items, int64_t col_items, int one, int two, int small) {
   const int64_t big = tsp::ceil_div(tsp::ceil_div(row_items, TILE) * tsp::ceil_div(col_items, TILE), 256);
-  const int64_t tiny = tsp::ceil_div(tsp::ceil_div(row_items, X::TM) * tsp::ceil_div(col_items, X::TM), 256);
+  const int64_t tiny = tsp::ceil_div(tsp::ceil_div(row_items, FT) * tsp::ceil_div(col_items, FT), 256);
   return big / 2 * two + big % 2 * one > tiny * small;
 }
 
@@ -407,14 +410,14 @@ struct FlexFwd {
   ActiveTiles<QT> act;
   QT qr[2];
   struct Regs {
-    X::Row x;
-    X::Col y;
+    FRow x;
+    FCol y;
     QT qk[4];
   };
   __device__ void load(int s, Regs& r) {
     const int64_t k0 = act.row(s);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) r.qk[e] = Q[k0 + X::Row::k() + e];  // zeros up to whole 128-row tiles
+    for (int e = 0; e < 4; ++e) r.qk[e] = Q[k0 + FRow::k() + e];  // zeros up to whole 128-row tiles
     r.x.load(A, lda, row0, m, k0, m);
     r.y.load(B, ldb, k0, m, n0, ncols);
   }
@@ -422,7 +425,7 @@ struct FlexFwd {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) r.x.v[j][e] *= (qr[j] * r.qk[e] > act.thr) ? 1.0f : 0.0f;
+      for (int e = 0; e < 4; ++e) r.x.q[j].v[e] *= (qr[j] * r.qk[e] > act.thr) ? 1.0f : 0.0f;
   }
 };
 
@@ -431,23 +434,22 @@ __global__ __launch_bounds__(X::NTHR, 4) void screened_f32_flex(
     const float* __restrict__ A, int64_t lda, const QT* __restrict__ Q, const QT* __restrict__ qmax, QT thr,
     int64_t m, const float* __restrict__ B, int64_t ldb, int64_t ncols, float* __restrict__ C, int64_t ldc, int nmt,
     int nnt) {
-  __shared__ __attribute__((aligned(16))) float lds[X::LDS_FLOATS];
+  __shared__ __attribute__((aligned(16))) float lds[X::lds_floats<FRow, FCol>()];
   int64_t mt;
   int nt;
   // XCD-aware: the column tiles of one row panel of A share an XCD (and its L2)
-  if (!T32::tile_item(blockIdx.x, nmt, nnt, nullptr, mt, nt)) return;
-  const int64_t row0 = mt * X::TM, n0 = (int64_t)nt * X::TM;
+  if (!tsp::tile_item(blockIdx.x, nmt, nnt, nullptr, mt, nt)) return;
+  const int64_t row0 = mt * FT, n0 = (int64_t)nt * FT;
   FlexFwd<QT> src{A, B, Q, lda, ldb, m, ncols, row0, n0, {qmax, (int)(row0 / TILE), thr}, {}};
 #pragma unroll
-  for (int j = 0; j < 2; ++j) src.qr[j] = Q[row0 + X::Row::i() + 32 * j];
+  for (int j = 0; j < 2; ++j) src.qr[j] = Q[row0 + FRow::i() + 32 * j];
   float acc[8];
-  X::run(src, src.act.slabs((int)tsp::ceil_div(m, TILE), m), lds, acc);
-  const X::Out o;
-  const int64_t c = n0 + o.col;
+  X::run<FSplit>(src, src.act.slabs((int)tsp::ceil_div(m, TILE), m), lds, acc);
+  const int64_t c = n0 + FSplit::col();
   if (c < ncols) {
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      const int64_t r = row0 + o.row(v);
+      const int64_t r = row0 + FSplit::row(v);
       if (r < m) C[r * ldc + c] = acc[v];
     }
   }
@@ -604,7 +606,7 @@ __global__ __launch_bounds__(256) void screened_bwd_b_f32(const float* __restric
   // XCD-aware: the column tiles of one row tile J share an XCD (and A's panel in its L2)
   int64_t jt64;
   int ntile;
-  if (!T32::tile_item(blockIdx.x, nmt, nnt, nullptr, jt64, ntile)) return;
+  if (!tsp::tile_item(blockIdx.x, nmt, nnt, nullptr, jt64, ntile)) return;
   const int J = (int)jt64;
   const int64_t k0 = (int64_t)J * TILE, n0 = (int64_t)ntile * TILE;
   const QT qJ = qmax[J];
@@ -701,7 +703,7 @@ struct FlexBwdA {
   const float *G, *B;
   int64_t ldg, ldb, m, ncols, r0, c0;
   struct Regs {
-    X::Row x, y;
+    FRow x, y;
   };
   __device__ void load(int s, Regs& r) {
     r.x.load(G, ldg, r0, m, (int64_t)s * X::KC, ncols);
@@ -716,24 +718,23 @@ __global__ __launch_bounds__(X::NTHR, 4) void screened_bwd_a_flex(const float* _
                                                                int64_t ncols, const QT* __restrict__ Q,
                                                                const QT* __restrict__ qmax, QT thr, int64_t m,
                                                                int nmt, float* __restrict__ dA, int64_t ldda) {
-  __shared__ __attribute__((aligned(16))) float lds[X::LDS_FLOATS];
+  __shared__ __attribute__((aligned(16))) float lds[X::lds_floats<FRow, FRow>()];
   // XCD-aware: XCD x takes a contiguous range of tiles, as in screened_bwd_a_f32
   const int64_t ntiles = (int64_t)nmt * nmt, per = tsp::ceil_div(ntiles, 8);
   const int64_t slot = blockIdx.x >> 3, tix = (blockIdx.x & 7) * per + slot;
   if (slot >= per || tix >= ntiles) return;
-  const int64_t r0 = tix / nmt * X::TM, c0 = tix % nmt * X::TM;
+  const int64_t r0 = tix / nmt * FT, c0 = tix % nmt * FT;
   float acc[8] = {};
   if (qmax[r0 / TILE] * qmax[c0 / TILE] > thr) {  // else every pair is masked: zeros
     FlexBwdA src{G, B, ldg, ldb, m, ncols, r0, c0};
-    X::run(src, (int)tsp::ceil_div(ncols, X::KC), lds, acc);
+    X::run<FSplit>(src, (int)tsp::ceil_div(ncols, X::KC), lds, acc);
   }
-  const X::Out o;
-  const int64_t c = c0 + o.col;
+  const int64_t c = c0 + FSplit::col();
   if (c < m) {
     const QT qc = Q[c];
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      const int64_t r = r0 + o.row(v);
+      const int64_t r = r0 + FSplit::row(v);
       if (r < m) dA[r * ldda + c] = acc[v] * ((Q[r] * qc > thr) ? 1.0f : 0.0f);
     }
   }
@@ -748,13 +749,13 @@ struct FlexBwdB {
   ActiveTiles<QT> act;
   QT qc[4];
   struct Regs {
-    X::Col x, y;
+    FCol x, y;
     QT qi[2];
   };
   __device__ void load(int s, Regs& r) {
     const int64_t i0 = act.row(s);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) r.qi[j] = Q[i0 + X::Col::k() + 32 * j];  // zeros up to whole 128-row tiles
+    for (int j = 0; j < 2; ++j) r.qi[j] = Q[i0 + FCol::k() + 32 * j];  // zeros up to whole 128-row tiles
     r.x.load(A, lda, i0, m, k0, m);
     r.y.load(G, ldg, i0, m, n0, ncols);
   }
@@ -762,7 +763,7 @@ struct FlexBwdB {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) r.x.v[j][e] *= (r.qi[j] * qc[e] > act.thr) ? 1.0f : 0.0f;
+      for (int e = 0; e < 4; ++e) r.x.q[j].v[e] *= (r.qi[j] * qc[e] > act.thr) ? 1.0f : 0.0f;
   }
 };
 
@@ -773,22 +774,21 @@ __global__ __launch_bounds__(X::NTHR, 4) void screened_bwd_b_flex(const float* _
                                                                const QT* __restrict__ qmax, QT thr, int64_t m,
                                                                int nmt, int nnt, float* __restrict__ dB,
                                                                int64_t lddb) {
-  __shared__ __attribute__((aligned(16))) float lds[X::LDS_FLOATS];
+  __shared__ __attribute__((aligned(16))) float lds[X::lds_floats<FCol, FCol>()];
   int64_t jt;
   int nt;
-  if (!T32::tile_item(blockIdx.x, nmt, nnt, nullptr, jt, nt)) return;
-  const int64_t k0 = jt * X::TM, n0 = (int64_t)nt * X::TM;
+  if (!tsp::tile_item(blockIdx.x, nmt, nnt, nullptr, jt, nt)) return;
+  const int64_t k0 = jt * FT, n0 = (int64_t)nt * FT;
   FlexBwdB<QT> src{A, G, Q, lda, ldg, m, ncols, k0, n0, {qmax, (int)(k0 / TILE), thr}, {}};
 #pragma unroll
-  for (int c = 0; c < 4; ++c) src.qc[c] = Q[k0 + X::Col::i() + c];
+  for (int c = 0; c < 4; ++c) src.qc[c] = Q[k0 + FCol::i() + c];
   float acc[8];
-  X::run(src, src.act.slabs((int)tsp::ceil_div(m, TILE), m), lds, acc);
-  const X::Out o;
-  const int64_t c = n0 + o.col;
+  X::run<FSplit>(src, src.act.slabs((int)tsp::ceil_div(m, TILE), m), lds, acc);
+  const int64_t c = n0 + FSplit::col();
   if (c < ncols) {
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      const int64_t r = k0 + o.row(v);
+      const int64_t r = k0 + FSplit::row(v);
       if (r < m) dB[r * lddb + c] = acc[v];
     }
   }
@@ -845,7 +845,7 @@ int launch_backward(const void* A, int dtype, int64_t lda, const void* diag, dou
     return (ld % 4) == 0 && ((uintptr_t)p % 16) == 0 && (m + TILE) * ld * 4 + 4 * TILE <= (int64_t)UINT32_MAX;
   };
   const bool f32 = dtype == TSP_F32 && fits(G, ldg);
-  const int64_t nmt64 = tsp::ceil_div(m, X::TM);
+  const int64_t nmt64 = tsp::ceil_div(m, FT);
   if (dA) {
     if (dtype == TSP_F32 && (!(f32 && fits(B, ldb)) || small_tiles_faster(m, m, 68, 136, 18))) {
       const int64_t grid = tsp::ceil_div(nmt64 * nmt64, 8) * 8;
@@ -872,7 +872,7 @@ int launch_backward(const void* A, int dtype, int64_t lda, const void* diag, dou
   }
   if (dB) {
     if (dtype == TSP_F32 && (!(f32 && fits(A, lda)) || small_tiles_faster(m, ncols, 77, 154, 21))) {
-      const int64_t nnt = tsp::ceil_div(ncols, X::TM), grid = tsp::ceil_div(nmt64, 8) * 8 * nnt;
+      const int64_t nnt = tsp::ceil_div(ncols, FT), grid = tsp::ceil_div(nmt64, 8) * 8 * nnt;
       if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm_backward: problem too large");
       hipLaunchKernelGGL((screened_bwd_b_flex<QT>), dim3((unsigned)grid), dim3(X::NTHR), 0, st, (const float*)A, lda,
                          (const float*)G, ldg, ncols, (const QT*)Q, (const QT*)qmax, thr, m, (int)nmt64, (int)nnt,
@@ -914,7 +914,7 @@ int launch(const void* A, int dtype, int64_t lda, const void* diag, double thr_s
                     (m + TILE) * lda * 4 + 4 * TILE <= (int64_t)UINT32_MAX &&
                     (m + TILE) * ldb * 4 + 4 * TILE <= (int64_t)UINT32_MAX;
   if (dtype == TSP_F32 && (!fits || small_tiles_faster(m, ncols, 88, 139, 21))) {
-    const int64_t nmt64 = tsp::ceil_div(m, X::TM), nnt = tsp::ceil_div(ncols, X::TM);
+    const int64_t nmt64 = tsp::ceil_div(m, FT), nnt = tsp::ceil_div(ncols, FT);
     const int64_t grid = tsp::ceil_div(nmt64, 8) * 8 * nnt;
     if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm: problem too large");
     hipLaunchKernelGGL((screened_f32_flex<QT>), dim3((unsigned)grid), dim3(X::NTHR), 0, st, (const float*)A, lda,

@@ -157,10 +157,13 @@ at::Tensor bsr_sddmm_meta(const at::Tensor& G, const at::Tensor&, const at::Tens
 at::Tensor bsr_spmm_t(const at::Tensor& blocks, const at::Tensor& cp, const at::Tensor& cbid, const at::Tensor& crow,
                       const at::Tensor& col_order, int64_t m, int64_t n, int64_t block_size, const at::Tensor& G) {
   for (auto* p : {&blocks, &cp, &cbid, &crow, &col_order}) need(*p, G, "pattern");
-  need(G, G, "dC");
   TORCH_CHECK(m >= 0 && n >= 0 && block_size > 0, "bsr_spmm_t: bad sizes");
   TORCH_CHECK(G.dim() == 2 && G.size(0) == m, "bsr_spmm_t: grad_out has shape ", G.sizes(), ", expected [", m,
               ", N]");
+  // (a padded grad_out is passed as its first N columns: the row stride stays)
+  const int64_t ldg = m > 1 ? G.stride(0) : G.size(1);
+  TORCH_CHECK((G.size(1) <= 1 || G.stride(1) == 1) && ldg >= G.size(1),
+              "bsr_spmm_t: grad_out must have unit column stride and rows that do not overlap");
   TORCH_CHECK(blocks.dim() == 3 && blocks.size(1) == block_size && blocks.size(2) == block_size,
               "bsr_spmm_t: blocks has shape ", blocks.sizes());
   need_dtype(blocks, G.scalar_type(), "bsr_spmm_t", "blocks (the dtype of grad_out)");
@@ -176,7 +179,7 @@ at::Tensor bsr_spmm_t(const at::Tensor& blocks, const at::Tensor& cp, const at::
   const int64_t ncols = G.size(1), nbc = cp.numel() - 1;
   auto out = at::empty({n, ncols}, G.options());
   check(tsp_bsr_spmm_t(blocks.data_ptr(), dtype_code(blocks.scalar_type()), cp.data_ptr<int64_t>(),
-                       cbid.data_ptr<int64_t>(), crow.data_ptr<int64_t>(), nbc, block_size, m, n, G.data_ptr(), ncols,
+                       cbid.data_ptr<int64_t>(), crow.data_ptr<int64_t>(), nbc, block_size, m, n, G.data_ptr(), ldg,
                        ncols, out.data_ptr(), ncols, col_order.numel() ? col_order.data_ptr<int32_t>() : nullptr,
                        stream_of(G)),
         "tsp_bsr_spmm_t");

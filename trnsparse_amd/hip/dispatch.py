@@ -110,14 +110,26 @@ def _bsr_spmm_launch(blocks, rp, ci, order, shape, b, B, out_dtype, dev) -> torc
                   blocks_d.shape[0], b, m, n, x.data_ptr(), 1.0, None, 0.0, None, 0.0, None, 0.0, C.data_ptr(),
                   order.data_ptr() if order is not None else None, _lib.stream_handle(dev))
         return C
-    ldb = ncols
-    vec = {torch.float32: 4, torch.bfloat16: 8, torch.float64: 2}.get(B_d.dtype)
-    if vec and b == 128 and ncols % vec:
-        # Row stride a multiple of 16 bytes for the vectorised B panel loads.
-        B_d = F.pad(B_d, (0, vec - ncols % vec))
-        ldb = B_d.shape[1]
-    # (a padded B is passed as its first ncols columns: the row stride stays ldb)
+    # (a padded B is passed as its first ncols columns: the row stride stays)
+    B_d = _pad_rows(B_d, b, blocks_d.numel())
     return _lib.ops().bsr_spmm(blocks_d, rp, ci, order, m, n, b, B_d[:, :ncols], out_dtype)
+
+
+def _pad_rows(t: torch.Tensor, b: int, block_elements: int, backward: bool = False) -> torch.Tensor:
+    """t (rows, N) with its row stride zero-padded to a multiple of 16 bytes
+    where the products over it then run on the 128x128-tile kernels and that
+    pays for the copy; the small-tile kernels take any stride, at the fp32
+    MFMA rate. bf16 forward: always (1896 x 3907, 113 blocks: N = 391 46 us
+    unpadded, 25 padded, N = 97 42 and 22); its gradients from about 1 GFLOP a
+    product (N = 391 55 and 39 us, N = 97 35 and 38); fp32 where 128x128 tiles
+    fill the chip (16384^2, 1638 blocks, N = 511: 300 and 254 us; 8192^2, 410
+    blocks: 80 and 98); fp64 always: it has no other MFMA kernel."""
+    ncols = t.shape[1]
+    vec = {torch.float32: 4, torch.bfloat16: 8, torch.float64: 2}.get(t.dtype, 1)
+    least = {torch.float32: 1e10, torch.bfloat16: 1e9 if backward else 0.0}.get(t.dtype, 0.0)
+    if b != 128 or ncols % vec == 0 or 2.0 * block_elements * ncols < least:
+        return t
+    return F.pad(t, (0, vec - ncols % vec))
 
 
 class _BSRSpMMFunction(torch.autograd.Function):
@@ -164,12 +176,14 @@ class _BSRSpMMFunction(torch.autograd.Function):
             G = _on(grad_out, dev, dt)
             brow, cp, cbid, crow, corder = _bsr_bwd_plan(rp, ci, mb, nbc, dev)
             grad_blocks = grad_B = None
+            Gp = _pad_rows(G, b, blocks.numel(), backward=True)
             if ctx.needs_input_grad[0]:
-                Bd = _on(B, dev, dt)
-                gb = _lib.ops().bsr_sddmm(G, Bd, brow, ci, m, n, b)
+                # (zero columns of dC and B add nothing to the products)
+                Bd = _pad_rows(_on(B, dev, dt), b, blocks.numel(), backward=True)
+                gb = _lib.ops().bsr_sddmm(Gp, Bd, brow, ci, m, n, b)
                 grad_blocks = gb.to(A_blocks.device)
             if ctx.needs_input_grad[5]:
-                dB = _lib.ops().bsr_spmm_t(blocks, cp, cbid, crow, corder, m, n, b, G)
+                dB = _lib.ops().bsr_spmm_t(blocks, cp, cbid, crow, corder, m, n, b, Gp[:, :ncols])
                 grad_B = dB.to(B.device, B.dtype)
         return grad_blocks, None, None, None, None, grad_B, None, None
 
