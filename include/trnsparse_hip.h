@@ -142,6 +142,14 @@ int tsp_bsr_col_view(const int64_t* block_row_ptrs,
                      int64_t* col_ptrs, int64_t* col_block_ids,
                      int64_t* col_block_rows, void* workspace,
                      int64_t workspace_bytes, void* stream);
+/* tsp_bsr_col_plan: tsp_bsr_col_view and, on its col_ptrs, tsp_bsr_row_order
+ *   (col_order, (n_block_cols,) int32), in one launch for small patterns.
+ *   workspace: tsp_bsr_col_plan_workspace_size bytes (0 for those). */
+int64_t tsp_bsr_col_plan_workspace_size(int64_t nnzb, int64_t n_block_rows, int64_t n_block_cols);
+int tsp_bsr_col_plan(const int64_t* block_row_ptrs, const int64_t* block_col_indices, int64_t n_block_rows,
+                     int64_t n_block_cols, int64_t nnzb, int64_t* block_rows, int64_t* col_ptrs,
+                     int64_t* col_block_ids, int64_t* col_block_rows, int32_t* col_order, void* workspace,
+                     int64_t workspace_bytes, void* stream);
 int tsp_bsr_sddmm(const void* G, int64_t ldg, int64_t m,
                   const void* B, int64_t ldb, int64_t n, int64_t ncols,
                   const int64_t* block_rows, const int64_t* block_col_indices,

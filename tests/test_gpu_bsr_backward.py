@@ -203,6 +203,22 @@ def test_block_column_view(mb, nbc, p):
     assert sorted(corder.cpu().numpy().tolist()[:nbc]) == list(range(nbc))
 
 
+@pytest.mark.parametrize("mb,nbc,p", [(128, 128, 1.0), (128, 129, 1.0), (4096, 4, 0.7), (4097, 3, 0.7), (3, 4096, 0.9),
+                                      (3, 4097, 0.9), (1, 4000, 1.0), (65, 9, 0.5)])
+def test_block_column_view_limits(mb, nbc, p):
+    """The same at and just past the sizes that the one-launch plan takes
+    (16384 blocks, 4096 rows and columns), and the columns ordered by length."""
+    from trnsparse_amd.hip import dispatch as D
+
+    test_block_column_view(mb, nbc, p)
+    mask = torch.rand(mb, nbc, generator=torch.Generator().manual_seed(3)) < p
+    A = W.bsr_from_block_mask(mask, 1)
+    rp, ci = A.block_row_ptrs.cuda(), A.block_col_indices.cuda()
+    _, cp, _, _, corder = D._bsr_bwd_plan(rp, ci, mb, nbc, torch.device("cuda"))
+    lens = cp.diff()[corder[:nbc].long()].clamp(max=1023)  # (the order does not tell longer columns apart)
+    assert bool((lens[1:] <= lens[:-1]).all())
+
+
 @pytest.mark.parametrize("b", [8, 16, 64, 128])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_sddmm_blocks_in_any_order(hip_backend, b, dtype):

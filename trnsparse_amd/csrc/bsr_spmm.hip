@@ -801,14 +801,21 @@ __global__ __launch_bounds__(1024) void bsr_row_order_kernel(const int64_t* __re
     atomicAdd(&cnt[bin], 1);
   }
   __syncthreads();
-  if (tid == 0) {
-    int run = 0;
-    for (int i = 0; i < NBIN; ++i) {
-      int c = cnt[i];
-      cnt[i] = run;
-      run += c;
-    }
+  // exclusive scan of the counts, one bin per thread (a serial scan by one
+  // thread was 7 of this kernel's 9.4 us on 128 rows)
+  const int lane = tid & 63, w = tid >> 6, own = cnt[tid];
+  int incl = own;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int below = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += below;
   }
+  __shared__ int wtot[NBIN / 64];
+  if (lane == 63) wtot[w] = incl;
+  __syncthreads();
+  int before = 0;
+  for (int i = 0; i < w; ++i) before += wtot[i];
+  cnt[tid] = before + incl - own;
   __syncthreads();
   for (int64_t r = tid; r < mb; r += blockDim.x) {
     int64_t len = rp[r + 1] - rp[r];

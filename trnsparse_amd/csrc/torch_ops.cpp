@@ -126,6 +126,40 @@ at::Tensor bsr_spmm_meta(const at::Tensor& blocks, const at::Tensor&, const at::
   return at::empty({m, B.size(1)}, B.options().dtype(out_dtype));
 }
 
+// (block_rows, col_ptrs, col_block_ids, col_block_rows, col_order)
+typedef std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor> ColPlan;
+
+ColPlan bsr_col_plan_empty(const at::Tensor& ci, int64_t nbc) {
+  const int64_t nnzb = ci.numel();
+  return ColPlan(at::empty({nnzb}, ci.options()), at::empty({nbc + 1}, ci.options()), at::empty({nnzb}, ci.options()),
+                 at::empty({nnzb}, ci.options()), at::empty({nbc > 0 ? nbc : 1}, ci.options().dtype(at::kInt)));
+}
+
+ColPlan bsr_col_plan(const at::Tensor& rp, const at::Tensor& ci, int64_t n_block_cols) {
+  need(rp, ci, "block_row_ptrs");
+  need(ci, ci, "block_col_indices");
+  need_dtype(rp, at::kLong, "bsr_col_plan", "block_row_ptrs");
+  need_dtype(ci, at::kLong, "bsr_col_plan", "block_col_indices");
+  TORCH_CHECK(rp.numel() >= 1 && n_block_cols >= 0, "bsr_col_plan: bad sizes");
+  const int64_t nnzb = ci.numel(), mb = rp.numel() - 1;
+  ColPlan out = bsr_col_plan_empty(ci, n_block_cols);
+  const int64_t wsb = tsp_bsr_col_plan_workspace_size(nnzb, mb, n_block_cols);
+  TORCH_CHECK(wsb >= 0, "tsp_bsr_col_plan_workspace_size failed for ", nnzb, " blocks, ", n_block_cols,
+              " block columns: ", tsp_last_error());
+  at::Tensor ws;
+  if (wsb > 0) ws = at::empty({wsb}, ci.options().dtype(at::kByte));
+  check(tsp_bsr_col_plan(rp.data_ptr<int64_t>(), ci.data_ptr<int64_t>(), mb, n_block_cols, nnzb,
+                         std::get<0>(out).data_ptr<int64_t>(), std::get<1>(out).data_ptr<int64_t>(),
+                         std::get<2>(out).data_ptr<int64_t>(), std::get<3>(out).data_ptr<int64_t>(),
+                         std::get<4>(out).data_ptr<int32_t>(), wsb > 0 ? ws.data_ptr() : nullptr, wsb, stream_of(ci)),
+        "tsp_bsr_col_plan");
+  return out;
+}
+
+ColPlan bsr_col_plan_meta(const at::Tensor&, const at::Tensor& ci, int64_t n_block_cols) {
+  return bsr_col_plan_empty(ci, n_block_cols);
+}
+
 at::Tensor bsr_sddmm(const at::Tensor& G, const at::Tensor& B, const at::Tensor& block_rows,
                      const at::Tensor& block_col_indices, int64_t m, int64_t n, int64_t block_size) {
   need(G, G, "dC");
@@ -463,6 +497,8 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> bsa_bwd_meta(
 TORCH_LIBRARY(trnsparse_hip, m) {
   m.def("bsr_spmm(Tensor blocks, Tensor block_row_ptrs, Tensor block_col_indices, Tensor? row_order, int m, int n, "
         "int block_size, Tensor B, ScalarType out_dtype) -> Tensor");
+  m.def("bsr_col_plan(Tensor block_row_ptrs, Tensor block_col_indices, int n_block_cols) -> (Tensor, Tensor, Tensor, "
+        "Tensor, Tensor)");
   m.def("bsr_sddmm(Tensor grad_out, Tensor B, Tensor block_rows, Tensor block_col_indices, int m, int n, "
         "int block_size) -> Tensor");
   m.def("bsr_spmm_t(Tensor blocks, Tensor col_ptrs, Tensor col_block_ids, Tensor col_block_rows, Tensor col_order, "
@@ -486,6 +522,7 @@ TORCH_LIBRARY(trnsparse_hip, m) {
 // the "CUDA" dispatch key is the GPU key of PyTorch-ROCm
 TORCH_LIBRARY_IMPL(trnsparse_hip, CUDA, m) {
   m.impl("bsr_spmm", &bsr_spmm);
+  m.impl("bsr_col_plan", &bsr_col_plan);
   m.impl("bsr_sddmm", &bsr_sddmm);
   m.impl("bsr_spmm_t", &bsr_spmm_t);
   m.impl("csr_spmv", &csr_spmv);
@@ -499,6 +536,7 @@ TORCH_LIBRARY_IMPL(trnsparse_hip, CUDA, m) {
 
 TORCH_LIBRARY_IMPL(trnsparse_hip, Meta, m) {
   m.impl("bsr_spmm", &bsr_spmm_meta);
+  m.impl("bsr_col_plan", &bsr_col_plan_meta);
   m.impl("bsr_sddmm", &bsr_sddmm_meta);
   m.impl("bsr_spmm_t", &bsr_spmm_t_meta);
   m.impl("csr_spmv", &csr_spmv_meta);
