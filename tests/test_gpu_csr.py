@@ -148,6 +148,44 @@ def test_csr_matmul_backward_on_device(hip_backend, N, index_dtype):
 # ---------------------------------------------------- partition edge cases
 
 
+@pytest.mark.parametrize("N", [1, 2, 3, 5, 6, 7, 9, 31, 33, 127, 129])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_spmm_any_width(hip_backend, N, offset):
+    """Column counts that are no multiple of 4 and operands on 4-byte
+    boundaries, forward (with alpha, beta C) and both gradients: the last
+    column part overlaps its neighbour. An infinity in one column stays in
+    that column. fp32 sums of at most 70 products: TOL on the absolute ones."""
+    rng = np.random.default_rng(N)
+    lens = rng.poisson(6, size=150)
+    lens[:4] = (0, 70, 1, 64)
+    v, c, p = W.random_csr(lens, 90, rng)
+    A = W.csr_matrix_from_arrays(v, c, p, (150, 90), device="cuda")
+    A.values.requires_grad_(True)
+
+    def operand(rows):
+        t = torch.from_numpy(rng.standard_normal(rows * N + offset, dtype=np.float32)).cuda()
+        return t[offset:].view(rows, N)
+
+    B, C, G = operand(90).requires_grad_(True), operand(150), operand(150)
+    out = ts.spmm(A, B, 1.5, C, -0.5)
+    dv, dB = torch.autograd.grad(out, (A.values, B), G)
+    Bn, Cn, Gn = (t.detach().cpu().numpy() for t in (B, C, G))
+    args = (v, c, p, (150, 90))
+    exact, scale = (ref.csr_spmm(*args, Bn, 1.5, Cn, -0.5, absolute=a) for a in (False, True))
+    assert ref.scaled_error(out.detach().cpu().numpy(), exact, scale) <= TOL
+    rows = np.repeat(np.arange(150), lens)
+    prod = 1.5 * Gn[rows].astype(np.float64) * Bn[c]
+    assert ref.scaled_error(dv.cpu().numpy(), prod.sum(1), np.abs(prod).sum(1)) <= TOL
+    D = np.zeros((150, 90))
+    D[rows, c] = v
+    assert ref.scaled_error(dB.cpu().numpy(), 1.5 * D.T @ Gn, np.abs(1.5 * D.T) @ np.abs(Gn) + 1e-300) <= TOL
+    if N > 1:
+        Bi = B.detach().clone()
+        Bi[:, 0] = float("inf")
+        again = ts.spmm(A, Bi, 1.5, C, -0.5)
+        assert torch.equal(again[:, 1:], out.detach()[:, 1:])
+
+
 def _csr_from_lengths(lens, n, seed, index_dtype=np.int64):
     vals, cols, ptr = W.random_csr(lens, n, np.random.default_rng(seed))
     return W.csr_matrix_from_arrays(vals, cols.astype(index_dtype), ptr.astype(index_dtype), (len(lens), n))
