@@ -16,14 +16,14 @@
 //
 // Kernels
 //   bsa_bwd_d             D in the accumulation type (f32; f64 for f64).
-//   bsa_bwd_dq_bf16_d128  bf16, b = 128, d = 128: workgroup per (head, query
-//       block row), wavefront per 32 queries; per 64-key half
+//   bsa_bwd_dq_bf16<D>  bf16, b = 128, D in {64, 128}: workgroup per (head,
+//       query block row), wavefront per 32 queries; per 64-key half
 //       S^T = K Q^T and dP^T = V dO^T on v_mfma_f32_32x32x16_bf16 with the
 //       wave's Q and dO rows in registers, P and dS in registers, then
 //       dQ^T += K^T dS^T with K read through ds_read_b64_tr_b16. K/V halves
 //       stream through a 4-stage LDS ring by direct buffer loads three
 //       halves ahead.
-//   bsa_bwd_dkdv_bf16_d128  same shapes: workgroup per (head, key block
+//   bsa_bwd_dkdv_bf16<D>  same shapes: workgroup per (head, key block
 //       column) over the block-column view of the mask, wavefront per 32 keys;
 //       per 64-query half S = Q K^T and dP = dO V^T with the wave's K and V
 //       rows in registers, then dV^T += dO^T P and dK^T += Q^T dS with Q and
@@ -38,9 +38,13 @@
 //       head_dim: one thread per (row, 32-wide slice of head_dim).
 // Swizzle: K (row pass) and Q, dO (column pass) are read both as 16-byte rows
 // (16 consecutive keys of one chunk) and through transpose reads (4
-// consecutive keys, 4 chunks); slot = chunk ^ (((key % 4) << 2) | ((key / 4) %
-// 4)) is conflict-free for both on the 64-bank LDS. V in the row pass is only
-// read as rows: slot = chunk ^ (key % 16).
+// consecutive keys, 4 chunks); abw::swz gives slots that are conflict-free for
+// both on the 64-bank LDS. V in the row pass is only read as rows, in the same
+// slots.
+// At d = 64 the operands used to be zero-padded to 128 (half of every product,
+// and 13 pad and slice launches): on 16 heads of 4096, window 4 and 2 global
+// blocks, both passes with the padding took 202 us, 81 at their own width; 11
+// heads of 7296, window 8, 395 and 181.
 #include <new>
 
 #include "common.h"
@@ -203,17 +207,20 @@ int launch_generic(const void* Q, const void* K, const void* V, const void* dO, 
   return tsp::check_launch("bsa_bwd_dkdv_generic launch");
 }
 
-// ------------------------------------------------------- bf16 MFMA, d = 128
+// --------------------------------------------- bf16 MFMA, d = 64 and 128
 
 namespace abw {
-constexpr int D = 128;
 constexpr int BS = 128;             // block size served by the MFMA kernels
 constexpr int HR = 64;              // rows (keys in the row pass, queries in the column pass) per ring stage
-constexpr int ROWB = D * 2;         // bytes per row
-constexpr int HBYTES = HR * ROWB;   // 16 KiB
-constexpr int KS = D / 16;          // k-steps over head_dim
-constexpr int NU = D / 32;          // 32-wide head_dim subtiles
 constexpr int SEG_MAX = 64;         // most block rows one column-pass item walks
+template <int D>
+struct Geo {
+  static constexpr int ROWB = D * 2;                // bytes per row
+  static constexpr int HBYTES = HR * ROWB;          // a half: 64 rows
+  static constexpr int KS = D / 16;                 // k-steps over head_dim
+  static constexpr int NU = D / 32;                 // 32-wide head_dim subtiles
+  static constexpr int LOADS = 2 * HBYTES / 4096;   // 1-KiB loads per wave of two operands' halves
+};
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 typedef float f32x8 __attribute__((ext_vector_type(8)));
@@ -221,27 +228,28 @@ typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
 
 // The 16-byte chunk c of stage row r sits in slot c ^ swz(r). Rows are read
 // as 16-byte pieces of 16 consecutive rows (one chunk) and through transpose
-// reads of 4 consecutive rows (4 chunks); swz is a bijection on r % 16 whose
-// low two bits follow r / 4 and high two bits r % 4, so both access forms hit
-// 16 (resp. 4 x 4) distinct slots.
-__host__ __device__ constexpr int swz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
+// reads of 4 consecutive rows (4 chunks). At d = 128 (256-byte rows, 16
+// chunks) swz is a bijection on r % 16 whose low two bits follow r / 4 and
+// high two bits r % 4; at d = 64 two rows share the 64 banks and the 8 chunks
+// of a row follow r / 2: its parity in the high bit, r / 4 in the low two. So
+// both access forms hit 16 (resp. 4 x 4) distinct slots.
+template <int D>
+__host__ __device__ constexpr int swz(int r) {
+  return D == 128 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
+}
 
 // One wave's share (rows [16w, 16w + 16)) of a 64-row half starting at global
 // row row0 of the buffer `rs`, into the stage at LDS address dst.
+template <int D>
 __device__ inline void dma_half(tsp::dma::i32x4 rs, int64_t row0, uint32_t dst, int w, int lane) {
+  constexpr int ROWB = Geo<D>::ROWB, CPR = ROWB / 16, RPI = 64 / CPR;  // chunks per row, rows per instruction
 #pragma unroll
-  for (int qq = 0; qq < 4; ++qq) {
-    const int j = 4 * w + qq;
-    const int rr = 4 * j + (lane >> 4);
-    const int p = lane & 15;
-    tsp::dma::buffer16(rs, (uint32_t)((row0 + rr) * ROWB + ((p ^ swz(rr)) << 4)), dst + j * 1024);
+  for (int qq = 0; qq < Geo<D>::LOADS / 2; ++qq) {
+    const int j = Geo<D>::LOADS / 2 * w + qq;
+    const int rr = RPI * j + lane / CPR;
+    const int p = lane % CPR;
+    tsp::dma::buffer16(rs, (uint32_t)((row0 + rr) * ROWB + ((p ^ swz<D>(rr)) << 4)), dst + j * 1024);
   }
-}
-
-// A operand of v_mfma_f32_32x32x16_bf16 from stage rows r0 + [0, 32) (lane
-// row r0 + l32), head_dim chunk 2 ks + h: lane offset l32 * ROWB, kx = swz(l32) ^ h.
-__device__ inline bf16x8 row_read(const uint8_t* base, int loff, int kx, int r0, int ks) {
-  return *(const bf16x8*)(base + loff + r0 * ROWB + (((2 * ks) ^ kx) << 4));
 }
 
 // A operand holding the transpose: rows (MFMA i) are head_dim 32u + l32 and
@@ -253,6 +261,7 @@ struct TrLane {
   int off[2];
   int xu;
 };
+template <int D>
 __device__ inline TrLane tr_lane(int lane) {
   const int gq = lane >> 4, jq = lane & 15;
   const int c0 = 2 * (gq & 1) + ((jq & 3) >> 1);
@@ -260,21 +269,14 @@ __device__ inline TrLane tr_lane(int lane) {
 #pragma unroll
   for (int rr = 0; rr < 2; ++rr) {
     const int row = 8 * rr + 4 * (gq >> 1) + (jq >> 2);
-    t.off[rr] = row * ROWB + ((c0 ^ (swz(row) & 3)) << 4) + 8 * (jq & 1);
+    t.off[rr] = row * Geo<D>::ROWB + ((c0 ^ (swz<D>(row) & 3)) << 4) + 8 * (jq & 1);
   }
-  t.xu = jq >> 2;  // swz(row) >> 2
+  t.xu = D == 128 ? jq >> 2 : jq >> 3;  // swz(row) >> 2
   return t;
 }
-__device__ inline bf16x8 tr_read(const uint8_t* base, const TrLane& t, int r0, int u) {
-  s16x4 r[2];
-#pragma unroll
-  for (int rr = 0; rr < 2; ++rr)
-    r[rr] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(base + t.off[rr] + r0 * ROWB + ((u ^ t.xu) << 6)));
-  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(r[0], r[1], 0, 1, 2, 3, 4, 5, 6, 7));
-}
 // Address form of the two reads for the slot kernels. A stage starts at an
-// LDS address that is a multiple of 256 and rows are 256 bytes, so the
-// swizzled chunk bits (4-7) of a lane's address are free in the stage base:
+// LDS address that is a multiple of 256 and rows are 256 (d = 64: 128) bytes,
+// so the swizzled chunk bits (4-7, 4-6) of a lane's address are free in the stage base:
 // per step one base per access kind is formed (row reads: stage + l32 * ROWB
 // + swz(l32)^h in bits 4-7; transpose reads: stage + off[rr] + xu in bits
 // 6-7) and each read is base ^ (k-step or subtile bits) plus a constant row
@@ -311,19 +313,23 @@ constexpr int PF = 4;  // operand reads in flight
 // side share its K/V in L2). Wavefront w owns queries m * 128 + 32 w + [0, 32)
 // with their Q and dO rows in registers; 64-key halves of K and V stream
 // through a 4-stage LDS ring by direct buffer loads issued three halves ahead.
-// Per half, slots 0-31: S^T and dP^T tiles of the two 32-key tiles tt (16
-// MFMAs each, K / V rows as A, Q / dO as B); slots 16-39 also form P^T and
-// dS^T of tile 0 (slots 16-31) and tile 1 (32-39); slots 32-47: dQ^T += K^T
-// dS^T (K through transpose reads). Also computes D and leaves per-query
+// Per half (slots at d = 128), 0-31: S^T and dP^T tiles of the two 32-key
+// tiles tt (16 MFMAs each, K / V rows as A, Q / dO as B); slots 16-39 also form
+// P^T and dS^T of tile 0 (slots 16-31) and tile 1 (32-39); slots 32-47: dQ^T +=
+// K^T dS^T (K through transpose reads). Also computes D and leaves per-query
 // stats for the column pass: plane 0 r = log2e * row_max + log2 row_denom
 // (P = exp2(log2e * scale * s - r)), plane 1 D.
-__global__ __launch_bounds__(256, 1) void bsa_bwd_dq_bf16_d128(
+template <int D>
+__global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bsa_bwd_dq_bf16(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
     const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, int64_t S, int64_t H,
     const int64_t* __restrict__ rp, const int64_t* __restrict__ ci, int64_t Mt, float scale_log2, float scale,
     const float* __restrict__ rmax, const float* __restrict__ rden, float* __restrict__ qstat,
     uint16_t* __restrict__ dQ) {
   using namespace abw;
+  constexpr int ROWB = Geo<D>::ROWB, HBYTES = Geo<D>::HBYTES, KS = Geo<D>::KS, NU = Geo<D>::NU;
+  constexpr int LOADS = Geo<D>::LOADS;  // per wave and stage
+  constexpr int S1 = 4 * KS, SLOTS = S1 + 4 * NU;  // slots of the S^T / dP^T products; all
   constexpr int STAGE = 2 * HBYTES;  // K half, V half
   constexpr int NST = 4;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NST * STAGE];
@@ -372,13 +378,13 @@ __global__ __launch_bounds__(256, 1) void bsa_bwd_dq_bf16_d128(
   auto issue = [&](int s) {
     const int64_t key0 = key_of(s, cb_i, cv_i);
     const uint32_t st = lds0 + (s % NST) * STAGE;
-    dma_half(krs, key0, st, w, lane);
-    dma_half(vrs, key0, st + HBYTES, w, lane);
+    dma_half<D>(krs, key0, st, w, lane);
+    dma_half<D>(vrs, key0, st + HBYTES, w, lane);
   };
 
   const int loff = l32 * ROWB;
-  const int kx = swz(l32) ^ h;
-  const TrLane trl = tr_lane(lane);
+  const int kx = swz<D>(l32) ^ h;
+  const TrLane trl = tr_lane<D>(lane);
   float nr = 0.f;
 
   auto compute = [&](uint32_t st, int64_t key0) {
@@ -386,13 +392,13 @@ __global__ __launch_bounds__(256, 1) void bsa_bwd_dq_bf16_d128(
     const uint32_t rb = st + (uint32_t)(loff + (kx << 4));
     const uint32_t tb0 = st + (uint32_t)(trl.off[0] + (trl.xu << 6));
     const uint32_t tb1 = st + (uint32_t)(trl.off[1] + (trl.xu << 6));
-    // slot -> LDS operand: 0-31 S^T / dP^T of tile k / 16 (even: K row, odd:
-    // V row, k-step (k % 16) / 2); 32-47 K^T for dQ of tile (k - 32) / 8,
-    // k-step a = (k / 4) % 2, head_dim subtile u = k % 4
+    // slot -> LDS operand: k < S1 S^T / dP^T of tile k / (2 KS) (even: K row,
+    // odd: V row, k-step (k % (2 KS)) / 2); then, j = k - S1, K^T for dQ of
+    // tile j / (2 NU), k-step a = (j / NU) % 2, head_dim subtile u = j % NU
     auto fetch = [&](int k) -> bf16x8 {
-      if (k < 32) return lds_row(rb, (k & 15) >> 1, (k & 1) * HBYTES + 32 * (k >> 4) * ROWB);
-      const int j = k - 32;
-      return lds_trp(tb0, tb1, j & 3, (32 * (j >> 3) + 16 * ((j >> 2) & 1)) * ROWB);
+      if (k < S1) return lds_row(rb, k % (2 * KS) >> 1, (k & 1) * HBYTES + 32 * (k / (2 * KS)) * ROWB);
+      const int j = k - S1;
+      return lds_trp(tb0, tb1, j % NU, (32 * (j / (2 * NU)) + 16 * (j / NU % 2)) * ROWB);
     };
     f32x16 sc[2], dp[2];
     float pd[2][16];
@@ -412,24 +418,30 @@ __global__ __launch_bounds__(256, 1) void bsa_bwd_dq_bf16_d128(
         db[tt][v >> 3] = __builtin_convertvector(t, bf16x8);
       }
     };
-    tsp::static_for<48>([&](auto kc) __attribute__((always_inline)) {
+    tsp::static_for<SLOTS>([&](auto kc) __attribute__((always_inline)) {
       constexpr int k = decltype(kc)::value;
       const bf16x8 op = ring[k % PF];
-      if constexpr (k + PF < 48) ring[k % PF] = fetch(k + PF);
-      if constexpr (k < 32) {
-        constexpr int tt = k >> 4, ks = (k & 15) >> 1;
+      if constexpr (k + PF < SLOTS) ring[k % PF] = fetch(k + PF);
+      if constexpr (k < S1) {
+        constexpr int tt = k / (2 * KS), ks = k % (2 * KS) >> 1;
         if constexpr (k & 1)
           dp[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op, dof[ks], ks ? dp[tt] : f32x16{}, 0, 0, 0);
         else
           sc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op, qf[ks], ks ? sc[tt] : f32x16{}, 0, 0, 0);
       } else {
-        constexpr int j = k - 32;
-        acc[j & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op, db[j >> 3][(j >> 2) & 1], acc[j & 3], 0, 0, 0);
+        constexpr int j = k - S1, u = j % NU;
+        acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op, db[j / (2 * NU)][j / NU % 2], acc[u], 0, 0, 0);
       }
-      if constexpr (k >= 16 && k < 32) ds_elem(0, k - 16);
-      if constexpr (k >= 32 && k < 40) {
-        ds_elem(1, 2 * (k - 32));
-        ds_elem(1, 2 * (k - 32) + 1);
+      // dS^T of tile 0 beside the products of tile 1, of tile 1 beside dQ's of tile 0
+      if constexpr (k >= S1 / 2 && k < S1) {
+        constexpr int n = 16 / (2 * KS);
+#pragma unroll
+        for (int e = 0; e < n; ++e) ds_elem(0, n * (k - S1 / 2) + e);
+      }
+      if constexpr (k >= S1 && k < S1 + 2 * NU) {
+        constexpr int n = 16 / (2 * NU);
+#pragma unroll
+        for (int e = 0; e < n; ++e) ds_elem(1, n * (k - S1) + e);
       }
       __builtin_amdgcn_sched_barrier(0);
     });
@@ -464,13 +476,13 @@ __global__ __launch_bounds__(256, 1) void bsa_bwd_dq_bf16_d128(
   }
   for (int s = 0; s < nsteps; ++s) {
     const int64_t key0 = key_of(s, cb_c, cv_c);
-    // this wave's loads of half s are done once only the later halves (8
-    // loads each) are outstanding
+    // this wave's loads of half s are done once only the later halves
+    // (LOADS loads each) are outstanding
     const int ahead = nsteps - 1 - s < NST - 2 ? nsteps - 1 - s : NST - 2;
     if (ahead >= 2)
-      tsp::dma::wait_vm<16>();
+      tsp::dma::wait_vm<2 * LOADS>();
     else if (ahead == 1)
-      tsp::dma::wait_vm<8>();
+      tsp::dma::wait_vm<LOADS>();
     else
       tsp::dma::wait_vm<0>();
     tsp::dma::barrier();  // every wave's part is in LDS; stage (s - 1) % NST is free
@@ -509,13 +521,17 @@ __global__ __launch_bounds__(256, 1) void bsa_bwd_dq_bf16_d128(
 // a whole column writes bf16 dK / dV, a segment of a split column writes
 // fp32 partials that bsa_bwd_reduce sums in segment order.
 constexpr int RCAP = 64;  // item records staged per batch
-__global__ __launch_bounds__(256, 1) void bsa_bwd_dkdv_bf16_d128(
+template <int D>
+__global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bsa_bwd_dkdv_bf16(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
     const uint16_t* __restrict__ dO, int64_t S, int64_t H, int nh, const int64_t* __restrict__ crow,
     const int32_t* __restrict__ items, int n_items, int n_partials, float scale_log2, float scale,
     const float* __restrict__ qstat, uint16_t* __restrict__ dK, uint16_t* __restrict__ dV,
     float* __restrict__ partial) {
   using namespace abw;
+  constexpr int ROWB = Geo<D>::ROWB, HBYTES = Geo<D>::HBYTES, KS = Geo<D>::KS, NU = Geo<D>::NU;
+  constexpr int LOADS = Geo<D>::LOADS;  // per wave and stage (one more, the stats, in wave 0)
+  constexpr int S1 = 4 * KS, SLOTS = S1 + 8 * NU;  // slots of the S / dP products; all
   constexpr int STAGE = 2 * HBYTES + 1024;  // Q half, dO half, stats [4][64] floats (r, D, D, D)
   constexpr int NST = 3;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NST * STAGE];
@@ -534,21 +550,23 @@ __global__ __launch_bounds__(256, 1) void bsa_bwd_dkdv_bf16_d128(
   bf16x8 kn[KS], vn[KS];  // the next item's, loaded during the current item's last half
 
   const int loff = l32 * ROWB;
-  const int kx = swz(l32) ^ h;
-  const TrLane trl = tr_lane(lane);
+  const int kx = swz<D>(l32) ^ h;
+  const TrLane trl = tr_lane<D>(lane);
 
   auto compute = [&](uint32_t st) {
     const uint32_t rb = st + (uint32_t)(loff + (kx << 4));
     const uint32_t tb0 = st + (uint32_t)(trl.off[0] + (trl.xu << 6));
     const uint32_t tb1 = st + (uint32_t)(trl.off[1] + (trl.xu << 6));
     const uint32_t sb = st + 2 * HBYTES + 16 * h;
-    // slot -> LDS operand: 0-31 S / dP of tile k / 16 (even: Q row, odd: dO
-    // row, k-step (k % 16) / 2); 32-63 of tile (k - 32) / 16, k-step
-    // a = (k / 8) % 2, subtile u = (k / 2) % 4 (even: dO^T for dV, odd: Q^T for dK)
+    // slot -> LDS operand: k < S1 S / dP of tile k / (2 KS) (even: Q row, odd:
+    // dO row, k-step (k % (2 KS)) / 2); then, j = k - S1, of tile j / (4 NU),
+    // k-step a = (j / (2 NU)) % 2, subtile u = (j / 2) % NU (even: dO^T for dV,
+    // odd: Q^T for dK)
     auto fetch = [&](int k) -> bf16x8 {
-      if (k < 32) return lds_row(rb, (k & 15) >> 1, (k & 1) * HBYTES + 32 * (k >> 4) * ROWB);
-      const int j = k - 32;
-      return lds_trp(tb0, tb1, (j >> 1) & 3, ((j & 1) ? 0 : HBYTES) + (32 * (j >> 4) + 16 * ((j >> 3) & 1)) * ROWB);
+      if (k < S1) return lds_row(rb, k % (2 * KS) >> 1, (k & 1) * HBYTES + 32 * (k / (2 * KS)) * ROWB);
+      const int j = k - S1;
+      return lds_trp(tb0, tb1, (j >> 1) % NU,
+                     ((j & 1) ? 0 : HBYTES) + (32 * (j / (4 * NU)) + 16 * (j / (2 * NU) % 2)) * ROWB);
     };
     f32x16 sc[2], dp[2];
     u32x4 pw[2][2], dw[2][2];  // bf16 pairs of P and dS, k order of the B operand
@@ -583,25 +601,30 @@ __global__ __launch_bounds__(256, 1) void bsa_bwd_dkdv_bf16_d128(
       pw[qt][v >> 3][(v & 7) >> 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2));
       dw[qt][v >> 3][(v & 7) >> 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector(d, bf16x2));
     };
-    tsp::static_for<64>([&](auto kc) __attribute__((always_inline)) {
+    tsp::static_for<SLOTS>([&](auto kc) __attribute__((always_inline)) {
       constexpr int k = decltype(kc)::value;
       const bf16x8 op = ring[k % PF];
-      if constexpr (k + PF < 64) ring[k % PF] = fetch(k + PF);
-      if constexpr (k == 12) stats(0, 0);
-      if constexpr (k < 32) {
-        constexpr int qt = k >> 4, ks = (k & 15) >> 1;
+      if constexpr (k + PF < SLOTS) ring[k % PF] = fetch(k + PF);
+      if constexpr (k == S1 / 2 - 4) stats(0, 0);
+      if constexpr (k < S1) {
+        constexpr int qt = k / (2 * KS), ks = k % (2 * KS) >> 1;
         if constexpr (k & 1)
           dp[qt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op, vf[ks], ks ? dp[qt] : f32x16{}, 0, 0, 0);
         else
           sc[qt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op, kf[ks], ks ? sc[qt] : f32x16{}, 0, 0, 0);
       } else {
-        constexpr int j = k - 32, qt = j >> 4, a = (j >> 3) & 1, u = (j >> 1) & 3;
+        constexpr int j = k - S1, qt = j / (4 * NU), a = j / (2 * NU) % 2, u = (j >> 1) % NU;
         if constexpr (j & 1)
           dk[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op, __builtin_bit_cast(bf16x8, dw[qt][a]), dk[u], 0, 0, 0);
         else
           dv[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op, __builtin_bit_cast(bf16x8, pw[qt][a]), dv[u], 0, 0, 0);
       }
-      if constexpr (k >= 16 && k < 48 && (k & 1) == 0) ds_pair((k - 16) >> 4, (k - 16) & 15);
+      // P and dS, two elements at a time: tile 0 beside the products of tile 1,
+      // tile 1 beside dV's and dK's of tile 0
+      if constexpr (k >= S1 / 2 && k < S1 + 4 * NU) {
+        constexpr int e = (k - S1 / 2) * (16 / (2 * KS));
+        if constexpr (e % 2 == 0) ds_pair(e >> 4, e & 15);
+      }
       __builtin_amdgcn_sched_barrier(0);
     });
   };
@@ -657,8 +680,8 @@ __global__ __launch_bounds__(256, 1) void bsa_bwd_dkdv_bf16_d128(
       const int64_t q0 = (int64_t)__builtin_amdgcn_readfirstlane(rrow[pr][pt >> 1]) * BS + HR * (pt & 1);
       const int64_t hs = (int64_t)head * S * D;
       const uint32_t st = lds0 + (pc % NST) * STAGE;
-      dma_half(tsp::dma::make_rsrc(Q + hs, (uint32_t)(S * ROWB)), q0, st, w, lane);
-      dma_half(tsp::dma::make_rsrc(dO + hs, (uint32_t)(S * ROWB)), q0, st + HBYTES, w, lane);
+      dma_half<D>(tsp::dma::make_rsrc(Q + hs, (uint32_t)(S * ROWB)), q0, st, w, lane);
+      dma_half<D>(tsp::dma::make_rsrc(dO + hs, (uint32_t)(S * ROWB)), q0, st + HBYTES, w, lane);
       if (w == 0)
         tsp::dma::global16(qstat + ((lane >> 4) ? HS : 0) + (int64_t)head * S + 4 * (lane & 15) + q0,
                            st + 2 * HBYTES);
@@ -695,15 +718,15 @@ __global__ __launch_bounds__(256, 1) void bsa_bwd_dkdv_bf16_d128(
 #pragma unroll
       for (int u = 0; u < NU; ++u) dk[u] = dv[u] = f32x16{};
       for (int t = 0; t < nst; ++t) {
-        // loads of half cc are done once only the next half's (8 or 9
-        // loads) may be outstanding
+        // loads of half cc are done once only the next half's (LOADS, or
+        // one more) may be outstanding
         if (pc > cc + 1)
-          tsp::dma::wait_vm<8>();
+          tsp::dma::wait_vm<LOADS>();
         else
           tsp::dma::wait_vm<0>();
         tsp::dma::barrier();  // every wave's part is in LDS; stage (cc + 2) % 3 is free
         issue_next();
-        if (t == nst - 1) {  // the next item's K and V rows
+        if (D == 128 && t == nst - 1) {  // the next item's K and V rows (at d = 64 another workgroup fills the gap)
           int rn = r + 1;
           while (rn < R && __builtin_amdgcn_readfirstlane(rhdr[rn][2]) < 0) ++rn;
           if (rn < R) {
@@ -756,6 +779,7 @@ __global__ __launch_bounds__(256, 1) void bsa_bwd_dkdv_bf16_d128(
 // order (deterministic), rounded to bf16. Workgroup per (split, 16-key chunk
 // of the column, head); thread per 4 consecutive head_dim values of one key
 // of dK or dV.
+template <int D>
 __global__ __launch_bounds__(256) void bsa_bwd_reduce(const int32_t* __restrict__ splits, int n_partials, int64_t S,
                                                       const float* __restrict__ partial, uint16_t* __restrict__ dK,
                                                       uint16_t* __restrict__ dV) {
@@ -1189,6 +1213,53 @@ __global__ __launch_bounds__(256) void bsa_bwd_reduce_f32(const int32_t* __restr
   }
 }
 
+// The two passes and the reduce at head_dim D. At d = 64 two workgroups share
+// a CU (registers and LDS halve), so the column pass is two per CU.
+template <int D>
+int launch_bf16(const void* Q, const void* K, const void* V, const void* O, const void* dO, int64_t H, int64_t S,
+                const int64_t* rp, const int64_t* ci, const int64_t* crow, int64_t Mt, double scale,
+                const void* rmax, const void* rden, void* dQ, void* dK, void* dV, const int32_t* plan, int64_t n_items,
+                int64_t n_splits, int64_t n_partials, void* workspace, hipStream_t st) {
+  const int64_t nh = tsp::ceil_div(H, 8);
+  const int64_t grid_a = nh * Mt * 8;
+  if (grid_a > INT32_MAX || n_items * nh > INT32_MAX || 8 * n_splits > INT32_MAX || H > 65535)
+    return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsa_bwd: problem too large");
+  const float sl2 = (float)(scale * 1.4426950408889634);
+  float* qstat = (float*)workspace;
+  float* partial = (float*)((char*)workspace + 16 * H * S);
+  if (Mt * abw::BS < S) {  // rows without a block row: zero dQ
+    const int64_t tail = (S - Mt * abw::BS) * D * 2;
+    for (int64_t hh = 0; hh < H; ++hh) {
+      int rc = tsp::zero_fill((char*)dQ + (hh * S + Mt * abw::BS) * D * 2, tail, st);
+      if (rc) return rc;
+    }
+  }
+  if (grid_a > 0) {
+    hipLaunchKernelGGL((bsa_bwd_dq_bf16<D>), dim3((unsigned)grid_a), dim3(256), 0, st, (const uint16_t*)Q,
+                       (const uint16_t*)K, (const uint16_t*)V, (const uint16_t*)O, (const uint16_t*)dO, S, H, rp, ci,
+                       Mt, sl2, (float)scale, (const float*)rmax, (const float*)rden, qstat, (uint16_t*)dQ);
+    int rc = tsp::check_launch("bsa_bwd_dq_bf16 launch");
+    if (rc) return rc;
+  }
+  if (n_items > 0) {
+    const int64_t nslots = n_items * nh, most = D == 64 ? 64 : 32;  // workgroups per XCD
+    const int64_t g8 = nslots < most ? nslots : most;
+    hipLaunchKernelGGL((bsa_bwd_dkdv_bf16<D>), dim3((unsigned)(8 * g8)), dim3(256), 0, st, (const uint16_t*)Q,
+                       (const uint16_t*)K, (const uint16_t*)V, (const uint16_t*)dO, S, H, (int)nh, crow, plan + 4,
+                       (int)n_items, (int)n_partials, sl2, (float)scale, (const float*)qstat, (uint16_t*)dK,
+                       (uint16_t*)dV, partial);
+    int rc = tsp::check_launch("bsa_bwd_dkdv_bf16 launch");
+    if (rc) return rc;
+  }
+  if (n_splits > 0) {
+    hipLaunchKernelGGL((bsa_bwd_reduce<D>), dim3((unsigned)(8 * n_splits), (unsigned)H), dim3(256), 0, st,
+                       plan + 4 + 4 * n_items, (int)n_partials, S, (const float*)partial, (uint16_t*)dK, (uint16_t*)dV);
+    int rc = tsp::check_launch("bsa_bwd_reduce launch");
+    if (rc) return rc;
+  }
+  return TSP_OK;
+}
+
 template <int D>
 int launch_f32(const void* Q, const void* K, const void* V, const void* O, const void* dO, int64_t H, int64_t S,
                const int64_t* rp, const int64_t* ci, const int64_t* crow, int64_t Mt, double scale,
@@ -1325,7 +1396,7 @@ extern "C" int64_t tsp_bsa_bwd_plan(const int64_t* col_ptrs, int64_t n_block_col
 
 extern "C" int64_t tsp_bsa_bwd_workspace_size(int64_t n_heads, int64_t seq_len, int64_t head_dim, int64_t n_partials) {
   if (n_heads < 0 || seq_len < 0 || head_dim < 0 || n_partials < 0) return -1;
-  const int64_t pd = head_dim > abw::D ? head_dim : abw::D;  // fp32 partial rows of dK and dV
+  const int64_t pd = head_dim > 128 ? head_dim : 128;  // fp32 partial rows of dK and dV
   return 16 * n_heads * seq_len + n_heads * n_partials * 2 * abw::BS * pd * 4;
 }
 
@@ -1351,51 +1422,18 @@ extern "C" int tsp_bsa_bwd(const void* Q, const void* K, const void* V, const vo
   const bool aligned = ((uintptr_t)Q % 16) == 0 && ((uintptr_t)K % 16) == 0 && ((uintptr_t)V % 16) == 0 &&
                        ((uintptr_t)O % 16) == 0 && ((uintptr_t)dO % 16) == 0 && ((uintptr_t)dQ % 8) == 0 &&
                        ((uintptr_t)dK % 8) == 0 && ((uintptr_t)dV % 8) == 0 && ((uintptr_t)workspace % 16) == 0;
-  if (dtype == TSP_BF16 && block_size == abw::BS && head_dim == abw::D && scale > 0 && plan && aligned &&
-      (seq_len + abw::BS) * abw::ROWB <= (int64_t)UINT32_MAX) {
+  if (dtype == TSP_BF16 && block_size == abw::BS && (head_dim == 64 || head_dim == 128) && scale > 0 && plan && aligned &&
+      (seq_len + abw::BS) * head_dim * 2 <= (int64_t)UINT32_MAX) {
     if (n_items < tsp::ceil_div(seq_len, block_size))
       return tsp::fail(TSP_EINVAL, "tsp_bsa_bwd: plan has %lld items for %lld key block columns", (long long)n_items,
                        (long long)tsp::ceil_div(seq_len, block_size));
-    const int64_t nh = tsp::ceil_div(n_heads, 8);
-    const int64_t grid_a = nh * Mt * 8;
-    if (grid_a > INT32_MAX || n_items * nh > INT32_MAX || 8 * n_splits > INT32_MAX || n_heads > 65535)
-      return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsa_bwd: problem too large");
-    const float sl2 = (float)(scale * 1.4426950408889634);
-    float* qstat = (float*)workspace;
-    float* partial = (float*)((char*)workspace + 16 * rows);
-    if (Mt * block_size < seq_len) {  // rows without a block row: zero dQ
-      const int64_t tail = (seq_len - Mt * block_size) * head_dim * 2;
-      for (int64_t hh = 0; hh < n_heads; ++hh) {
-        int rc = tsp::zero_fill((char*)dQ + (hh * seq_len + Mt * block_size) * head_dim * 2, tail, stream_);
-        if (rc) return rc;
-      }
-    }
-    if (grid_a > 0) {
-      hipLaunchKernelGGL(bsa_bwd_dq_bf16_d128, dim3((unsigned)grid_a), dim3(256), 0, stream_, (const uint16_t*)Q,
-                         (const uint16_t*)K, (const uint16_t*)V, (const uint16_t*)O, (const uint16_t*)dO, seq_len,
-                         n_heads, block_row_ptrs, block_col_indices, Mt, sl2, (float)scale, (const float*)row_max,
-                         (const float*)row_denom, qstat, (uint16_t*)dQ);
-      int rc = tsp::check_launch("bsa_bwd_dq_bf16_d128 launch");
-      if (rc) return rc;
-    }
-    if (n_items > 0) {
-      const int64_t nslots = n_items * nh;
-      const int64_t g8 = nslots < 32 ? nslots : 32;
-      hipLaunchKernelGGL(bsa_bwd_dkdv_bf16_d128, dim3((unsigned)(8 * g8)), dim3(256), 0, stream_, (const uint16_t*)Q,
-                         (const uint16_t*)K, (const uint16_t*)V, (const uint16_t*)dO, seq_len, n_heads, (int)nh,
-                         col_block_rows, plan + 4, (int)n_items, (int)n_partials, sl2, (float)scale,
-                         (const float*)qstat, (uint16_t*)dK, (uint16_t*)dV, partial);
-      int rc = tsp::check_launch("bsa_bwd_dkdv_bf16_d128 launch");
-      if (rc) return rc;
-    }
-    if (n_splits > 0) {
-      hipLaunchKernelGGL(bsa_bwd_reduce, dim3((unsigned)(8 * n_splits), (unsigned)n_heads), dim3(256), 0, stream_,
-                         plan + 4 + 4 * n_items, (int)n_partials, seq_len, (const float*)partial, (uint16_t*)dK,
-                         (uint16_t*)dV);
-      int rc = tsp::check_launch("bsa_bwd_reduce launch");
-      if (rc) return rc;
-    }
-    return TSP_OK;
+    if (head_dim == 64)
+      return launch_bf16<64>(Q, K, V, O, dO, n_heads, seq_len, block_row_ptrs, block_col_indices, col_block_rows, Mt,
+                             scale, row_max, row_denom, dQ, dK, dV, plan, n_items, n_splits, n_partials, workspace,
+                             stream_);
+    return launch_bf16<128>(Q, K, V, O, dO, n_heads, seq_len, block_row_ptrs, block_col_indices, col_block_rows, Mt,
+                            scale, row_max, row_denom, dQ, dK, dV, plan, n_items, n_splits, n_partials, workspace,
+                            stream_);
   }
 
   const bool aligned16 = aligned && ((uintptr_t)dQ % 16) == 0 && ((uintptr_t)dK % 16) == 0 && ((uintptr_t)dV % 16) == 0;
