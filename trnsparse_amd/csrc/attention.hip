@@ -39,6 +39,7 @@
 //       the accumulation type (double for fp64).
 #include "common.h"
 #include "lds_dma.h"
+#include "tile_item.h"
 
 namespace {
 
@@ -126,13 +127,10 @@ __global__ __launch_bounds__(256, 2) void bsa_fwd_bf16_mfma(
   __shared__ __attribute__((aligned(16))) uint16_t Ks[AB * K_LD];
   __shared__ __attribute__((aligned(16))) uint16_t Vt[D * V_LD];
 
-  // XCD-aware order: XCD x walks heads x, x+8, ...; the block rows of one
-  // head run side by side and share that head's K/V in the XCD's L2.
-  const int64_t g = blockIdx.x;
-  const int64_t xcd = g & 7, slot = g >> 3;
-  const int64_t head = xcd + 8 * (slot / Mt);
-  const int64_t m = slot % Mt;
-  if (head >= H) return;
+  // XCD-aware order: the block rows of one head run side by side and share
+  // that head's K/V in the XCD's L2.
+  int64_t head, m;
+  if (!tsp::head_item(blockIdx.x, Mt, H, head, m)) return;
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int h = lane >> 5, l32 = lane & 31;
@@ -362,13 +360,10 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void bsa_fwd_bf16_stream(
   constexpr int HK = G::HK, NT = G::NT, SPB = G::SPB;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NST * STAGE];
 
-  // XCD-aware order: XCD x walks heads x, x+8, ...; the block rows of one
-  // head run side by side and share that head's K/V in the XCD's L2.
-  const int64_t g = blockIdx.x;
-  const int64_t xcd = g & 7, slot = g >> 3;
-  const int64_t head = xcd + 8 * (slot / Mt);
-  const int64_t m = slot % Mt;
-  if (head >= H) return;
+  // XCD-aware order: the block rows of one head run side by side and share
+  // that head's K/V in the XCD's L2.
+  int64_t head, m;
+  if (!tsp::head_item(blockIdx.x, Mt, H, head, m)) return;
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int h = lane >> 5, l32 = lane & 31;
@@ -614,11 +609,8 @@ __global__ __launch_bounds__(512, 1) void bsa_fwd_bf16_d512(
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NST * STAGE + XBYTES];
   float* xch = (float*)(lds + NST * STAGE);
 
-  const int64_t g = blockIdx.x;
-  const int64_t xcd = g & 7, slot = g >> 3;
-  const int64_t head = xcd + 8 * (slot / Mt);
-  const int64_t m = slot % Mt;
-  if (head >= H) return;
+  int64_t head, m;
+  if (!tsp::head_item(blockIdx.x, Mt, H, head, m)) return;
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wq = w & 3, dh = w >> 2;  // query group, head-dim half
@@ -853,13 +845,10 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void bsa_fwd_f32_mfma(
   typedef typename attf::VRow<NUH>::type vrow_t;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NST * STAGE];
 
-  // XCD-aware order: XCD x walks heads x, x+8, ...; the block rows of one
-  // head run side by side and share that head's K/V in the XCD's L2.
-  const int64_t g = blockIdx.x;
-  const int64_t xcd = g & 7, slot = g >> 3;
-  const int64_t head = xcd + 8 * (slot / Mt);
-  const int64_t m = slot % Mt;
-  if (head >= H) return;
+  // XCD-aware order: the block rows of one head run side by side and share
+  // that head's K/V in the XCD's L2.
+  int64_t head, m;
+  if (!tsp::head_item(blockIdx.x, Mt, H, head, m)) return;
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int h = lane >> 5, l32 = lane & 31;
@@ -1087,7 +1076,7 @@ extern "C" int tsp_bsa_fwd(const void* Q, const void* K, const void* V, int dtyp
       (head_dim == 64 || head_dim == 128 || ((head_dim == 256 || head_dim == 512) && bf16_streamed)) &&
       ((uintptr_t)Q % 16) == 0 &&
       ((uintptr_t)K % 16) == 0 && ((uintptr_t)V % 16) == 0 && ((uintptr_t)O % 8) == 0) {
-    const int64_t grid = tsp::ceil_div(n_heads, 8) * Mt * 8;
+    const int64_t grid = tsp::head_grid(Mt, n_heads);
     if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsa_fwd: problem too large");
     const float sl2 = (float)(scale * 1.4426950408889634);
 #define TSP_FWD_BF16(KERNEL)                                                                                        \
@@ -1114,7 +1103,7 @@ extern "C" int tsp_bsa_fwd(const void* Q, const void* K, const void* V, int dtyp
   if (dtype == TSP_F32 && block_size == AB && (head_dim == 64 || head_dim == 128 || head_dim == 256) && scale > 0 &&
       ((uintptr_t)Q % 16) == 0 && ((uintptr_t)K % 16) == 0 && ((uintptr_t)V % 16) == 0 && ((uintptr_t)O % 16) == 0 &&
       (seq_len + AB) * head_dim * 4 <= (int64_t)UINT32_MAX) {
-    const int64_t grid = tsp::ceil_div(n_heads, 8) * Mt * 8;
+    const int64_t grid = tsp::head_grid(Mt, n_heads);
     if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsa_fwd: problem too large");
     const float sl2 = (float)(scale * 1.4426950408889634);
 #define TSP_FWD_F32(KERNEL)                                                                                       \

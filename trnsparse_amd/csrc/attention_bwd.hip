@@ -50,6 +50,8 @@
 #include "common.h"
 
 #include "lds_dma.h"
+#include "tile_item.h"
+#include "attention_tiles.h"
 #include "slots.h"
 
 namespace tsp {
@@ -65,6 +67,8 @@ int bsa_bwd_f32_d256_cols(const float* Q, const float* K, const float* V, const 
 
 namespace {
 
+namespace abw = tsp::abw;
+namespace abf = tsp::abf;
 constexpr float LOG2E = 1.4426950408889634f;
 
 template <typename T> struct AAcc { typedef float type; };
@@ -209,95 +213,6 @@ int launch_generic(const void* Q, const void* K, const void* V, const void* dO, 
 
 // --------------------------------------------- bf16 MFMA, d = 64 and 128
 
-namespace abw {
-constexpr int BS = 128;             // block size served by the MFMA kernels
-constexpr int HR = 64;              // rows (keys in the row pass, queries in the column pass) per ring stage
-constexpr int SEG_MAX = 64;         // most block rows one column-pass item walks
-template <int D>
-struct Geo {
-  static constexpr int ROWB = D * 2;                // bytes per row
-  static constexpr int HBYTES = HR * ROWB;          // a half: 64 rows
-  static constexpr int KS = D / 16;                 // k-steps over head_dim
-  static constexpr int NU = D / 32;                 // 32-wide head_dim subtiles
-  static constexpr int LOADS = 2 * HBYTES / 4096;   // 1-KiB loads per wave of two operands' halves
-};
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-typedef float f32x8 __attribute__((ext_vector_type(8)));
-typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
-
-// The 16-byte chunk c of stage row r sits in slot c ^ swz(r). Rows are read
-// as 16-byte pieces of 16 consecutive rows (one chunk) and through transpose
-// reads of 4 consecutive rows (4 chunks). At d = 128 (256-byte rows, 16
-// chunks) swz is a bijection on r % 16 whose low two bits follow r / 4 and
-// high two bits r % 4; at d = 64 two rows share the 64 banks and the 8 chunks
-// of a row follow r / 2: its parity in the high bit, r / 4 in the low two. So
-// both access forms hit 16 (resp. 4 x 4) distinct slots.
-template <int D>
-__host__ __device__ constexpr int swz(int r) {
-  return D == 128 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
-}
-
-// One wave's share (rows [16w, 16w + 16)) of a 64-row half starting at global
-// row row0 of the buffer `rs`, into the stage at LDS address dst.
-template <int D>
-__device__ inline void dma_half(tsp::dma::i32x4 rs, int64_t row0, uint32_t dst, int w, int lane) {
-  constexpr int ROWB = Geo<D>::ROWB, CPR = ROWB / 16, RPI = 64 / CPR;  // chunks per row, rows per instruction
-#pragma unroll
-  for (int qq = 0; qq < Geo<D>::LOADS / 2; ++qq) {
-    const int j = Geo<D>::LOADS / 2 * w + qq;
-    const int rr = RPI * j + lane / CPR;
-    const int p = lane % CPR;
-    tsp::dma::buffer16(rs, (uint32_t)((row0 + rr) * ROWB + ((p ^ swz<D>(rr)) << 4)), dst + j * 1024);
-  }
-}
-
-// A operand holding the transpose: rows (MFMA i) are head_dim 32u + l32 and
-// the 8 k values are stage rows r0 + 4h + {0..3} and r0 + 8 + 4h + {0..3}
-// (the k order of the lane's own accumulator rows), from two
-// ds_read_b64_tr_b16: lane j of 16-lane group gq points at row
-// r0 + 8 rr + 4 (gq / 2) + j / 4, column 32u + 16 (gq % 2) + 4 (j % 4).
-struct TrLane {
-  int off[2];
-  int xu;
-};
-template <int D>
-__device__ inline TrLane tr_lane(int lane) {
-  const int gq = lane >> 4, jq = lane & 15;
-  const int c0 = 2 * (gq & 1) + ((jq & 3) >> 1);
-  TrLane t;
-#pragma unroll
-  for (int rr = 0; rr < 2; ++rr) {
-    const int row = 8 * rr + 4 * (gq >> 1) + (jq >> 2);
-    t.off[rr] = row * Geo<D>::ROWB + ((c0 ^ (swz<D>(row) & 3)) << 4) + 8 * (jq & 1);
-  }
-  t.xu = D == 128 ? jq >> 2 : jq >> 3;  // swz(row) >> 2
-  return t;
-}
-// Address form of the two reads for the slot kernels. A stage starts at an
-// LDS address that is a multiple of 256 and rows are 256 (d = 64: 128) bytes,
-// so the swizzled chunk bits (4-7, 4-6) of a lane's address are free in the stage base:
-// per step one base per access kind is formed (row reads: stage + l32 * ROWB
-// + swz(l32)^h in bits 4-7; transpose reads: stage + off[rr] + xu in bits
-// 6-7) and each read is base ^ (k-step or subtile bits) plus a constant row
-// offset that the ds_read immediate absorbs.
-// Round 4 floats to bf16 (round to nearest even, v_cvt_pk_bf16_f32) as 4 halfwords.
-__device__ inline u16x4 bf16x4_rne(f32x4 v) {
-  return __builtin_bit_cast(u16x4, __builtin_convertvector(v, bf16x4));
-}
-
-
-typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
-__device__ inline bf16x8 lds_row(uint32_t rb, int ks, uint32_t off) {
-  return *(const lds_bf16x8*)(uintptr_t)((rb ^ (uint32_t)(ks << 5)) + off);
-}
-__device__ inline bf16x8 lds_trp(uint32_t tb0, uint32_t tb1, int u, uint32_t off) {
-  const s16x4 r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)((tb0 ^ (uint32_t)(u << 6)) + off));
-  const s16x4 r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)((tb1 ^ (uint32_t)(u << 6)) + off));
-  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(r0, r1, 0, 1, 2, 3, 4, 5, 6, 7));
-}
-}  // namespace abw
-
 // Both passes run one wavefront per SIMD (a 256-thread workgroup per CU)
 // and issue their work in a fixed slot order: slot k is one MFMA whose LDS
 // operand was read PF slots earlier (a register ring, so LDS latency hides
@@ -309,8 +224,7 @@ constexpr int PF = 4;  // operand reads in flight
 
 
 // Row pass: workgroup per (head, query block row m < Mt), XCD-aware order as
-// the forward (XCD x walks heads x, x + 8, ...; block rows of one head side by
-// side share its K/V in L2). Wavefront w owns queries m * 128 + 32 w + [0, 32)
+// the forward. Wavefront w owns queries m * 128 + 32 w + [0, 32)
 // with their Q and dO rows in registers; 64-key halves of K and V stream
 // through a 4-stage LDS ring by direct buffer loads issued three halves ahead.
 // Per half (slots at d = 128), 0-31: S^T and dP^T tiles of the two 32-key
@@ -334,11 +248,8 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bsa_bwd_dq_bf16(
   constexpr int NST = 4;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NST * STAGE];
 
-  const int64_t g = blockIdx.x;
-  const int64_t xcd = g & 7, slot = g >> 3;
-  const int64_t head = xcd + 8 * (slot / Mt);
-  const int64_t m = slot % Mt;
-  if (head >= H) return;
+  int64_t head, m;
+  if (!tsp::head_item(blockIdx.x, Mt, H, head, m)) return;
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int h = lane >> 5, l32 = lane & 31;
@@ -504,7 +415,8 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bsa_bwd_dq_bf16(
 
 // Column pass, persistent: 8 * G8 workgroups (G8 <= 32 per XCD, one per
 // CU); workgroup j of XCD x takes the slots j, j + G8, j + 2 G8, ... of its
-// XCD's slot list, slot s = (item s / nh, head x + 8 (s % nh)); an item is
+// XCD's slot list, slot s being pair 8 s + x of the (item, head) pairs, heads
+// fastest (so with a multiple of 8 heads an XCD keeps to its own); an item is
 // (block column, range [p0, p1) of its column view, partial slot or -1) and
 // items are sorted heaviest first, so the round robin spreads the work. The
 // item records and their block rows (gathered from the column view) are
@@ -524,7 +436,7 @@ constexpr int RCAP = 64;  // item records staged per batch
 template <int D>
 __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bsa_bwd_dkdv_bf16(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
-    const uint16_t* __restrict__ dO, int64_t S, int64_t H, int nh, const int64_t* __restrict__ crow,
+    const uint16_t* __restrict__ dO, int64_t S, int64_t H, const int64_t* __restrict__ crow,
     const int32_t* __restrict__ items, int n_items, int n_partials, float scale_log2, float scale,
     const float* __restrict__ qstat, uint16_t* __restrict__ dK, uint16_t* __restrict__ dV,
     float* __restrict__ partial) {
@@ -539,7 +451,8 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bsa_bwd_dkdv_bf16(
   __shared__ int32_t rrow[RCAP][SEG_MAX];  // block rows of the item
 
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3, G8 = gridDim.x >> 3;
-  const int64_t nslots = (int64_t)n_items * nh;
+  const uint32_t heads = (uint32_t)H, total = (uint32_t)n_items * heads;  // within int32 (checked by the host)
+  const int64_t nslots = (total + 7) / 8;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int h = lane >> 5, l32 = lane & 31;
   const int64_t HS = H * S;
@@ -647,16 +560,16 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bsa_bwd_dkdv_bf16(
     __syncthreads();  // the previous batch's records and ring are no longer read
     if (tid < R) {
       const int64_t sl = j + (r0 + tid) * G8;
-      const int64_t it = sl / nh, head = xcd + 8 * (sl % nh);
+      const uint32_t idx = 8 * (uint32_t)sl + xcd, it = idx < total ? idx / heads : 0;
       rhdr[tid][0] = items[4 * it];
       rhdr[tid][1] = items[4 * it + 3];
-      rhdr[tid][2] = head < H ? items[4 * it + 2] - items[4 * it + 1] : -1;
-      rhdr[tid][3] = (int32_t)head;
+      rhdr[tid][2] = idx < total ? items[4 * it + 2] - items[4 * it + 1] : -1;
+      rhdr[tid][3] = (int32_t)(idx % heads);
     }
     for (int e = tid; e < R * SEG_MAX; e += 256) {
       const int r = e / SEG_MAX, i = e % SEG_MAX;
       const int64_t sl = j + (r0 + r) * G8;
-      const int64_t it = sl / nh;
+      const uint32_t idx = 8 * (uint32_t)sl + xcd, it = idx < total ? idx / heads : 0;
       const int p0 = items[4 * it + 1], n = items[4 * it + 2] - p0;
       if (i < n) rrow[r][i] = (int32_t)crow[p0 + i];
     }
@@ -696,7 +609,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bsa_bwd_dkdv_bf16(
     bool have_next = false;
     for (int r = 0; r < R; ++r) {
       const int nst = nsteps_of(r);
-      if (__builtin_amdgcn_readfirstlane(rhdr[r][2]) < 0) continue;  // head past H
+      if (__builtin_amdgcn_readfirstlane(rhdr[r][2]) < 0) continue;  // past the last pair
       const int col = __builtin_amdgcn_readfirstlane(rhdr[r][0]);
       const int pslot = __builtin_amdgcn_readfirstlane(rhdr[r][1]);
       const int head = __builtin_amdgcn_readfirstlane(rhdr[r][3]);
@@ -820,69 +733,6 @@ __global__ __launch_bounds__(256) void bsa_bwd_reduce(const int32_t* __restrict_
 // Stage rows are stored 16-byte chunk ^ (row % 16): chunk reads of one chunk
 // from 32 rows hit distinct banks, and a row read is a permutation of one
 // row.
-namespace abf {
-template <int D>
-struct Cfg {
-  static constexpr int BS = 128;
-  static constexpr int HR = 4096 / D;       // rows per ring stage
-  static constexpr int ROWB = D * 4;        // bytes per row
-  static constexpr int HBYTES = HR * ROWB;  // 16 KiB
-  static constexpr int NT = HR / 32;        // 32-row tiles per stage
-  static constexpr int NU = D / 32;         // head_dim subtiles of row products
-  static constexpr int KT = D / 8;          // b128 chunk reads per 32-row tile
-  static constexpr int SPB = BS / HR;       // stages per block
-};
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-template <int NU> struct VRow;
-template <> struct VRow<4> { typedef f32x4 type; };
-template <> struct VRow<2> { typedef f32x2 type; };
-
-// One wave's share of a stage: rows [row0, row0 + HR) of the buffer rs into
-// LDS dst, 16 instructions of 1 KiB, 4 per wave.
-template <int D>
-__device__ inline void dma_rows(tsp::dma::i32x4 rs, int64_t row0, uint32_t dst, int w, int lane) {
-  constexpr int LPR = D / 4, RPI = 64 / LPR, ROWB = D * 4;
-#pragma unroll
-  for (int qq = 0; qq < 4; ++qq) {
-    const int j = 4 * w + qq;
-    const int rr = RPI * j + lane / LPR;
-    const int p = lane % LPR;
-    tsp::dma::buffer16(rs, (uint32_t)((row0 + rr) * ROWB + ((p ^ (rr & 15)) << 4)), dst + j * 1024);
-  }
-}
-// chunk read: logical chunk c of stage row `row` (row % 16 == kx)
-template <int D>
-__device__ inline f32x4 chunk_read(const uint8_t* base, int row, int c, int kx) {
-  return *(const f32x4*)(base + row * (D * 4) + ((c ^ kx) << 4));
-}
-// row read: floats [NU * l32, NU * l32 + NU) of stage row `row`
-template <int D>
-__device__ inline typename VRow<D / 32>::type row_read(const uint8_t* base, int row, int l32) {
-  constexpr int NU = D / 32;
-  const int byte = NU * 4 * l32;
-  return *(const typename VRow<NU>::type*)(base + row * (D * 4) + ((((byte >> 4) ^ (row & 15))) << 4) + (byte & 15));
-}
-// Store a 32-row x D tile held as NU accumulators (element v of subtile u is
-// head_dim NU * (8 (v / 4) + 4 h + v % 4) + u of the lane's row) to dst, times f.
-template <int D>
-__device__ inline void store_rows(float* dst, const f32x16* acc, int h, float f) {
-  constexpr int NU = D / 32;
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    float* d = dst + NU * (8 * a + 4 * h);
-#pragma unroll
-    for (int k = 0; k < NU; ++k) {
-      f32x4 t;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int idx = 4 * k + e;
-        t[e] = acc[idx % NU][4 * a + idx / NU] * f;
-      }
-      *(f32x4*)(d + 4 * k) = t;
-    }
-  }
-}
-}  // namespace abf
 
 // Row pass: workgroup per (head, query block row m < Mt), XCD-aware order as
 // the forward; wavefront w owns queries m * 128 + 32 w + [0, 32) with their Q
@@ -902,11 +752,8 @@ __global__ __launch_bounds__(256, 1) void bsa_bwd_dq_f32(
   typedef typename abf::VRow<NU>::type vrow_t;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NST * STAGE];
 
-  const int64_t g = blockIdx.x;
-  const int64_t xcd = g & 7, slot = g >> 3;
-  const int64_t head = xcd + 8 * (slot / Mt);
-  const int64_t m = slot % Mt;
-  if (head >= H) return;
+  int64_t head, m;
+  if (!tsp::head_item(blockIdx.x, Mt, H, head, m)) return;
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int h = lane >> 5, l32 = lane & 31;
@@ -1220,9 +1067,8 @@ int launch_bf16(const void* Q, const void* K, const void* V, const void* O, cons
                 const int64_t* rp, const int64_t* ci, const int64_t* crow, int64_t Mt, double scale,
                 const void* rmax, const void* rden, void* dQ, void* dK, void* dV, const int32_t* plan, int64_t n_items,
                 int64_t n_splits, int64_t n_partials, void* workspace, hipStream_t st) {
-  const int64_t nh = tsp::ceil_div(H, 8);
-  const int64_t grid_a = nh * Mt * 8;
-  if (grid_a > INT32_MAX || n_items * nh > INT32_MAX || 8 * n_splits > INT32_MAX || H > 65535)
+  const int64_t grid_a = tsp::head_grid(Mt, H);
+  if (grid_a > INT32_MAX || n_items * H > INT32_MAX || 8 * n_splits > INT32_MAX || H > 65535)
     return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsa_bwd: problem too large");
   const float sl2 = (float)(scale * 1.4426950408889634);
   float* qstat = (float*)workspace;
@@ -1242,12 +1088,11 @@ int launch_bf16(const void* Q, const void* K, const void* V, const void* O, cons
     if (rc) return rc;
   }
   if (n_items > 0) {
-    const int64_t nslots = n_items * nh, most = D == 64 ? 64 : 32;  // workgroups per XCD
+    const int64_t nslots = tsp::ceil_div(n_items * H, 8), most = D == 64 ? 64 : 32;  // workgroups per XCD
     const int64_t g8 = nslots < most ? nslots : most;
     hipLaunchKernelGGL((bsa_bwd_dkdv_bf16<D>), dim3((unsigned)(8 * g8)), dim3(256), 0, st, (const uint16_t*)Q,
-                       (const uint16_t*)K, (const uint16_t*)V, (const uint16_t*)dO, S, H, (int)nh, crow, plan + 4,
-                       (int)n_items, (int)n_partials, sl2, (float)scale, (const float*)qstat, (uint16_t*)dK,
-                       (uint16_t*)dV, partial);
+                       (const uint16_t*)K, (const uint16_t*)V, (const uint16_t*)dO, S, H, crow, plan + 4, (int)n_items,
+                       (int)n_partials, sl2, (float)scale, (const float*)qstat, (uint16_t*)dK, (uint16_t*)dV, partial);
     int rc = tsp::check_launch("bsa_bwd_dkdv_bf16 launch");
     if (rc) return rc;
   }
@@ -1265,8 +1110,7 @@ int launch_f32(const void* Q, const void* K, const void* V, const void* O, const
                const int64_t* rp, const int64_t* ci, const int64_t* crow, int64_t Mt, double scale,
                const void* rmax, const void* rden, void* dQ, void* dK, void* dV, const int32_t* plan, int64_t n_items,
                int64_t n_splits, int64_t n_partials, void* workspace, hipStream_t st) {
-  const int64_t nh = tsp::ceil_div(H, 8);
-  const int64_t grid_a = nh * Mt * 8 * (D == 256 ? 2 : 1), grid_b = n_items * H * (D == 256 ? 2 : 1);
+  const int64_t grid_a = tsp::head_grid(Mt * (D == 256 ? 2 : 1), H), grid_b = n_items * H * (D == 256 ? 2 : 1);
   if (grid_a > INT32_MAX || grid_b > INT32_MAX || 8 * n_splits > INT32_MAX || H > 65535)
     return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsa_bwd: problem too large");
   const float sl2 = (float)(scale * 1.4426950408889634);

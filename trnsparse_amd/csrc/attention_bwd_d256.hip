@@ -30,6 +30,7 @@
 // dV) accumulator registers per lane live in AGPRs.
 #include "common.h"
 #include "lds_dma.h"
+#include "tile_item.h"
 
 namespace {
 
@@ -97,12 +98,9 @@ __global__ __launch_bounds__(256, 1) void bsa_bwd_dq_f32_d256(
   constexpr int STAGE = 2 * HBYTES;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NST * STAGE];
 
-  const int64_t gid = blockIdx.x;
-  const int64_t xcd = gid & 7, slot = gid >> 3;
-  const int64_t head = xcd + 8 * (slot / (2 * Mt));
-  const int64_t rem = slot % (2 * Mt);
+  int64_t head, rem;
+  if (!tsp::head_item(blockIdx.x, 2 * Mt, H, head, rem)) return;
   const int64_t m = rem >> 1, half = rem & 1;
-  if (head >= H) return;
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 4, l16 = lane & 15;
@@ -388,7 +386,7 @@ namespace tsp {
 int bsa_bwd_f32_d256_rows(const float* Q, const float* K, const float* V, const float* O, const float* dO, int64_t S,
                         int64_t H, const int64_t* rp, const int64_t* ci, int64_t Mt, float scale_log2, float scale,
                         const float* rmax, const float* rden, float* qstat, float* dQ, hipStream_t st) {
-  const int64_t grid = tsp::ceil_div(H, 8) * Mt * 2 * 8;
+  const int64_t grid = tsp::head_grid(2 * Mt, H);
   if (grid == 0) return TSP_OK;
   if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsa_bwd: problem too large");
   hipLaunchKernelGGL(bsa_bwd_dq_f32_d256, dim3((unsigned)grid), dim3(256), 0, st, Q, K, V, O, dO, S, H, rp, ci, Mt,
