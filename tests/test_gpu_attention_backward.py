@@ -176,6 +176,37 @@ def test_backward_f32_long_row(hip_backend):
                 sel_q=sel_q, sel_k=sel_k)
 
 
+@pytest.mark.parametrize("H", [1, 9, 130])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_small_and_full_grids(hip_backend, dtype, D, H):
+    """Forward and backward at 4, 36 and 520 (head, block row) pairs: 32
+    queries / keys to a workgroup up to one round of the chip, 128 beyond it
+    (head counts around the 8 chiplets the pairs are dealt to). An empty block
+    row, a never-stored block column, a full row and column (split between
+    work items), rows past the last whole block and a key block past the
+    sequence."""
+    S = 600
+    mask = local_mask(5, 1)
+    mask[0, :] = True
+    mask[:, 0] = True
+    mask[2, :] = False
+    mask[:, 3] = False
+    mask_bsr = W.bsr_from_block_mask(mask, 128)
+    g = torch.Generator().manual_seed(21)
+    Q, K, V, dO = (torch.randn(H, S, D, generator=g).to(dtype) for _ in range(4))
+    O, dQ, dK, dV = _run(Q, K, V, dO, mask_bsr)
+    assert torch.count_nonzero(O[:, 256:384]).item() == 0 and torch.count_nonzero(dQ[:, 256:384]).item() == 0
+    assert torch.count_nonzero(dQ[:, 512:]).item() == 0
+    assert torch.count_nonzero(dK[:, 384:512]).item() == 0 and torch.count_nonzero(dV[:, 384:512]).item() == 0
+    for hh in sorted({0, H // 2, H - 1}):
+        fwd = (mask_bsr.block_row_ptrs.numpy(), mask_bsr.block_col_indices.numpy(), 128, D**-0.5)
+        exact = ref.block_sparse_attention(_np(Q[hh]), _np(K[hh]), _np(V[hh]), *fwd)[0]
+        bound = ref.block_sparse_attention(_np(Q[hh]), _np(K[hh]), np.abs(_np(V[hh])), *fwd)[0]
+        assert ref.scaled_error(_np(O[hh]), exact, np.maximum(bound, 1e-30)) <= TOL[dtype]
+        _check_head(Q[hh], K[hh], V[hh], dO[hh], O[hh], (dQ[hh], dK[hh], dV[hh]), mask_bsr, D**-0.5, TOL[dtype])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_backward_deterministic(hip_backend, dtype):
     torch.manual_seed(13)

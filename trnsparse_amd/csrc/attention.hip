@@ -1079,6 +1079,9 @@ extern "C" int tsp_bsa_fwd(const void* Q, const void* K, const void* V, int dtyp
     const int64_t grid = tsp::head_grid(Mt, n_heads);
     if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsa_fwd: problem too large");
     const float sl2 = (float)(scale * 1.4426950408889634);
+    if (bf16_streamed && tsp::attn_split_fwd_pays(dtype, head_dim, n_heads, Mt))
+      return tsp::launch_attn_split_fwd(dtype, head_dim, Q, K, V, n_heads, seq_len, block_row_ptrs, block_col_indices,
+                                        Mt, scale, O, row_max, row_denom, st);
 #define TSP_FWD_BF16(KERNEL)                                                                                        \
   hipLaunchKernelGGL((KERNEL), dim3((unsigned)grid), dim3(256), 0, st, (const uint16_t*)Q, (const uint16_t*)K,       \
                      (const uint16_t*)V, seq_len, seq_len * head_dim, n_heads, block_row_ptrs, block_col_indices, Mt, \
@@ -1106,6 +1109,9 @@ extern "C" int tsp_bsa_fwd(const void* Q, const void* K, const void* V, int dtyp
     const int64_t grid = tsp::head_grid(Mt, n_heads);
     if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsa_fwd: problem too large");
     const float sl2 = (float)(scale * 1.4426950408889634);
+    if (tsp::attn_split_fwd_pays(dtype, head_dim, n_heads, Mt))
+      return tsp::launch_attn_split_fwd(dtype, head_dim, Q, K, V, n_heads, seq_len, block_row_ptrs, block_col_indices,
+                                        Mt, scale, O, row_max, row_denom, st);
 #define TSP_FWD_F32(KERNEL)                                                                                       \
   hipLaunchKernelGGL((KERNEL), dim3((unsigned)grid), dim3(256), 0, st, (const float*)Q, (const float*)K,           \
                      (const float*)V, seq_len, seq_len * head_dim, n_heads, block_row_ptrs, block_col_indices, Mt, \

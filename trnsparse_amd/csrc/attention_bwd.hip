@@ -32,8 +32,10 @@
 //       the items of a persistent workgroup.
 //   bsa_bwd_dq_f32<D> / bsa_bwd_dkdv_f32<D> / bsa_bwd_reduce_f32<D>  fp32,
 //       b = 128, D in {64, 128}: the same passes on v_mfma_f32_32x32x2_f32
-//       (operand forms at the kernels); D = 256 runs the row and column
-//       passes of attention_bwd_d256.hip (16-row tiles) and the reduce here.
+//       (operand forms at the kernels; the column pass at D = 64 is
+//       attention_split.hip's); D = 256 runs the row and column passes of
+//       attention_bwd_d256.hip (16-row tiles) and the reduce here. On small
+//       grids both passes of either type are attention_split.hip's.
 //   bsa_bwd_dq_generic / bsa_bwd_dkdv_generic  any dtype / block size /
 //       head_dim: one thread per (row, 32-wide slice of head_dim).
 // Swizzle: K (row pass) and Q, dO (column pass) are read both as 16-byte rows
@@ -1081,19 +1083,31 @@ int launch_bf16(const void* Q, const void* K, const void* V, const void* O, cons
     }
   }
   if (grid_a > 0) {
-    hipLaunchKernelGGL((bsa_bwd_dq_bf16<D>), dim3((unsigned)grid_a), dim3(256), 0, st, (const uint16_t*)Q,
-                       (const uint16_t*)K, (const uint16_t*)V, (const uint16_t*)O, (const uint16_t*)dO, S, H, rp, ci,
-                       Mt, sl2, (float)scale, (const float*)rmax, (const float*)rden, qstat, (uint16_t*)dQ);
-    int rc = tsp::check_launch("bsa_bwd_dq_bf16 launch");
+    int rc;
+    if (tsp::attn_split_dq_pays(TSP_BF16, D, H, Mt)) {
+      rc = tsp::launch_attn_split_dq(TSP_BF16, D, Q, K, V, O, dO, H, S, rp, ci, Mt, scale, rmax, rden, qstat, dQ, st);
+    } else {
+      hipLaunchKernelGGL((bsa_bwd_dq_bf16<D>), dim3((unsigned)grid_a), dim3(256), 0, st, (const uint16_t*)Q,
+                         (const uint16_t*)K, (const uint16_t*)V, (const uint16_t*)O, (const uint16_t*)dO, S, H, rp, ci,
+                         Mt, sl2, (float)scale, (const float*)rmax, (const float*)rden, qstat, (uint16_t*)dQ);
+      rc = tsp::check_launch("bsa_bwd_dq_bf16 launch");
+    }
     if (rc) return rc;
   }
   if (n_items > 0) {
-    const int64_t nslots = tsp::ceil_div(n_items * H, 8), most = D == 64 ? 64 : 32;  // workgroups per XCD
-    const int64_t g8 = nslots < most ? nslots : most;
-    hipLaunchKernelGGL((bsa_bwd_dkdv_bf16<D>), dim3((unsigned)(8 * g8)), dim3(256), 0, st, (const uint16_t*)Q,
-                       (const uint16_t*)K, (const uint16_t*)V, (const uint16_t*)dO, S, H, crow, plan + 4, (int)n_items,
-                       (int)n_partials, sl2, (float)scale, (const float*)qstat, (uint16_t*)dK, (uint16_t*)dV, partial);
-    int rc = tsp::check_launch("bsa_bwd_dkdv_bf16 launch");
+    int rc;
+    if (tsp::attn_split_dkdv_pays(TSP_BF16, D, H, n_items)) {
+      rc = tsp::launch_attn_split_dkdv(TSP_BF16, D, Q, K, V, dO, H, S, crow, Mt, scale, plan + 4, n_items, n_partials,
+                                       qstat, dK, dV, partial, st);
+    } else {
+      const int64_t nslots = tsp::ceil_div(n_items * H, 8), most = D == 64 ? 64 : 32;  // workgroups per XCD
+      const int64_t g8 = nslots < most ? nslots : most;
+      hipLaunchKernelGGL((bsa_bwd_dkdv_bf16<D>), dim3((unsigned)(8 * g8)), dim3(256), 0, st, (const uint16_t*)Q,
+                         (const uint16_t*)K, (const uint16_t*)V, (const uint16_t*)dO, S, H, crow, plan + 4,
+                         (int)n_items, (int)n_partials, sl2, (float)scale, (const float*)qstat, (uint16_t*)dK,
+                         (uint16_t*)dV, partial);
+      rc = tsp::check_launch("bsa_bwd_dkdv_bf16 launch");
+    }
     if (rc) return rc;
   }
   if (n_splits > 0) {
@@ -1134,17 +1148,28 @@ int launch_f32(const void* Q, const void* K, const void* V, const void* O, const
     if (rc) return rc;
   } else {
     if (grid_a > 0) {
-      hipLaunchKernelGGL((bsa_bwd_dq_f32<D>), dim3((unsigned)grid_a), dim3(256), 0, st, (const float*)Q,
-                         (const float*)K, (const float*)V, (const float*)O, (const float*)dO, S, H, rp, ci, Mt, sl2,
-                         (float)scale, (const float*)rmax, (const float*)rden, qstat, (float*)dQ);
-      int rc = tsp::check_launch("bsa_bwd_dq_f32 launch");
+      int rc;
+      if (tsp::attn_split_dq_pays(TSP_F32, D, H, Mt)) {
+        rc = tsp::launch_attn_split_dq(TSP_F32, D, Q, K, V, O, dO, H, S, rp, ci, Mt, scale, rmax, rden, qstat, dQ, st);
+      } else {
+        hipLaunchKernelGGL((bsa_bwd_dq_f32<D>), dim3((unsigned)grid_a), dim3(256), 0, st, (const float*)Q,
+                           (const float*)K, (const float*)V, (const float*)O, (const float*)dO, S, H, rp, ci, Mt, sl2,
+                           (float)scale, (const float*)rmax, (const float*)rden, qstat, (float*)dQ);
+        rc = tsp::check_launch("bsa_bwd_dq_f32 launch");
+      }
       if (rc) return rc;
     }
     if (grid_b > 0) {
-      hipLaunchKernelGGL((bsa_bwd_dkdv_f32<D>), dim3((unsigned)grid_b), dim3(256), 0, st, (const float*)Q,
-                         (const float*)K, (const float*)V, (const float*)dO, S, H, crow, plan + 4, (int)n_partials, Mt,
-                         sl2, (float)scale, (const float*)qstat, (float*)dK, (float*)dV, partial);
-      int rc = tsp::check_launch("bsa_bwd_dkdv_f32 launch");
+      int rc;
+      if (D == 64 || tsp::attn_split_dkdv_pays(TSP_F32, D, H, n_items)) {
+        rc = tsp::launch_attn_split_dkdv(TSP_F32, D, Q, K, V, dO, H, S, crow, Mt, scale, plan + 4, n_items, n_partials,
+                                         qstat, dK, dV, partial, st);
+      } else if constexpr (D != 64) {
+        hipLaunchKernelGGL((bsa_bwd_dkdv_f32<D>), dim3((unsigned)grid_b), dim3(256), 0, st, (const float*)Q,
+                           (const float*)K, (const float*)V, (const float*)dO, S, H, crow, plan + 4, (int)n_partials,
+                           Mt, sl2, (float)scale, (const float*)qstat, (float*)dK, (float*)dV, partial);
+        rc = tsp::check_launch("bsa_bwd_dkdv_f32 launch");
+      }
       if (rc) return rc;
     }
   }

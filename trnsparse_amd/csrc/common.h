@@ -53,6 +53,23 @@ int launch_bsr_flex_sddmm(int dtype, int64_t b, const void* G, int64_t ldg, int6
                           int64_t n, int64_t ncols, const int64_t* brow, const int64_t* bcol, int64_t nnzb, void* out,
                           hipStream_t st);
 
+// Attention on small grids (attention_split.hip): fp32 or bf16, 128-blocks,
+// 16-byte aligned operands, scale > 0. Each pass pays where the full-grid
+// kernel leaves CUs idle (never at head_dims other than 64 and 128).
+bool attn_split_fwd_pays(int dtype, int64_t D, int64_t H, int64_t Mt);
+bool attn_split_dq_pays(int dtype, int64_t D, int64_t H, int64_t Mt);
+bool attn_split_dkdv_pays(int dtype, int64_t D, int64_t H, int64_t n_items);
+int launch_attn_split_fwd(int dtype, int64_t D, const void* Q, const void* K, const void* V, int64_t H, int64_t S,
+                          const int64_t* rp, const int64_t* ci, int64_t Mt, double scale, void* O, void* rmax,
+                          void* rden, hipStream_t st);
+int launch_attn_split_dq(int dtype, int64_t D, const void* Q, const void* K, const void* V, const void* O,
+                         const void* dO, int64_t H, int64_t S, const int64_t* rp, const int64_t* ci, int64_t Mt,
+                         double scale, const void* rmax, const void* rden, float* qstat, void* dQ, hipStream_t st);
+int launch_attn_split_dkdv(int dtype, int64_t D, const void* Q, const void* K, const void* V, const void* dO, int64_t H,
+                           int64_t S, const int64_t* crow, int64_t Mt, double scale, const int32_t* items,
+                           int64_t n_items, int64_t n_partials, const float* qstat, void* dK, void* dV, float* partial,
+                           hipStream_t st);
+
 // ---------------------------------------------------------------- bf16
 // Round-to-nearest-even fp32 -> bf16 bit pattern (NaN kept quiet), the same
 // rounding torch applies in `tensor.to(torch.bfloat16)`.
