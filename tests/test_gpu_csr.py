@@ -18,6 +18,7 @@ import trnsparse_amd as ts
 from oracle import build as oracle_c
 from oracle import ref
 from trnsparse_amd import workloads as W
+from trnsparse_amd.hip import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -184,6 +185,25 @@ def test_spmm_any_width(hip_backend, N, offset):
         Bi[:, 0] = float("inf")
         again = ts.spmm(A, Bi, 1.5, C, -0.5)
         assert torch.equal(again[:, 1:], out.detach()[:, 1:])
+
+
+@pytest.mark.parametrize("N", [2, 7, 64, 129, 130, 131, 259])
+def test_spmm_in_place(hip_backend, N):
+    """The C entry with C and out one array: every element is scaled and added
+    to once, also where the last column part overlaps its neighbour's (in
+    another wavefront past 128 columns). fp32 sums of at most 70 products."""
+    rng = np.random.default_rng(N)
+    lens = rng.poisson(6, size=3000)
+    lens[:4] = (0, 70, 1, 64)
+    v, c, p = W.random_csr(lens, 900, rng)
+    Bn, Cn = (rng.standard_normal((rows, N), dtype=np.float32) for rows in (900, 3000))
+    vd, cd, pd, B, C = (torch.from_numpy(np.ascontiguousarray(t)).cuda() for t in (v, c, p, Bn, Cn))
+    assert vd.dtype == torch.float32 and cd.dtype == pd.dtype == torch.int64
+    _lib.call("tsp_csr_spmm", vd.data_ptr(), _lib.TSP_F32, cd.data_ptr(), pd.data_ptr(),
+              _lib.TSP_I64, 3000, 900, vd.numel(), B.data_ptr(), N, N, 1.5, C.data_ptr(), N, -0.5,
+              C.data_ptr(), N, _lib.stream_handle(C.device))
+    exact, scale = (ref.csr_spmm(v, c, p, (3000, 900), Bn, 1.5, Cn, -0.5, absolute=a) for a in (False, True))
+    assert ref.scaled_error(C.cpu().numpy(), exact, scale) <= TOL
 
 
 def _csr_from_lengths(lens, n, seed, index_dtype=np.int64):

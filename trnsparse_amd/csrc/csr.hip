@@ -234,15 +234,16 @@ struct Part<T, 3> {
 // side in a wavefront, so narrow B still fills the wavefront and every B
 // access is a 16-byte load at any alignment. Where 4 does not divide ncols
 // the last quad starts at ncols - 4: it overlaps its neighbour, and both
-// write the same values (the same products added in the same order). Fewer
+// write the same values (the same products added in the same order); with a
+// C it writes its own columns only, so that C and out may be one array. Fewer
 // than 4 columns are one part of V = ncols. U nonzeros per group are fetched
 // before their B rows are loaded (U independent gathers in flight per lane).
 // The groups' partial sums are added with xor shuffles at the end of the rows.
 template <typename IdxT, int V, int P, int G>
 __global__ __launch_bounds__(256) void csr_spmm_narrow_kernel(
     const float* __restrict__ vals, const IdxT* __restrict__ cols, const IdxT* __restrict__ ptr, int64_t m,
-    const float* __restrict__ B, int64_t ldb, int64_t ncols, float alpha, const float* __restrict__ Cin,
-    int64_t ldci, float beta, float* __restrict__ out, int64_t ldo) {
+    const float* __restrict__ B, int64_t ldb, int64_t ncols, float alpha, const float* Cin,
+    int64_t ldci, float beta, float* out, int64_t ldo) {
   typedef Part<float, V> Q;
   typedef typename Q::reg vec;
   constexpr int R = 64 / (P * G);
@@ -287,7 +288,15 @@ __global__ __launch_bounds__(256) void csr_spmm_narrow_kernel(
     }
     if (gi == 0 && r < m && cvalid) {
       vec res = alpha * acc;
-      if (Cin) res = res + beta * Q::load(Cin + r * ldci + c0);
+      if (Cin) {
+        res = res + beta * Q::load(Cin + r * ldci + c0);
+        if (c0 != cw) {  // out may be C, where another wavefront's columns are not to be added twice
+#pragma unroll
+          for (int i = 1; i < V; ++i)
+            if (c0 + i >= cw) out[r * ldo + c0 + i] = res[i];
+          continue;
+        }
+      }
       Q::store(out + r * ldo + c0, res);
     }
   }
