@@ -26,6 +26,7 @@ import torch
 import trnsparse_amd as ts
 from oracle import ref
 from trnsparse_amd import workloads as W
+from trnsparse_amd.hip import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -271,3 +272,22 @@ def test_backward_block_products_batched_heads(hip_backend, D, dtype):
     assert torch.count_nonzero(dQ[:, 256:384]).item() == 0
     for hh in range(H):
         _check_head(Q[hh], K[hh], V[hh], dO[hh], O[hh], (dQ[hh], dK[hh], dV[hh]), mask_bsr, D**-0.5, TOL[dtype])
+
+
+@pytest.mark.parametrize(
+    "H,S,D,b,dtype",
+    [(6, 1243, 128, 128, torch.bfloat16), (3, 300, 64, 128, torch.float32), (1100, 19, 3, 8, torch.bfloat16),
+     (5, 19, 3, 8, torch.float32), (2, 5, 1, 8, torch.float64), (1, 129, 2, 128, torch.bfloat16)],
+)
+def test_rows_past_the_whole_blocks(hip_backend, H, S, D, b, dtype):
+    """The forward entry on a mask without blocks zeroes every head's rows,
+    those past its whole blocks too (stores of 16, 4 and 1 bytes, more heads
+    than one grid's rows), and nothing past the last head."""
+    Q = torch.randn(H, S, D, device="cuda").to(dtype)
+    O = torch.full((H * S * D + 64,), float("nan"), dtype=dtype, device="cuda")
+    rp = torch.zeros(S // b + 1, dtype=torch.int64, device="cuda")
+    ci = torch.zeros(1, dtype=torch.int64, device="cuda")
+    _lib.call("tsp_bsa_fwd", Q.data_ptr(), Q.data_ptr(), Q.data_ptr(), _lib.dtype_code(dtype), H, S, D, rp.data_ptr(),
+              ci.data_ptr(), b, D**-0.5, O.data_ptr(), None, None, _lib.stream_handle(O.device))
+    assert torch.count_nonzero(O[: H * S * D]).item() == 0
+    assert torch.isnan(O[H * S * D :]).all().item()

@@ -1061,14 +1061,14 @@ extern "C" int tsp_bsa_fwd(const void* Q, const void* K, const void* V, int dtyp
   if (n_heads == 0 || seq_len == 0 || head_dim == 0) return TSP_OK;
   if (!Q || !K || !V || !O || !block_row_ptrs || !block_col_indices) return tsp::fail(TSP_EINVAL, "tsp_bsa_fwd: null pointer");
   hipStream_t st = (hipStream_t)stream;
-  // rows past Mt*block_size have no block row: zero output (the reference's out starts at zero)
+  // rows past Mt*block_size have no block row: zero output (the reference's out starts at zero).
+  // One launch for all heads, here and for dQ: one per head took 13 us of 6 heads' forward and as
+  // much of their backward
   if (Mt * block_size < seq_len) {
     const int64_t es = dtype == TSP_F64 ? 8 : (dtype == TSP_F32 ? 4 : 2);
     const int64_t tail = (seq_len - Mt * block_size) * head_dim * es;
-    for (int64_t hh = 0; hh < n_heads; ++hh) {
-      int rc = tsp::zero_fill((char*)O + (hh * seq_len + Mt * block_size) * head_dim * es, tail, st);
-      if (rc) return rc;
-    }
+    int rc = tsp::zero_fill_rows((char*)O + Mt * block_size * head_dim * es, n_heads, seq_len * head_dim * es, tail, st);
+    if (rc) return rc;
   }
   if (Mt == 0) return TSP_OK;
   const bool bf16_streamed = scale > 0 && (seq_len + AB) * head_dim * 2 <= (int64_t)UINT32_MAX;

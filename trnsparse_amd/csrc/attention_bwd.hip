@@ -1077,10 +1077,8 @@ int launch_bf16(const void* Q, const void* K, const void* V, const void* O, cons
   float* partial = (float*)((char*)workspace + 16 * H * S);
   if (Mt * abw::BS < S) {  // rows without a block row: zero dQ
     const int64_t tail = (S - Mt * abw::BS) * D * 2;
-    for (int64_t hh = 0; hh < H; ++hh) {
-      int rc = tsp::zero_fill((char*)dQ + (hh * S + Mt * abw::BS) * D * 2, tail, st);
-      if (rc) return rc;
-    }
+    int rc = tsp::zero_fill_rows((char*)dQ + Mt * abw::BS * D * 2, H, S * D * 2, tail, st);
+    if (rc) return rc;
   }
   if (grid_a > 0) {
     int rc;
@@ -1132,10 +1130,8 @@ int launch_f32(const void* Q, const void* K, const void* V, const void* O, const
   float* partial = (float*)((char*)workspace + 16 * H * S);
   if (Mt * 128 < S) {  // rows without a block row: zero dQ
     const int64_t tail = (S - Mt * 128) * D * 4;
-    for (int64_t hh = 0; hh < H; ++hh) {
-      int rc = tsp::zero_fill((char*)dQ + (hh * S + Mt * 128) * D * 4, tail, st);
-      if (rc) return rc;
-    }
+    int rc = tsp::zero_fill_rows((char*)dQ + Mt * 128 * D * 4, H, S * D * 4, tail, st);
+    if (rc) return rc;
   }
   if constexpr (D == 256) {  // 16-row tiles, half a block per workgroup (attention_bwd_d256.hip)
     int rc = tsp::bsa_bwd_f32_d256_rows((const float*)Q, (const float*)K, (const float*)V, (const float*)O,

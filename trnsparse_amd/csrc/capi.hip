@@ -23,18 +23,33 @@ int check_hip(hipError_t e, const char* what) {
 
 int check_launch(const char* what) { return check_hip(hipGetLastError(), what); }
 
-__global__ __launch_bounds__(256) void zero_fill_kernel(uint8_t* __restrict__ p, int64_t n) {
+// rows of n units, `ld` units apart. Bound by the launch for small fills and by
+// the writes for large ones.
+template <typename U>
+__global__ __launch_bounds__(256) void zero_fill_kernel(U* __restrict__ p, int64_t rows, int64_t ld, int64_t n) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = 0;
+  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y)
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[r * ld + i] = U{};
 }
 
-int zero_fill(void* p, int64_t bytes, hipStream_t st) {
-  if (bytes <= 0) return TSP_OK;
-  int64_t grid = ceil_div(bytes, 256);
-  if (grid > 4096) grid = 4096;
-  hipLaunchKernelGGL(zero_fill_kernel, dim3((unsigned)grid), dim3(256), 0, st, (uint8_t*)p, bytes);
-  return check_launch("zero_fill launch");
+int zero_fill_rows(void* p, int64_t rows, int64_t ld, int64_t bytes, hipStream_t st) {
+  if (rows <= 0 || bytes <= 0) return TSP_OK;
+  auto go = [&](auto unit) {
+    typedef decltype(unit) U;
+    const int64_t n = bytes / (int64_t)sizeof(U), gy = rows < 1024 ? rows : 1024, most = 4096 / gy;
+    const int64_t gx = ceil_div(n, 256) < most ? ceil_div(n, 256) : most;
+    hipLaunchKernelGGL(zero_fill_kernel<U>, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, st, (U*)p, rows,
+                       ld / (int64_t)sizeof(U), n);
+    return check_launch("zero_fill launch");
+  };
+  // the widest store that the address, the row stride and the row length allow
+  const uint64_t all = (uint64_t)(uintptr_t)p | (uint64_t)bytes | (rows > 1 ? (uint64_t)ld : 0);
+  if (all % 16 == 0) return go(u32x4{});
+  if (all % 4 == 0) return go(uint32_t{});
+  return go(uint8_t{});
 }
+
+int zero_fill(void* p, int64_t bytes, hipStream_t st) { return zero_fill_rows(p, 1, 0, bytes, st); }
 
 }  // namespace tsp
 

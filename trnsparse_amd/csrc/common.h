@@ -30,6 +30,8 @@ int check_launch(const char* what);
 // Zero `bytes` bytes at device pointer p with a fill kernel on `st` (used
 // instead of hipMemsetAsync so callers may capture the work in a HIP graph).
 int zero_fill(void* p, int64_t bytes, hipStream_t st);
+// The same for `rows` runs of `bytes` bytes that start `ld` bytes apart, in one launch.
+int zero_fill_rows(void* p, int64_t rows, int64_t ld, int64_t bytes, hipStream_t st);
 
 // Whether bsr_spmm_small serves these operands (block sizes 8 and 16; B or, in
 // the backward, dC).

@@ -1062,11 +1062,7 @@ extern "C" int tsp_screened_spmm_backward(const void* A, int dtype, int64_t lda,
   if (ncols == 0) {  // dA = 0 (an empty sum); dB has no columns
     if (!dA) return TSP_OK;
     const int64_t es = dtype == TSP_F64 ? 8 : 4;
-    for (int64_t r = 0; r < m; ++r) {
-      int rc = tsp::zero_fill((char*)dA + r * ldda * es, m * es, st);
-      if (rc) return rc;
-    }
-    return TSP_OK;
+    return tsp::zero_fill_rows(dA, m, ldda * es, m * es, st);
   }
   return diag_dtype == TSP_F32
              ? launch_backward<float>(A, dtype, lda, diag, threshold_sqrt, m, B, ldb, ncols, dC, lddc, dA, ldda, dB,
