@@ -274,6 +274,18 @@ def test_backward_block_products_batched_heads(hip_backend, D, dtype):
         _check_head(Q[hh], K[hh], V[hh], dO[hh], O[hh], (dQ[hh], dK[hh], dV[hh]), mask_bsr, D**-0.5, TOL[dtype])
 
 
+@pytest.mark.parametrize("H", [1, 3])
+@pytest.mark.parametrize("D,dtype", [(320, torch.float32), (512, torch.float32), (640, torch.bfloat16)])
+def test_backward_block_products_without_blocks(hip_backend, D, dtype, H):
+    """Block products over a mask that keeps no block: the output and every
+    gradient are zero (the one-pass kernels refuse such a mask)."""
+    mask_bsr = W.bsr_from_block_mask(torch.zeros(3, 3, dtype=torch.bool), 128)
+    g = torch.Generator().manual_seed(71)
+    Q, K, V, dO = (torch.randn(H, 384, D, generator=g).to(dtype) for _ in range(4))
+    for t in _run(Q, K, V, dO, mask_bsr):
+        assert t.shape == Q.shape and torch.count_nonzero(t).item() == 0
+
+
 @pytest.mark.parametrize(
     "H,S,D,b,dtype",
     [(6, 1243, 128, 128, torch.bfloat16), (3, 300, 64, 128, torch.float32), (1100, 19, 3, 8, torch.bfloat16),

@@ -105,6 +105,19 @@ def test_backward_empty_rows_and_columns(hip_backend):
     assert torch.count_nonzero(dB[128:256]).item() == 0  # block column 1 holds no blocks
 
 
+@pytest.mark.parametrize("b,N", [(8, 24), (16, 130), (32, 24), (128, 64), (128, 77), (24, 5)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float64])
+def test_backward_empty_pattern(hip_backend, dtype, b, N):
+    """No stored block at all: dB is zero and dA has no blocks."""
+    bsr = ts.BSRMatrix.from_dense(torch.zeros(300, 260, dtype=dtype), block_size=b)
+    assert bsr.n_blocks == 0
+    g = torch.Generator().manual_seed(8)
+    B, G = (torch.randn(rows, N, generator=g, dtype=torch.float64).to(dtype) for rows in (260, 300))
+    db, dB = _grads(bsr, B, G)
+    assert db.shape == (0, b, b) and db.dtype == dtype
+    assert dB.shape == (260, N) and dB.dtype == dtype and torch.count_nonzero(dB).item() == 0
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float64])
 def test_backward_long_block_column(hip_backend, dtype):
     """A block column with 65 stored blocks (the dB kernels read a column's

@@ -212,10 +212,13 @@ at::Tensor bsr_spmm_t(const at::Tensor& blocks, const at::Tensor& cp, const at::
   }
   const int64_t ncols = G.size(1), nbc = cp.numel() - 1;
   auto out = at::empty({n, ncols}, G.options());
+  // The entry point refuses null lists, and those of a pattern without blocks
+  // have no storage: col_ptrs stands in for them (nothing reads an empty list).
+  const bool stored = blocks.size(0) > 0;
   check(tsp_bsr_spmm_t(blocks.data_ptr(), dtype_code(blocks.scalar_type()), cp.data_ptr<int64_t>(),
-                       cbid.data_ptr<int64_t>(), crow.data_ptr<int64_t>(), nbc, block_size, m, n, G.data_ptr(), ldg,
-                       ncols, out.data_ptr(), ncols, col_order.numel() ? col_order.data_ptr<int32_t>() : nullptr,
-                       stream_of(G)),
+                       (stored ? cbid : cp).data_ptr<int64_t>(), (stored ? crow : cp).data_ptr<int64_t>(), nbc,
+                       block_size, m, n, G.data_ptr(), ldg, ncols, out.data_ptr(), ncols,
+                       col_order.numel() ? col_order.data_ptr<int32_t>() : nullptr, stream_of(G)),
         "tsp_bsr_spmm_t");
   return out;
 }
