@@ -303,3 +303,39 @@ def test_rows_past_the_whole_blocks(hip_backend, H, S, D, b, dtype):
               ci.data_ptr(), b, D**-0.5, O.data_ptr(), None, None, _lib.stream_handle(O.device))
     assert torch.count_nonzero(O[: H * S * D]).item() == 0
     assert torch.isnan(O[H * S * D :]).all().item()
+
+
+@pytest.mark.parametrize("S", [300, 10])
+@pytest.mark.parametrize("D", [64, 128])
+def test_column_rows_past_the_whole_blocks_f32(hip_backend, D, S):
+    """A column view that lists block rows past the whole blocks (all of a
+    sequence shorter than a block): they have no queries, so nothing is read
+    for them, no non-finite value of another block row reaches dK or dV, and
+    the workspace of 16 bytes per row suffices."""
+    H, nb, Mt = 2, -(-S // 128), S // 128
+    g = torch.Generator().manual_seed(72)
+    Q, K, V, O, dO = (torch.randn(H, S, D, generator=g).cuda() for _ in range(5))
+    Q[:, :128] = float("nan")
+    dO[:, :128] = float("inf")
+    cols = [[c, Mt] if c < Mt else [Mt] for c in range(nb)]  # block c keeps its own rows and the ragged ones
+    cols[0] = [Mt]
+    cp = np.concatenate([[0], np.cumsum([len(c) for c in cols])]).astype(np.int64)
+    lib = _lib.load()
+    n = lib.tsp_bsa_bwd_plan(cp.ctypes.data, nb, H, S, 128, None, 0)
+    plan = np.empty(n, dtype=np.int32)
+    assert lib.tsp_bsa_bwd_plan(cp.ctypes.data, nb, H, S, 128, plan.ctypes.data, n) == n
+    dev = [torch.from_numpy(a).cuda() for a in (cp, np.concatenate(cols).astype(np.int64), plan)]
+    rp, ci = torch.arange(Mt + 1).cuda(), torch.arange(max(Mt, 1)).cuda()
+    rmax, rden = torch.zeros(H, max(Mt, 1) * 128).cuda(), torch.full((H, max(Mt, 1) * 128), 128.0).cuda()
+    out = [torch.full_like(Q, float("nan")) for _ in range(3)]
+    ws = torch.empty(lib.tsp_bsa_bwd_workspace_size(H, S, D, int(plan[2])), dtype=torch.uint8, device="cuda")
+    _lib.call("tsp_bsa_bwd", Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dO.data_ptr(), _lib.TSP_F32, H, S,
+              D, rp.data_ptr(), ci.data_ptr(), dev[0].data_ptr(), dev[1].data_ptr(), nb, 128, D**-0.5,
+              rmax.data_ptr(), rden.data_ptr(), *(t.data_ptr() for t in out), dev[2].data_ptr(),
+              *(int(x) for x in plan[:3]), ws.data_ptr(), _lib.stream_handle(Q.device))
+    own = slice(128, 128 * Mt)  # keys with queries of their own
+    for t in out[1:]:
+        assert torch.isfinite(t).all().item()
+        t[:, own] = 0.0
+        assert torch.count_nonzero(t).item() == 0
+    assert torch.count_nonzero(out[0][:, 128 * Mt :]).item() == 0

@@ -465,16 +465,21 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bsa_bwd_dkdv_split(
   List ahead(crow + p0, nblk, lane), here(crow + p0, nblk, lane);
   auto st = make_stream<T, D, 1>(
       [&](int i, int which, uint32_t dst) {
-        const int64_t row = ahead.get(i, lane), q0 = (row < Mt ? row : 0) * BS + 32 * w;
+        // rows past the whole blocks have no queries and no statistics: their
+        // tiles are read past the buffers' ends, as zeros, and any 16 bytes of
+        // this head stand in for the statistics
+        const int64_t row = ahead.get(i, lane), q0 = row < Mt ? row * BS + 32 * w : S;
         TL::fetch(which ? qrs : ors, q0, dst, lane);
         // with dO: lanes 0-7 r, the rest D (from lane 16 on repeated)
-        if (which == 0)
-          tsp::dma::global16(qstat + (lane & 8 ? HS : 0) + head * S + q0 + 4 * (lane & 7), dst + TL::BYTES);
+        if (which == 0) {
+          const float* stat = qstat + (lane & 8 ? HS : 0) + head * S + q0 + 4 * (lane & 7);
+          tsp::dma::global16(row < Mt ? (const void*)stat : (const void*)(Q + hs), dst + TL::BYTES);
+        }
       },
       tsp::dma::lds_addr(lds) + w * WAVE, nblk);
   st.start();
   for (int i = 0; i < nblk; ++i) {
-    const bool there = here.get(i, lane) < Mt;  // rows past the whole blocks have no queries
+    const bool there = here.get(i, lane) < Mt;
     const uint8_t* ot = lds_ptr(st.first(i));
     f32x16 dp = TL::scores(ot, vf, h, l32);
     const uint8_t* qt = lds_ptr(st.template second<false>(i));
