@@ -334,3 +334,34 @@ def test_small_tiles_forward_and_backward(hip_backend, n, N, offset):
     _check(A.detach(), diag, B.detach(), thr, C.detach())
     dA, dB = torch.autograd.grad(C, (A, B), G)
     _check_backward(A.detach(), diag, B.detach(), thr, G, dA, dB, TOL)
+
+
+@pytest.mark.parametrize("n,N,N_odd", [(321, 130, True), (321, 132, False), (320, 131, True)])
+def test_non_finite_entries_beside_masked_pairs(hip_backend, n, N, N_odd):
+    """Rows that are not 16-byte aligned: infinities and NaN in A, B and dC
+    whose pairs the threshold masks in whole 128-row tiles reach C, dA and dB
+    as inf * 0 does in the definition, (A * mask) @ B. A row or column without
+    one is unchanged. (n = 321, N = 132: dA's operands are aligned, and its
+    masked tiles are written as zeros.)"""
+    g = torch.Generator().manual_seed(n + N)
+    A, B, G = (torch.randn(n, k, generator=g) for k in (n, N, N))
+    diag = torch.pow(10.0, -4.0 * torch.arange(n) / (n - 1)).float()  # 1 .. 1e-4, descending
+    thr = 1.0437e-5  # masks the last tile's rows against each other, whole tiles of them
+    mask = torch.from_numpy(ref.screened_mask(diag.numpy(), thr))
+    assert not mask[256:, 256:].any()
+    A[300, 310] = float("inf")  # masked: NaN in row 300 of C, row 310 of dB
+    B[305, 7] = float("nan")    # column 7 of C; dA: column 305
+    G[290, 9] = float("-inf")   # column 9 of dB; dA: row 290
+    Ad, Bd = A.cuda().requires_grad_(True), B.cuda().requires_grad_(True)
+    C = ts.screened_spmm(Ad, diag.cuda(), Bd, threshold=thr)
+    dA, dB = torch.autograd.grad(C, (Ad, Bd), G.cuda())
+    Am = A.double() * mask
+    exact = [Am @ B.double(), (G.double() @ B.double().T) * mask, Am.T @ G.double()]
+    for name, got, want in zip(("C", "dA", "dB"), (C, dA, dB), exact):
+        if name == "dA" and not N_odd:
+            want[256:, 256:] = 0.0
+        got = got.detach().cpu().double()
+        for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(kind(got), kind(want)), (name, kind)
+        there = torch.isfinite(want)
+        assert (got - want)[there].abs().max().item() <= 1e-3, name  # |sums of 321 products| below 100, fp32

@@ -14,7 +14,9 @@
 // then every pair in it is masked (all Q >= 0 and rounded multiplication is
 // monotonic), so the K tile is skipped. With finite A and B this is exactly
 // the reference result; with non-finite entries inside a fully masked tile
-// the reference would propagate NaN from inf * 0 and the skip does not.
+// the reference would propagate NaN from inf * 0 and the skip does not. fp32
+// operands whose rows are not 16-byte aligned visit every tile (`skip` below),
+// and so have the reference's result for non-finite entries too.
 //
 // Kernels
 //   screened_q          Q and the per-128-row-tile maximum of Q (workspace).
@@ -349,7 +351,9 @@ __global__ __launch_bounds__(256) void screened_f64_dma(
 // multiplies each A element once, while it is staged. The tile skip keeps
 // its 128-row granularity. Rows that are not 16-byte aligned always take
 // them: n = N = 1111 forward 767 -> 62 us, dA 4080 -> 54, dB 834 -> 64 against
-// one thread per output (host-timed calls, launch of screened_q included).
+// one thread per output (host-timed calls, launch of screened_q included);
+// like that form they take every tile (!skip), so that an infinity or NaN
+// beside a masked pair reaches the result as the definition has it.
 namespace X = tsp::flex;
 constexpr int FT = 64;  // output tile: FT x FT
 typedef X::Split<32, FT, FT> FSplit;
@@ -373,15 +377,18 @@ bool small_tiles_faster(int64_t row_items, int64_t col_items, int one, int two, 
   return big / 2 * two + big % 2 * one > tiny * small;
 }
 
-// Walks the 128-row tiles t with qo * qmax[t] > thr in order.
+// Walks the 128-row tiles t with qo * qmax[t] > thr, or all (!skip), in order.
 template <typename QT>
 struct ActiveTiles {
   const QT* __restrict__ qmax;
   QT qo, thr;
   int t;
-  __device__ ActiveTiles(const QT* qmax_, int own, QT thr_) : qmax(qmax_), qo(qmax_[own]), thr(thr_), t(-1) {}
+  bool skip;
+  __device__ ActiveTiles(const QT* qmax_, int own, QT thr_, bool skip_)
+      : qmax(qmax_), qo(qmax_[own]), thr(thr_), t(-1), skip(skip_) {}
   // slabs of all active tiles (rows at or past m, in the last tile, have none)
   __device__ int slabs(int nkt, int64_t m) const {
+    if (!skip) return (int)tsp::ceil_div(m, X::KC);
     int c = 0;
     for (int t0 = 0; t0 < nkt; t0 += 64) {
       const int i = t0 + (int)(threadIdx.x & 63);
@@ -395,7 +402,7 @@ struct ActiveTiles {
   __device__ int64_t row(int s) {
     if (s % SPT == 0) {
       ++t;
-      while (!(qo * qmax[t] > thr)) ++t;
+      while (skip && !(qo * qmax[t] > thr)) ++t;
     }
     return (int64_t)t * TILE + (s % SPT) * X::KC;
   }
@@ -433,14 +440,14 @@ template <typename QT>
 __global__ __launch_bounds__(X::NTHR, 4) void screened_f32_flex(
     const float* __restrict__ A, int64_t lda, const QT* __restrict__ Q, const QT* __restrict__ qmax, QT thr,
     int64_t m, const float* __restrict__ B, int64_t ldb, int64_t ncols, float* __restrict__ C, int64_t ldc, int nmt,
-    int nnt) {
+    int nnt, bool skip) {
   __shared__ __attribute__((aligned(16))) float lds[X::lds_floats<FRow, FCol>()];
   int64_t mt;
   int nt;
   // XCD-aware: the column tiles of one row panel of A share an XCD (and its L2)
   if (!tsp::tile_item(blockIdx.x, nmt, nnt, nullptr, mt, nt)) return;
   const int64_t row0 = mt * FT, n0 = (int64_t)nt * FT;
-  FlexFwd<QT> src{A, B, Q, lda, ldb, m, ncols, row0, n0, {qmax, (int)(row0 / TILE), thr}, {}};
+  FlexFwd<QT> src{A, B, Q, lda, ldb, m, ncols, row0, n0, {qmax, (int)(row0 / TILE), thr, skip}, {}};
 #pragma unroll
   for (int j = 0; j < 2; ++j) src.qr[j] = Q[row0 + FRow::i() + 32 * j];
   float acc[8];
@@ -717,7 +724,8 @@ __global__ __launch_bounds__(X::NTHR, 4) void screened_bwd_a_flex(const float* _
                                                                const float* __restrict__ B, int64_t ldb,
                                                                int64_t ncols, const QT* __restrict__ Q,
                                                                const QT* __restrict__ qmax, QT thr, int64_t m,
-                                                               int nmt, float* __restrict__ dA, int64_t ldda) {
+                                                               int nmt, float* __restrict__ dA, int64_t ldda,
+                                                               bool skip) {
   __shared__ __attribute__((aligned(16))) float lds[X::lds_floats<FRow, FRow>()];
   // XCD-aware: XCD x takes a contiguous range of tiles, as in screened_bwd_a_f32
   const int64_t ntiles = (int64_t)nmt * nmt, per = tsp::ceil_div(ntiles, 8);
@@ -725,7 +733,7 @@ __global__ __launch_bounds__(X::NTHR, 4) void screened_bwd_a_flex(const float* _
   if (slot >= per || tix >= ntiles) return;
   const int64_t r0 = tix / nmt * FT, c0 = tix % nmt * FT;
   float acc[8] = {};
-  if (qmax[r0 / TILE] * qmax[c0 / TILE] > thr) {  // else every pair is masked: zeros
+  if (!skip || qmax[r0 / TILE] * qmax[c0 / TILE] > thr) {  // else every pair is masked: zeros
     FlexBwdA src{G, B, ldg, ldb, m, ncols, r0, c0};
     X::run<FSplit>(src, (int)tsp::ceil_div(ncols, X::KC), lds, acc);
   }
@@ -773,13 +781,13 @@ __global__ __launch_bounds__(X::NTHR, 4) void screened_bwd_b_flex(const float* _
                                                                int64_t ncols, const QT* __restrict__ Q,
                                                                const QT* __restrict__ qmax, QT thr, int64_t m,
                                                                int nmt, int nnt, float* __restrict__ dB,
-                                                               int64_t lddb) {
+                                                               int64_t lddb, bool skip) {
   __shared__ __attribute__((aligned(16))) float lds[X::lds_floats<FCol, FCol>()];
   int64_t jt;
   int nt;
   if (!tsp::tile_item(blockIdx.x, nmt, nnt, nullptr, jt, nt)) return;
   const int64_t k0 = jt * FT, n0 = (int64_t)nt * FT;
-  FlexBwdB<QT> src{A, G, Q, lda, ldg, m, ncols, k0, n0, {qmax, (int)(k0 / TILE), thr}, {}};
+  FlexBwdB<QT> src{A, G, Q, lda, ldg, m, ncols, k0, n0, {qmax, (int)(k0 / TILE), thr, skip}, {}};
 #pragma unroll
   for (int c = 0; c < 4; ++c) src.qc[c] = Q[k0 + FCol::i() + c];
   float acc[8];
@@ -847,12 +855,13 @@ int launch_backward(const void* A, int dtype, int64_t lda, const void* diag, dou
   const bool f32 = dtype == TSP_F32 && fits(G, ldg);
   const int64_t nmt64 = tsp::ceil_div(m, FT);
   if (dA) {
-    if (dtype == TSP_F32 && (!(f32 && fits(B, ldb)) || small_tiles_faster(m, m, 68, 136, 18))) {
+    const bool streamed = f32 && fits(B, ldb);
+    if (dtype == TSP_F32 && (!streamed || small_tiles_faster(m, m, 68, 136, 18))) {
       const int64_t grid = tsp::ceil_div(nmt64 * nmt64, 8) * 8;
       if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm_backward: problem too large");
       hipLaunchKernelGGL((screened_bwd_a_flex<QT>), dim3((unsigned)grid), dim3(X::NTHR), 0, st, (const float*)G, ldg,
                          (const float*)B, ldb, ncols, (const QT*)Q, (const QT*)qmax, thr, m, (int)nmt64, (float*)dA,
-                         ldda);
+                         ldda, streamed);
       rc = tsp::check_launch("screened_bwd_a_flex launch");
     } else if (dtype == TSP_F32) {
       const int64_t grid = tsp::ceil_div(nmt * nmt, 8) * 8;
@@ -871,12 +880,13 @@ int launch_backward(const void* A, int dtype, int64_t lda, const void* diag, dou
     if (rc) return rc;
   }
   if (dB) {
-    if (dtype == TSP_F32 && (!(f32 && fits(A, lda)) || small_tiles_faster(m, ncols, 77, 154, 21))) {
+    const bool streamed = f32 && fits(A, lda);
+    if (dtype == TSP_F32 && (!streamed || small_tiles_faster(m, ncols, 77, 154, 21))) {
       const int64_t nnt = tsp::ceil_div(ncols, FT), grid = tsp::ceil_div(nmt64, 8) * 8 * nnt;
       if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm_backward: problem too large");
       hipLaunchKernelGGL((screened_bwd_b_flex<QT>), dim3((unsigned)grid), dim3(X::NTHR), 0, st, (const float*)A, lda,
                          (const float*)G, ldg, ncols, (const QT*)Q, (const QT*)qmax, thr, m, (int)nmt64, (int)nnt,
-                         (float*)dB, lddb);
+                         (float*)dB, lddb, streamed);
       rc = tsp::check_launch("screened_bwd_b_flex launch");
     } else if (dtype == TSP_F32) {
       const int64_t nnt = tsp::ceil_div(ncols, TILE);
@@ -910,8 +920,8 @@ int launch(const void* A, int dtype, int64_t lda, const void* diag, double thr_s
   int rc = tsp::check_launch("screened_q launch");
   if (rc) return rc;
   // streamed fp32 kernel: 16-byte aligned rows, buffer offsets within 32 bits
-  const bool fits = (lda % 4) == 0 && (ldb % 4) == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)B % 16) == 0 &&
-                    (m + TILE) * lda * 4 + 4 * TILE <= (int64_t)UINT32_MAX &&
+  const bool rows16 = (lda % 4) == 0 && (ldb % 4) == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)B % 16) == 0;
+  const bool fits = rows16 && (m + TILE) * lda * 4 + 4 * TILE <= (int64_t)UINT32_MAX &&
                     (m + TILE) * ldb * 4 + 4 * TILE <= (int64_t)UINT32_MAX;
   if (dtype == TSP_F32 && (!fits || small_tiles_faster(m, ncols, 88, 139, 21))) {
     const int64_t nmt64 = tsp::ceil_div(m, FT), nnt = tsp::ceil_div(ncols, FT);
@@ -919,7 +929,7 @@ int launch(const void* A, int dtype, int64_t lda, const void* diag, double thr_s
     if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "tsp_screened_spmm: problem too large");
     hipLaunchKernelGGL((screened_f32_flex<QT>), dim3((unsigned)grid), dim3(X::NTHR), 0, st, (const float*)A, lda,
                        (const QT*)Q, (const QT*)qmax, thr, m, (const float*)B, ldb, ncols, (float*)C, ldc, (int)nmt64,
-                       (int)nnt);
+                       (int)nnt, rows16);
     return tsp::check_launch("screened_f32_flex launch");
   }
   if (dtype == TSP_F32) {
