@@ -101,6 +101,20 @@ def test_screened_noalloc_size_limit_is_host_side():
     assert lib.tsp_screened_spmm_noalloc(None, 0, 4, None, 0, 0.0, 4, None, 0, 0, None, 0, None) == 0  # no columns
 
 
+@pytest.mark.skipif(not LIB.exists(), reason="library not built (run __graft_entry__.build())")
+@pytest.mark.parametrize("head_dim,per_pair", [(64, 4), (128, 1), (256, 2)])
+def test_attention_backward_grid_limit_is_host_side(head_dim, per_pair):
+    """A column pass of 2^31 or more workgroups (`per_pair` for each plan item
+    and head) is refused before any device work (dummy pointers)."""
+    from trnsparse_amd.hip import _lib
+
+    lib = _lib.load()
+    d = ctypes.c_void_p(256)
+    st = lib.tsp_bsa_bwd(d, d, d, d, d, _lib.TSP_F32, 8, 100, head_dim, d, d, d, d, 1, 128, 0.1, d, d, d, d, d, d,
+                         (1 << 31) // per_pair // 8, 0, 0, d, None)
+    assert st == -2 and b"too large" in lib.tsp_last_error()
+
+
 def _plan(cp, H, S, b):
     import numpy as np
 

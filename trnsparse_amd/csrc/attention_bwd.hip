@@ -1123,7 +1123,8 @@ int launch_f32(const void* Q, const void* K, const void* V, const void* O, const
                const void* rmax, const void* rden, void* dQ, void* dK, void* dV, const int32_t* plan, int64_t n_items,
                int64_t n_splits, int64_t n_partials, void* workspace, hipStream_t st) {
   const int64_t grid_a = tsp::head_grid(Mt * (D == 256 ? 2 : 1), H), grid_b = n_items * H * (D == 256 ? 2 : 1);
-  if (grid_a > INT32_MAX || grid_b > INT32_MAX || 8 * n_splits > INT32_MAX || H > 65535)
+  // (at d = 64 the column pass is always four workgroups a pair, attention_split.hip)
+  if (grid_a > INT32_MAX || grid_b > INT32_MAX / (D == 64 ? 4 : 1) - 8 || 8 * n_splits > INT32_MAX || H > 65535)
     return tsp::fail(TSP_EUNSUPPORTED, "tsp_bsa_bwd: problem too large");
   const float sl2 = (float)(scale * 1.4426950408889634);
   float* qstat = (float*)workspace;
