@@ -137,7 +137,19 @@ def test_ops_reject_mismatched_arguments(hip_backend):
     blocks = torch.randn(3, 128, 128, device=dev)
     B = torch.randn(256, 16, device=dev)
     ops.bsr_spmm(blocks, rp, ci, None, 256, 256, 128, B, torch.float32)  # the well-formed call runs
+    # dC as the first columns of padded rows runs; from a later column on, the
+    # storage ends inside the last row's padding
+    cp, crow = torch.tensor([0, 1, 3], **i64), torch.tensor([0, 0, 1], **i64)
+    wide = torch.randn(256, 24, device=dev)
+
+    def spmm_t(G):
+        return ops.bsr_spmm_t(blocks, cp, torch.arange(3, device=dev), crow, torch.empty(0, dtype=torch.int32, device=dev),
+                              256, 256, 128, G)
+
+    torch.testing.assert_close(spmm_t(wide[:, :16]), spmm_t(wide[:, :16].contiguous()), rtol=0, atol=0)
+    assert spmm_t(wide[:, :0]).shape == (256, 0)
     bad_bsr = [
+        lambda: spmm_t(wide[:, 8:]),
         lambda: ops.bsr_spmm(blocks, rp, ci, None, 256, 256, 128, B[:200], torch.float32),  # B shorter than n
         lambda: ops.bsr_spmm(blocks, rp, ci, None, 384, 256, 128, B, torch.float32),  # row_ptrs vs m
         lambda: ops.bsr_spmm(blocks, rp, ci[:2], None, 256, 256, 128, B, torch.float32),  # indices vs blocks

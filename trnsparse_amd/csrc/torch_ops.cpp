@@ -198,6 +198,9 @@ at::Tensor bsr_spmm_t(const at::Tensor& blocks, const at::Tensor& cp, const at::
   const int64_t ldg = m > 1 ? G.stride(0) : G.size(1);
   TORCH_CHECK((G.size(1) <= 1 || G.stride(1) == 1) && ldg >= G.size(1),
               "bsr_spmm_t: grad_out must have unit column stride and rows that do not overlap");
+  // (the 128x128-tile kernels read whole rows of the stride, the last one too)
+  TORCH_CHECK(G.numel() == 0 || m * ldg <= (int64_t)(G.storage().nbytes() / G.element_size()) - G.storage_offset(),
+              "bsr_spmm_t: grad_out's storage ends inside the padding of its last row");
   TORCH_CHECK(blocks.dim() == 3 && blocks.size(1) == block_size && blocks.size(2) == block_size,
               "bsr_spmm_t: blocks has shape ", blocks.sizes());
   need_dtype(blocks, G.scalar_type(), "bsr_spmm_t", "blocks (the dtype of grad_out)");
