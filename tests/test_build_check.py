@@ -4,9 +4,16 @@ compiler-generated instruction may use M0 in kernels that include it.
 The scanner is checked on synthetic assembly (a use outside the asm blocks
 is reported, uses inside are not), and on the assembly the last build
 emitted for each such kernel, when present.
+
+And the small-tile BSR kernels' use of scratch memory, from the metadata of
+their last build.
 """
 
 from __future__ import annotations
+
+import re
+import shutil
+import subprocess
 
 import pytest
 
@@ -39,3 +46,19 @@ def test_last_build_assembly_has_no_m0_outside_asm():
         pytest.skip("library not built in this tree (run __graft_entry__.build())")
     for a in asms:
         assert build_lib.m0_uses_outside_asm(a.read_text()) == [], a.name
+
+
+def test_small_tile_kernels_use_no_scratch(tmp_path):
+    """A launch of a kernel that uses scratch memory takes over 10 us longer,
+    more than the small-tile BSR kernels' whole time on small operands."""
+    obj = build_lib.BUILD / "bsr_flex.o"
+    tools = [shutil.which(t, path="/opt/rocm/llvm/bin") for t in ("clang-offload-bundler", "llvm-readelf", "llvm-objcopy")]
+    if not obj.exists() or not all(tools):
+        pytest.skip("library not built in this tree (run __graft_entry__.build())")
+    fat, code = tmp_path / "fatbin", tmp_path / "code"
+    subprocess.run([tools[2], f"--dump-section=.hip_fatbin={fat}", str(obj), str(tmp_path / "o")], check=True)
+    subprocess.run([tools[0], "--unbundle", "--type=o", f"--targets=hipv4-amdgcn-amd-amdhsa--{build_lib.ARCH}",
+                    f"--input={fat}", f"--output={code}"], check=True)
+    notes = subprocess.run([tools[1], "--notes", str(code)], check=True, capture_output=True, text=True).stdout
+    sizes = re.findall(r"\.private_segment_fixed_size:\s*(\d+)", notes)
+    assert len(sizes) >= 30 and set(sizes) == {"0"}, sizes

@@ -20,24 +20,41 @@ namespace {
 
 namespace X = tsp::flex;
 
-// A list walked in order, 64 entries at a time in the lanes of a wavefront,
-// the next 64 loaded ahead.
+// A list walked in order, 64 entries at a time in the lanes of a wavefront;
+// AHEAD: the next 64 loaded ahead (64 entries of 64 rows and more last 64 slabs
+// or more, where a wait for the next is little and the register is short).
+template <bool AHEAD>
 struct Walk {
   const int64_t* p;
   int n, base;
   int cur, next;
-  __device__ Walk(const int64_t* p_, int n_) : p(p_), n(n_), base(0), cur(fetch(0)), next(fetch(64)) {}
+  __device__ Walk(const int64_t* p_, int n_) : p(p_), n(n_), base(0), cur(fetch(0)), next(AHEAD ? fetch(64) : 0) {}
   __device__ int fetch(int at) const {
     const int i = at + ((int)threadIdx.x & 63);
     return i < n ? (int)p[i] : 0;
   }
-  __device__ int get(int i) {
-    if (i - base >= 64) {
+  // brings in entry q and the PER - 1 after it (q a multiple of PER and
+  // ascending from call to call; PER divides 64)
+  __device__ void to(int q) {
+    if (q - base >= 64) {
       base += 64;
-      cur = next;
-      next = fetch(base + 64);
+      cur = AHEAD ? next : fetch(base);
+      if (AHEAD) next = fetch(base + 64);
     }
-    return __builtin_amdgcn_readlane(cur, i - base);
+  }
+  // entry q + e; e may differ between lanes. Selected from scalars: as an array
+  // the PER of them lived in scratch memory, which costs a launch some 13 us
+  // (b = 16, 512 rows of 3 blocks, N = 8: 18.4 -> 4.7 us, its dB 19.6 -> 5.6; a
+  // wavefront per 64 columns took 6.2).
+  template <int PER>
+  __device__ int get(int q, int e) const {
+    int x = __builtin_amdgcn_readlane(cur, q - base);
+#pragma unroll
+    for (int i = 1; i < PER; ++i) {
+      const int v = __builtin_amdgcn_readlane(cur, q - base + i);
+      x = e == i ? v : x;
+    }
+    return x;
   }
 };
 
@@ -57,7 +74,7 @@ struct Stream {
   const T *blocks, *dense;
   int64_t ldd, rows, ncols, n0, p0;
   int nblk, off;  // off: first row (TA: column) of the block in this tile
-  Walk cols, ids;
+  Walk<(B < 64)> cols, ids;
   struct Regs {
     XF x;
     YF y;
@@ -67,21 +84,11 @@ struct Stream {
     // the slab's blocks: entry q0 + e holds its k from e * B (B < 64), or the
     // slab is k kk .. of entry q0
     const int q0 = B < 64 ? s * PER : s / (B / 64), kk = B < 64 ? 0 : s % (B / 64) * 64;
-    int col[PER], id[PER];
-#pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      col[e] = cols.get(q0 + e);
-      if constexpr (TA) id[e] = ids.get(q0 + e);
-    }
-    auto pick = [&](const int (&v)[PER], int e) {
-      int x = v[0];
-#pragma unroll
-      for (int i = 1; i < PER; ++i) x = e == i ? v[i] : x;
-      return x;
-    };
+    cols.to(q0);
+    if constexpr (TA) ids.to(q0);
     auto block = [&](int e) -> const T* {
       if constexpr (TA)
-        return blocks + (int64_t)pick(id, e) * (B * B);
+        return blocks + (int64_t)ids.template get<PER>(q0, e) * (B * B);
       else
         return blocks + (p0 + q0 + e) * (B * B);
     };
@@ -95,7 +102,7 @@ struct Stream {
 #pragma unroll
     for (int j = 0; j < YF::PIECES; ++j) {
       const int k = YF::k() + YF::KSTEP * j, e = B < 64 ? k / B : 0;
-      const int64_t row = (int64_t)pick(col, e) * B + (B < 64 ? k % B : kk + k), c = n0 + YF::i();
+      const int64_t row = (int64_t)cols.template get<PER>(q0, e) * B + (B < 64 ? k % B : kk + k), c = n0 + YF::i();
       r.y.q[j].load(dense + row * ldd + c, !YF::idle() && q0 + e < nblk && row < rows ? ncols - c : 0);
     }
   }
@@ -124,7 +131,7 @@ __global__ __launch_bounds__(X::NTHR, 4) void bsr_flex(const T* __restrict__ blo
   const int64_t n0 = (int64_t)(item / PARTS) * YN;
   const int64_t p0 = ptr[li];
   const int nblk = (int)(ptr[li + 1] - p0);
-  S src{blocks, dense, ldd, dense_rows, ncols, n0, p0, nblk, off, Walk(cols + p0, nblk), Walk(TA ? ids + p0 : cols, TA ? nblk : 0)};
+  S src{blocks, dense, ldd, dense_rows, ncols, n0, p0, nblk, off, {cols + p0, nblk}, {TA ? ids + p0 : cols, TA ? nblk : 0}};
   float acc[S::Split::NOUT];
   X::run<typename S::Split>(src, src.slabs(), lds, acc);
   const int64_t c = n0 + S::Split::col();
