@@ -12,7 +12,9 @@
 // forward 76 us = 90 TFLOP/s, dA 76, dB 81; a wavefront per 64 columns or per
 // block with operands straight from memory, the form before this one, took
 // 132, 92 and 177), by the longest list of slabs, about 1.5 us each, where they
-// do not (1024^2, 19 blocks of 128, N = 256: 12 us, from 28 on 128x128 tiles).
+// do not (1024^2, 19 blocks of 128, N = 256: 12 us, from 28 on 128x128 tiles),
+// and by the start and end of a workgroup, 4 us together, where lists are one
+// slab (256 rows of one block of 32, N = 512: 18 us, a wavefront per tile 11).
 #include "f32_flex.h"
 #include "tile_item.h"
 
@@ -59,11 +61,15 @@ struct Walk {
 };
 
 constexpr int part(int b) { return b < 64 ? b : 64; }  // rows of an output tile
+// Columns of an output tile: 128 were slower for 32-row tiles (107 against 95 us
+// where the chip is full) and for 16-row ones where it is not (8192^2, 10 %
+// blocks, N = 509: 136 against 124; 2992^2, 20 %, N = 80: 22 against 16).
+constexpr int YN = 64;
 
 // The slab stream of one list of stored blocks. TA: the blocks enter
 // transposed (dB); ids[q] is then entry q's block, else its block is p0 + q.
 // dense rows of entry q start at cols[q] * b.
-template <typename T, int B_, int YN, bool TA>
+template <typename T, int B_, bool TA>
 struct Stream {
   static constexpr int B = B_, MS = B < 32 ? 16 : 32, XN = part(B), PER = B < 64 ? 64 / B : 1;
   typedef X::Split<MS, XN, YN> Split;
@@ -113,7 +119,7 @@ struct Stream {
 // (TA: transposed) times dense rows. C = A B: lists are block rows, `cols`
 // the block columns; dB = A^T dC: lists are block columns, `cols` the block
 // rows and `ids` the block numbers.
-template <typename T, typename OutT, int B, int YN, bool TA>
+template <typename T, typename OutT, int B, bool TA>
 __global__ __launch_bounds__(X::NTHR, 4) void bsr_flex(const T* __restrict__ blocks, const int64_t* __restrict__ ptr,
                                                        const int64_t* __restrict__ cols,
                                                        const int64_t* __restrict__ ids, int64_t lists, int nnt,
@@ -121,7 +127,7 @@ __global__ __launch_bounds__(X::NTHR, 4) void bsr_flex(const T* __restrict__ blo
                                                        const T* __restrict__ dense, int64_t ldd, int64_t ncols,
                                                        OutT* __restrict__ out, int64_t ldo,
                                                        const int32_t* __restrict__ order) {
-  typedef Stream<T, B, YN, TA> S;
+  typedef Stream<T, B, TA> S;
   __shared__ __attribute__((aligned(16))) float lds[X::lds_floats<typename S::XF, typename S::YF>()];
   constexpr int PARTS = B / S::XN;
   int64_t li;
@@ -208,22 +214,13 @@ template <typename T, typename OutT, int B, bool TA>
 int launch_product(const void* blocks, const int64_t* ptr, const int64_t* cols, const int64_t* ids, int64_t lists,
                    int64_t out_rows, int64_t dense_rows, const void* dense, int64_t ldd, int64_t ncols, void* out,
                    int64_t ldo, const int32_t* order, hipStream_t st) {
-  auto go = [&](auto ync) {
-    constexpr int YN = decltype(ync)::value;
-    const int64_t nnt = tsp::ceil_div(ncols, YN), parts = B / part(B);
-    const int64_t grid = tsp::ceil_div(lists, 8) * 8 * nnt * parts;
-    if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "bsr_flex: problem too large");
-    hipLaunchKernelGGL((bsr_flex<T, OutT, B, YN, TA>), dim3((unsigned)grid), dim3(X::NTHR), 0, st, (const T*)blocks,
-                       ptr, cols, ids, lists, (int)nnt, out_rows, dense_rows, (const T*)dense, ldd, ncols, (OutT*)out,
-                       ldo, order);
-    return tsp::check_launch("bsr_flex launch");
-  };
-  // 16-row tiles are worth 128 columns (8192^2, 10 % blocks, N = 512: 145 against
-  // 164 us on 64; 3000^2, 20 %, N = 77: 27 against 32); 32-row ones are not (107
-  // against 95)
-  if constexpr (B == 16)
-    if (ncols > 64) return go(std::integral_constant<int, 128>{});
-  return go(std::integral_constant<int, 64>{});
+  const int64_t nnt = tsp::ceil_div(ncols, YN), parts = B / part(B);
+  const int64_t grid = tsp::ceil_div(lists, 8) * 8 * nnt * parts;
+  if (grid > INT32_MAX) return tsp::fail(TSP_EUNSUPPORTED, "bsr_flex: problem too large");
+  hipLaunchKernelGGL((bsr_flex<T, OutT, B, TA>), dim3((unsigned)grid), dim3(X::NTHR), 0, st, (const T*)blocks, ptr,
+                     cols, ids, lists, (int)nnt, out_rows, dense_rows, (const T*)dense, ldd, ncols, (OutT*)out, ldo,
+                     order);
+  return tsp::check_launch("bsr_flex launch");
 }
 
 template <typename T, typename OutT, bool TA, typename... Args>

@@ -14,9 +14,8 @@
 //                      128x128 tiles of C to fill the chip: one tile per
 //                      workgroup, streamed through LDS (below).
 //   bsr_flex           (bsr_flex.hip) fp32 MFMA on tiles of at most 64x64:
-//                      b == 128 otherwise, b == 64 and 32, b == 16 for rows
-//                      and column counts that the small-block kernel does not
-//                      read whole.
+//                      b == 128 otherwise, b == 64 and 32, b == 16 where
+//                      the small-block kernel is slower (small_blocks_whole).
 //   bsr_spmm_bf16_mfma b == 128, bf16 in, fp32 accumulation, fp32/bf16 out
 //                      (v_mfma_f32_32x32x16_bf16, 64x32 wave tiles,
 //                      direct-to-LDS 4-deep ring, B operand through LDS
@@ -840,13 +839,16 @@ int launch_generic(const void* blocks, const int64_t* rp, const int64_t* ci, int
 }  // namespace
 
 // At b = 16 the small-block kernel beats the tiles of bsr_flex where it reads
-// B rows in whole 16-byte pieces and its 64-column tiles are nearly full
-// (8192^2, 10 % blocks: N = 256 53 against 77 us, N = 64 37 against 45); reading
-// element by element it loses (N = 65 68 against 49, N = 509 247 against 168;
-// 3000^2, 20 %, N = 80 44 against 26).
+// B rows in whole 16-byte pieces, its 64-column tiles are full or nearly, and
+// it has two or more of them a row (us, this kernel and bsr_flex: 8192^2, 10 %
+// blocks, N = 64 36 and 20, N = 128 36 and 35, N = 256 50 and 57, N = 512 98
+// and 112; rows of equal length, N = 128 28 and 31; a few blocks a row, N = 256
+// 6 and 10); reading element by element it loses (N = 65 67 and 38, N = 509 234
+// and 124).
 bool tsp::small_blocks_whole(int64_t b, int64_t elem, const void* blocks, const void* B, int64_t ldb, int64_t ncols) {
   if ((uintptr_t)blocks % 16) return false;
-  return b == 8 || (b == 16 && (uintptr_t)B % (4 * elem) == 0 && ldb % 4 == 0 && (ncols % 64 == 0 || ncols >= 256));
+  return b == 8 || (b == 16 && (uintptr_t)B % (4 * elem) == 0 && ldb % 4 == 0 &&
+                    ((ncols % 64 == 0 && ncols >= 128) || ncols >= 256));
 }
 
 // dB = A^T X for block sizes 8 and 16 (the backward of bsr_spmm):
@@ -893,7 +895,10 @@ extern "C" int tsp_bsr_spmm(const void* blocks, int dtype, const int64_t* block_
   // streamed fp32 kernel, one 128x128 tile per CU at a time, needs about 1.5
   // tiles per CU: 8192^2, 10 % blocks, N = 512 (256 tiles) 103 against 81 us,
   // N = 256 (128 tiles) 100 against 49; 12800 x 8192, 5 %, N = 512 (400 tiles)
-  // 63 against 64; 16384^2, N = 512 (512 tiles) 260 against 304.
+  // 63 against 64; 16384^2, N = 512 (512 tiles) 260 against 304. What it loses
+  // there is the wait for the longest rows, which are not known here: where 256
+  // tiles have rows of equal length it is ahead, 62 against 71 us, and far
+  // behind where one row in 16 is full, 522 against 200.
   const bool flex = (dtype == TSP_F32 || dtype == TSP_BF16) && n_blocks <= INT32_MAX &&
                     tsp::ceil_div(n, block_size) <= INT32_MAX &&
                     (block_size == 16 || block_size == 32 || block_size == 64 || block_size == BS);
