@@ -561,6 +561,12 @@ int dkdv(const void* Q, const void* K, const void* V, const void* dO, int64_t H,
 // kernel's registers allowed one: 184 work items 61 of 74 us, 276 95 of 142,
 // 368 112 of 140, 1104 311 of 345, 32 heads of 8192 894 of 918, and 78 of 76
 // only just below one full round (230), so that kernel is gone.
+// Rows of one block pay for the merge at the end and no more: 12 heads of 2048 at
+// 128 (192 block rows, 3 rounds of 1) take 37 us forward where the full-grid
+// kernel takes 31, dQ 54 of 45, dK / dV 60 of 50, and dK / dV at 64 257 of 221 on
+// 32 heads of 8192. The lengths are not known here, and other masks gain: the
+// same 12 heads forward, window 4 110 of 115 us, causal 203 of 278, one global
+// block row and column 137 of 277.
 // bf16 products are too short to pay for the fourfold loads once a second
 // round starts: 72 block rows at 128 (288 workgroups) 20.4 against 18.6 us, 64
 // (256) 20.6 against 28.3; at 64, 128 block rows (512 workgroups, two to a CU)
