@@ -217,7 +217,7 @@ def test_block_column_view(mb, nbc, p):
 
 
 @pytest.mark.parametrize("mb,nbc,p", [(128, 128, 1.0), (128, 129, 1.0), (4096, 4, 0.7), (4097, 3, 0.7), (3, 4096, 0.9),
-                                      (3, 4097, 0.9), (1, 4000, 1.0), (65, 9, 0.5)])
+                                      (3, 4097, 0.9), (1, 4000, 1.0), (65, 9, 0.5), (4096, 4096, 0.0009)])
 def test_block_column_view_limits(mb, nbc, p):
     """The same at and just past the sizes that the one-launch plan takes
     (16384 blocks, 4096 rows and columns), and the columns ordered by length."""
@@ -230,6 +230,25 @@ def test_block_column_view_limits(mb, nbc, p):
     _, cp, _, _, corder = D._bsr_bwd_plan(rp, ci, mb, nbc, torch.device("cuda"))
     lens = cp.diff()[corder[:nbc].long()].clamp(max=1023)  # (the order does not tell longer columns apart)
     assert bool((lens[1:] <= lens[:-1]).all())
+
+
+@pytest.mark.parametrize("rows", [[31, 32, 33], [0], [4095], [0, 2047, 4095], list(range(100, 3000, 7))])
+@pytest.mark.parametrize("per_row", [1, 4, 32])
+def test_block_rows_of_the_one_launch_plan(rows, per_row):
+    """Block rows of each entry where most rows are empty, the first and last
+    among them, and rows start around the 32 entries that a thread scans."""
+    from trnsparse_amd.hip import dispatch as D
+
+    lens = torch.zeros(4096, dtype=torch.int64)
+    lens[rows] = per_row
+    lens[rows[0]] += 3
+    rp = torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)])
+    ci = (torch.arange(int(rp[-1])) * 7) % 40
+    brow, cp, cbid, crow, _ = D._bsr_bwd_plan(rp.cuda(), ci.cuda(), 4096, 40, torch.device("cuda"))
+    want = torch.repeat_interleave(torch.arange(4096), lens)
+    order = torch.argsort(ci, stable=True)
+    assert torch.equal(brow.cpu(), want) and torch.equal(cbid.cpu(), order) and torch.equal(crow.cpu(), want[order])
+    assert torch.equal(cp.cpu().diff(), torch.bincount(ci, minlength=40))
 
 
 @pytest.mark.parametrize("b", [8, 16, 64, 128])

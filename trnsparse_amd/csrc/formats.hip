@@ -1669,10 +1669,11 @@ __global__ __launch_bounds__(512) void bsr_col_plan_small(const int64_t* __restr
                                                           int64_t* __restrict__ brow, int64_t* __restrict__ cp,
                                                           int64_t* __restrict__ cbid, int64_t* __restrict__ crow,
                                                           int32_t* __restrict__ corder) {
-  __shared__ uint16_t scol[SV_NNZ], srow[SV_NNZ];
-  __shared__ int cnt[SV_COLS], srp[SV_ROWS + 1];
+  __shared__ __attribute__((aligned(16))) uint16_t scol[SV_NNZ], srow[SV_NNZ];
+  __shared__ int cnt[SV_COLS], srp[SV_ROWS + 1], wtop[8];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   for (int i = tid; i < nbc; i += 512) cnt[i] = 0;
+  for (int i = tid; i < SV_NNZ / 8; i += 512) *(u32x4*)(srow + 8 * i) = u32x4{};
   for (int i = tid; i <= mb; i += 512) srp[i] = (int)rp[i];
   __syncthreads();
   for (int k0 = tid; k0 < nnzb; k0 += 8 * 512) {  // 8 loads in flight
@@ -1687,9 +1688,50 @@ __global__ __launch_bounds__(512) void bsr_col_plan_small(const int64_t* __restr
       if (in) atomicAdd(&cnt[c[u]], 1);
     }
   }
-  for (int r = tid >> 4; r < mb; r += 32)  // 16 lanes per block row
-    for (int k = srp[r] + (tid & 15); k < srp[r + 1] && k < nnzb; k += 16)
-      if (k >= 0) srow[k] = (uint16_t)r;
+  // the block row of each entry: each row's number at its first entry, and the
+  // largest so far from there on. (16 lanes to a row, row after row, made this
+  // launch slower than the nine where rows are many or long: whole calls of 4096
+  // rows and columns, 15048 blocks, 112 -> 67 us, the nine 76; 4096 x 16, 13274
+  // blocks, 57 -> 35, the nine 52; 4 x 4096, 14700 blocks, 68 -> 62 of 65.)
+  for (int r = tid; r < mb; r += 512) {
+    const int k = srp[r];
+    if (k < srp[r + 1] && k >= 0 && k < nnzb) srow[k] = (uint16_t)r;
+  }
+  __syncthreads();
+  {
+    constexpr int EACH = SV_NNZ / 512;
+    typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+    u16x8 v[EACH / 8];
+    int top = 0;
+#pragma unroll
+    for (int i = 0; i < EACH / 8; ++i) {
+      v[i] = *(const u16x8*)(srow + EACH * tid + 8 * i);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        top = top > (int)v[i][e] ? top : (int)v[i][e];
+        v[i][e] = (uint16_t)top;
+      }
+    }
+    int incl = top;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl = incl > y ? incl : y;
+    }
+    if (lane == 63) wtop[w] = incl;
+    __syncthreads();
+    int before = __shfl_up(incl, 1, 64);
+    if (lane == 0) before = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < w && wtop[i] > before) before = wtop[i];
+#pragma unroll
+    for (int i = 0; i < EACH / 8; ++i) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[i][e] = (int)v[i][e] > before ? v[i][e] : (uint16_t)before;
+      *(u16x8*)(srow + EACH * tid + 8 * i) = v[i];
+    }
+  }
   __syncthreads();
   for (int k = blockIdx.x * 512 + tid; k < nnzb; k += gridDim.x * 512) brow[k] = srow[k];
   const int j = blockIdx.x * 8 + w;
