@@ -123,8 +123,9 @@ def test_fp32_mfma(hip_backend, S, D, mask, H):
 
 @pytest.mark.parametrize("D", [64, 256])
 def test_fp32_mfma_long_row(hip_backend, D):
-    """A block row with more than 64 stored blocks (the kernel reads the
-    row's block columns 64 at a time)."""
+    """A block row with more than 64 stored blocks (the kernel, of 32 queries to
+    a workgroup at these 67 pairs for D = 64 and 128, reads the row's block
+    columns 64 at a time)."""
     nb = 67
     S = nb * 128
     mask = local_mask(nb, 0)

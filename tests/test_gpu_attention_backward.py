@@ -9,8 +9,9 @@ measure per gradient element: |g - g_exact| / g_abs, with g_abs the oracle's
 absolute form (|dS| replaced by P (|dO V^T| + |D|), operands by their
 magnitudes). fp32 <= 1e-4, bf16 <= 2e-2, fp64 <= 1e-10. fp32 with b = 128
 and d in {64, 128, 256} runs the fp32 MFMA kernels (16-row tiles at
-d = 256), bf16 with d <= 128 the bf16 MFMA kernels of d = 128 (d below 128
-zero-padded to 128), bf16 with d = 256 and fp32 / bf16 with d > 256
+d = 256), bf16 with d in {64, 128} the bf16 MFMA kernels (both at d <= 128 with
+32 or 128 queries and keys to a workgroup, by the number of block rows and
+heads), bf16 with d = 256 and fp32 / bf16 with d > 256
 block products over the mask stacked over heads (SDDMM, elementwise softmax
 gradient, BSR SpMMs) when S is a whole number of blocks, other d below 256
 zero-padded to 64, 128 or 256 first; everything else (fp64, ragged S at
@@ -81,9 +82,9 @@ def _check_head(Q, K, V, dO, O, grads, mask_bsr, scale, tol, rows=None, cols=Non
         (512, 128, global_mask(4, 1, 1), torch.bfloat16),
         (300, 128, local_mask(3, 2), torch.bfloat16),     # MFMA, last key block crosses S
         (1024, 128, global_mask(8, 1, 1), torch.bfloat16),  # MFMA, global column split into 2 segments
-        (256, 64, local_mask(2, 1), torch.bfloat16),      # bf16 d = 64: zero-padded to 128, bf16 MFMA kernels
+        (256, 64, local_mask(2, 1), torch.bfloat16),      # bf16 MFMA kernels of d = 64
         (640, 64, W.cfg5_block_mask(5), torch.bfloat16),
-        (256, 32, local_mask(2, 1), torch.bfloat16),      # head_dim zero-padded to 128
+        (256, 32, local_mask(2, 1), torch.bfloat16),      # head_dim zero-padded to 64
         (300, 96, local_mask(3, 1), torch.bfloat16),      # zero-padded to 128, last key block crosses S
         (256, 100, global_mask(2, 0, 1), torch.float32),  # head_dim zero-padded to 128
         (256, 160, local_mask(2, 1), torch.bfloat16),     # head_dim zero-padded to 256: block products
@@ -132,8 +133,7 @@ def test_backward_empty_rows_and_ragged(hip_backend, dtype, D):
 
 @pytest.mark.parametrize("D", [128, 64])
 def test_backward_batched_heads_bf16(hip_backend, D):
-    """Leading (batch, head) dims; at D = 64 the operands are zero-padded to
-    128 and the gradients cut back to 64 columns."""
+    """Leading (batch, head) dims."""
     torch.manual_seed(12)
     S = 512
     mask_bsr = W.bsr_from_block_mask(global_mask(4, 1, 1), 128)
@@ -160,8 +160,9 @@ def test_backward_batched_heads_f32(hip_backend, D):
 
 
 def test_backward_f32_long_row(hip_backend):
-    """A query block row with more than 64 stored blocks (the row pass reads
-    the row's block columns 64 at a time)."""
+    """A query block row with more than 64 stored blocks (the row pass, of 32
+    queries to a workgroup at these 67 pairs, reads the row's block columns 64 at
+    a time)."""
     nb, D = 67, 64
     S = nb * 128
     mask = local_mask(nb, 0)
@@ -339,3 +340,67 @@ def test_column_rows_past_the_whole_blocks_f32(hip_backend, D, S):
         t[:, own] = 0.0
         assert torch.count_nonzero(t).item() == 0
     assert torch.count_nonzero(out[0][:, 128 * Mt :]).item() == 0
+
+
+@pytest.mark.parametrize("H", [1, 40])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rows_past_64_blocks_on_both_grids(hip_backend, dtype, D, H):
+    """A block row of 80 entries (the row passes read block columns 64 at a
+    time), forward and backward, on 20 (head, block row) pairs and on 800: 32
+    queries to a workgroup and 128. A block listed four times counts four
+    times."""
+    nb = 20
+    S = nb * 128
+    lists = [list(range(nb)) * 4 if i == 1 else [i] for i in range(nb)]
+    ptr = torch.tensor([0] + [len(c) for c in lists]).cumsum(0)
+    mask_bsr = ts.BSRMatrix(torch.ones(int(ptr[-1]), 128, 128), torch.tensor(sum(lists, [])), ptr, (S, S), 128)
+    g = torch.Generator().manual_seed(17)
+    Q, K, V, dO = (torch.randn(H, S, D, generator=g).to(dtype) for _ in range(4))
+    O, dQ, dK, dV = _run(Q, K, V, dO, mask_bsr)
+    fwd = (mask_bsr.block_row_ptrs.numpy(), mask_bsr.block_col_indices.numpy(), 128, D**-0.5)
+    for hh in sorted({0, H - 1}):
+        exact = ref.block_sparse_attention(_np(Q[hh]), _np(K[hh]), _np(V[hh]), *fwd)[0]
+        bound = ref.block_sparse_attention(_np(Q[hh]), _np(K[hh]), np.abs(_np(V[hh])), *fwd)[0]
+        assert ref.scaled_error(_np(O[hh]), exact, np.maximum(bound, 1e-30)) <= TOL[dtype]
+        _check_head(Q[hh], K[hh], V[hh], dO[hh], O[hh], (dQ[hh], dK[hh], dV[hh]), mask_bsr, D**-0.5, TOL[dtype])
+
+
+@pytest.mark.parametrize("H", [1, 70])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_non_finite_operands_on_both_grids(hip_backend, dtype, D, H):
+    """Infinite scores, an infinite V element and a NaN query in block 0, on 8
+    (head, block row) pairs (32 queries to a workgroup) and on 560: O is what
+    float64 gives over the stored blocks, and queries and keys that do not meet
+    block 0 have their gradients unchanged."""
+    S, scale = 1024, D**-0.5
+    mask = local_mask(8, 1)
+    mask_bsr = W.bsr_from_block_mask(mask, 128)
+    g = torch.Generator().manual_seed(18)
+    Q, K, V, dO = (torch.randn(1, S, D, generator=g).to(dtype) for _ in range(4))
+    clean = tuple(t[0].clone() for t in (Q, K, V, dO))
+    K[0, 20] = 0.0
+    K[0, 20, 0] = float("inf")   # scores +-inf by the sign of Q[:, 0]: NaN rows and absent keys
+    V[0, 10, 7] = float("inf")
+    Q[0, 30, 3] = float("nan")
+    O, dQ, dK, dV = _run(*(t.expand(H, -1, -1).contiguous() for t in (Q, K, V, dO)), mask_bsr)
+    seen = mask.repeat_interleave(128, 0).repeat_interleave(128, 1)
+    want = torch.empty(S, D, dtype=torch.float64)
+    for m in range(8):
+        rows, keys = slice(128 * m, 128 * m + 128), seen[128 * m]
+        want[rows] = (Q[0, rows].double() @ K[0, keys].double().T * scale).softmax(1) @ V[0, keys].double()
+    fwd = (mask_bsr.block_row_ptrs.numpy(), mask_bsr.block_col_indices.numpy(), 128, scale)
+    Oc = torch.from_numpy(ref.block_sparse_attention(*(_np(t) for t in clean[:3]), *fwd)[0])
+    args = (*(_np(t) for t in clean[:3]), Oc.numpy(), _np(clean[3]), *fwd)
+    exact = ref.block_sparse_attention_backward(*args)
+    bound = ref.block_sparse_attention_backward(*args, absolute=True)
+    far_q, far_k = slice(256, S), slice(384, S)  # blocks 0 and 1 meet block 0; their queries meet keys up to block 2
+    for hh in sorted({0, H - 1}):
+        got = O[hh].double()
+        for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(kind(got), kind(want)), kind
+        there = torch.isfinite(want)
+        assert (got - want)[there].abs().max().item() <= 4 * TOL[dtype]  # |O| is at most 4 of unit normals
+        for t, e, a, sel in zip((dQ, dK, dV), exact, bound, (far_q, far_k, far_k)):
+            assert ref.scaled_error(_np(t[hh])[sel], e[sel], np.maximum(a[sel], 1e-30)) <= TOL[dtype]

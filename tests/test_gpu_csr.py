@@ -293,3 +293,29 @@ def _cfg2_windowed(dist, index_dtype):
     assert abs(got.astype(np.float64).sum() - colsum @ x) <= TOL * float(np.abs(v).astype(np.float64) @ np.abs(x[c]))
     # repeat call through the cached plan is bit-identical
     assert np.array_equal(ts.spmv(A, xd).cpu().numpy(), got)
+
+
+@pytest.mark.parametrize("dtype,N", [(torch.float32, 5), (torch.float32, 7), (torch.float32, 18), (torch.float32, 131),
+                                     (torch.float64, 3), (torch.float64, 65)])
+def test_values_gradient_non_finite_columns(hip_backend, dtype, N):
+    """Column counts whose last part overlaps its neighbour in the values
+    gradient: an infinity or NaN in any column of dC or B counts once (what
+    the parts share counts as zero in the later one, 0 and not inf * 0)."""
+    g = torch.Generator().manual_seed(N)
+    A = ts.from_dense((torch.rand(60, 40, generator=g) < 0.3).to(dtype))
+    rows = torch.repeat_interleave(torch.arange(60), A.row_ptrs.diff())
+    for where in ("X", "G"):
+        for c in sorted({0, N - 4, N - 3, N - 2, N - 1} & set(range(N))):
+            X, G = torch.randn(40, N, generator=g, dtype=torch.float64), torch.randn(60, N, generator=g, dtype=torch.float64)
+            X, G = X.to(dtype), G.to(dtype)
+            bad = X if where == "X" else G
+            bad[3, c], bad[7, c] = float("inf"), float("nan")
+            v = A.values.cuda().requires_grad_(True)
+            C = ts.spmm(ts.CSRMatrix(v, A.col_indices.cuda(), A.row_ptrs.cuda(), A.shape), X.cuda())
+            (dv,) = torch.autograd.grad(C, v, G.cuda())
+            want = (G.double()[rows] * X.double()[A.col_indices]).sum(1)
+            got = dv.cpu().double()
+            for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+                assert torch.equal(kind(got), kind(want)), (where, c, kind)
+            there = torch.isfinite(want)
+            assert (got - want)[there].abs().max().item() <= 1e-3  # 131 products of unit normals in fp32: below 1e-4
