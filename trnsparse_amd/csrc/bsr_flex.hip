@@ -23,8 +23,10 @@ namespace {
 namespace X = tsp::flex;
 
 // A list walked in order, 64 entries at a time in the lanes of a wavefront;
-// AHEAD: the next 64 loaded ahead (64 entries of 64 rows and more last 64 slabs
-// or more, where a wait for the next is little and the register is short).
+// AHEAD: the next 64 loaded ahead. (Not for dB at b >= 64, whose registers are
+// short: two spilled there, 94 against 86 us on 8192^2, 10 % blocks of 128, N =
+// 512, and 64 entries last 64 slabs or more, where a wait for the next is
+// little.)
 template <bool AHEAD>
 struct Walk {
   const int64_t* p;
@@ -80,7 +82,7 @@ struct Stream {
   const T *blocks, *dense;
   int64_t ldd, rows, ncols, n0, p0;
   int nblk, off;  // off: first row (TA: column) of the block in this tile
-  Walk<(B < 64)> cols, ids;
+  Walk<(B < 64 || !TA)> cols, ids;
   struct Regs {
     XF x;
     YF y;

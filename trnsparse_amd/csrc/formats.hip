@@ -1673,7 +1673,9 @@ __global__ __launch_bounds__(512) void bsr_col_plan_small(const int64_t* __restr
   __shared__ int cnt[SV_COLS], srp[SV_ROWS + 1], wtop[8];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   for (int i = tid; i < nbc; i += 512) cnt[i] = 0;
-  for (int i = tid; i < SV_NNZ / 8; i += 512) *(u32x4*)(srow + 8 * i) = u32x4{};
+  // each thread scans `vecs` runs of 8 entries for their block rows (below)
+  const int vecs = (nnzb + 8 * 512 - 1) / (8 * 512);
+  for (int i = tid; i < 512 * vecs; i += 512) *(u32x4*)(srow + 8 * i) = u32x4{};
   for (int i = tid; i <= mb; i += 512) srp[i] = (int)rp[i];
   __syncthreads();
   for (int k0 = tid; k0 < nnzb; k0 += 8 * 512) {  // 8 loads in flight
@@ -1699,13 +1701,15 @@ __global__ __launch_bounds__(512) void bsr_col_plan_small(const int64_t* __restr
   }
   __syncthreads();
   {
-    constexpr int EACH = SV_NNZ / 512;
+    constexpr int MOST = SV_NNZ / (8 * 512);
     typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
-    u16x8 v[EACH / 8];
+    uint16_t* const mine = srow + 8 * vecs * tid;
+    u16x8 v[MOST];
     int top = 0;
 #pragma unroll
-    for (int i = 0; i < EACH / 8; ++i) {
-      v[i] = *(const u16x8*)(srow + EACH * tid + 8 * i);
+    for (int i = 0; i < MOST; ++i) {
+      if (i >= vecs) break;
+      v[i] = *(const u16x8*)(mine + 8 * i);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         top = top > (int)v[i][e] ? top : (int)v[i][e];
@@ -1726,10 +1730,11 @@ __global__ __launch_bounds__(512) void bsr_col_plan_small(const int64_t* __restr
     for (int i = 0; i < 8; ++i)
       if (i < w && wtop[i] > before) before = wtop[i];
 #pragma unroll
-    for (int i = 0; i < EACH / 8; ++i) {
+    for (int i = 0; i < MOST; ++i) {
+      if (i >= vecs) break;
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[i][e] = (int)v[i][e] > before ? v[i][e] : (uint16_t)before;
-      *(u16x8*)(srow + EACH * tid + 8 * i) = v[i];
+      *(u16x8*)(mine + 8 * i) = v[i];
     }
   }
   __syncthreads();
