@@ -467,8 +467,8 @@ int tsp_bsa_block_pgrad(const void* Q, const void* K, const void* V,
  * copy of the whole plan. `workspace` holds
  * tsp_bsa_bwd_workspace_size(n_heads, seq_len, head_dim, n_partials) bytes.
  * block_size 128 with scale > 0 runs on the MFMA kernels for bf16 at
- * head_dim 128 and fp32 at head_dim 64, 128 and 256; other shapes and fp64
- * run on the generic kernels (which ignore the plan).
+ * head_dim 64 and 128 and fp32 at head_dim 64, 128 and 256; other shapes and
+ * fp64 run on the generic kernels (which ignore the plan).
  * Replaces nki_bsr_attn_bwd (trnsparse/nki/dispatch.py:813-929; its host
  * gathers _attn_bwd_gather, dispatch.py:680-810) and the torch backward
  * _block_sparse_attn_backward (trnsparse/ops.py:360-473).

@@ -215,8 +215,8 @@ int launch_generic(const void* Q, const void* K, const void* V, const void* dO, 
 
 // --------------------------------------------- bf16 MFMA, d = 64 and 128
 
-// Both passes run one wavefront per SIMD (a 256-thread workgroup per CU)
-// and issue their work in a fixed slot order: slot k is one MFMA whose LDS
+// Both passes run one wavefront per SIMD (a 256-thread workgroup per CU; two at
+// d = 64) and issue their work in a fixed slot order: slot k is one MFMA whose LDS
 // operand was read PF slots earlier (a register ring, so LDS latency hides
 // behind the MFMAs of the same wave), plus a slice of the softmax-gradient
 // VALU work of the previous 32-row tile, so that the VALU runs while the

@@ -26,11 +26,11 @@
 // SDDMM (values gradient of A X, tsp_csr_sddmm): per nonzero the dot product
 // of G's row and X's row over the dense columns, lanes as in the narrow SpMM.
 //
-// SpMM: one wavefront per row, lanes across the columns of B (coalesced B
-// row reads), the row's (col, value) pairs loaded 64 at a time and broadcast
-// with shuffles. fp32 B with a multiple of 4 columns takes the narrow
-// variant: several rows per wavefront, each row's nonzeros split over lane
-// groups, 16-byte B loads, 128-column passes.
+// SpMM: fp32 takes the narrow kernel at any column count and alignment:
+// several rows per wavefront, each row's nonzeros split over lane groups,
+// 16-byte B loads, 128-column passes. fp64: one wavefront per row, lanes across
+// the columns of B (coalesced B row reads), the row's (col, value) pairs loaded
+// 64 at a time and broadcast with shuffles.
 #include "common.h"
 
 namespace {
