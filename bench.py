@@ -27,6 +27,8 @@ All inputs are synthetic and seeded (trnsparse_amd/workloads.py).
 from __future__ import annotations
 
 import argparse
+import functools
+import gc
 import json
 import os
 import pathlib
@@ -61,6 +63,27 @@ def prewarm(fn, seconds: float = 0.25):
         torch.cuda.synchronize()
 
 
+def without_collection(timer):
+    """Python's collector held off while `timer` runs, after a collection
+    before it. One of the whole heap takes some 40 ms with torch imported, and
+    started in whichever call reached its count: 20 launches of the headline
+    take 5 ms."""
+
+    @functools.wraps(timer)
+    def held(*args, **kwargs):
+        gc.collect()
+        on = gc.isenabled()
+        gc.disable()
+        try:
+            return timer(*args, **kwargs)
+        finally:
+            if on:
+                gc.enable()
+
+    return held
+
+
+@without_collection
 def time_gpu(fn, steps: int, warmup: int, flush=None, prewarm_s: float = 0.25):
     """(wall ms/step, event ms/step). With `flush`, each step is timed alone
     after `flush()` evicts L2/MALL, and the event time is the median.
@@ -97,6 +120,7 @@ def time_gpu(fn, steps: int, warmup: int, flush=None, prewarm_s: float = 0.25):
     return wall, times[len(times) // 2]
 
 
+@without_collection
 def time_gpu_spread(fn, steps: int, warmup: int, segments: int = 5, prewarm_s: float = 0.25):
     """Per-launch event times of `segments` back-to-back timed segments of
     `steps` launches each (same pre-warm and warmup as time_gpu), as
